@@ -277,22 +277,18 @@ int sph_count_pairs(sph_solver* s, uint64_t counts[2]);
 /* ---- launch variants and the autotuner -------------------------------------
  * The reference launches fixed block shapes (Solver.cu:1082-1198).  Here the
  * density and force passes have launch variants, selected by a tune word:
- *   bits 0-3   density LDS tile: 0 = 1280, 1 = 512, 2 = 1536, 3 = 2048, 4 = 768,
- *              5 = 1024 particles
- *   bits 4-7   force LDS tile / neighbour-list capacity / entry width:
- *              0 = 640/16/16-bit, 1 = 768/16/16, 2 = 768/24/16, 3 = 768/8/32,
- *              4 = 512/16/16, 5 = 1024/16/16, 6 = 512/8/32, 7 = 640/24/16,
- *              8 = 1024/8/32, 9 = 512/24/16
- *   bits 8-11  density grid, bits 12-15 force grid: 0 = one block per
- *              block-size particles; 1..4 = persistent grid of 1, 2, 4, 8
+ *   bits 0-3   density, bits 4-7 force: waves per block, each handling 32
+ *              particles at a time on an LDS tile of its own: 0 = the default
+ *              (4); density 1..5 and force 1..9 choose others (1 to 6)
+ *   bits 8-11  density grid, bits 12-15 force grid: 0 = one block per its
+ *              waves' particles; 1..4 = persistent grid of 1, 2, 4, 8
  *              blocks per CU looping over those blocks
  *   bits 16-17 density block size, bits 18-19 force block size: 0 = 256,
- *              1 = 128, 2 = 512 threads; a non-zero block size requires that
- *              pass's tile/list field to be 0
- *   bits 20-21 density, bits 22-23 force: particles per lane, 0 = 1, 1 = 2
- *              (particles per wavefront 64 or 128; a block's targets share
- *              one staged union per row); 2 requires that pass's tile/list
- *              and block-size fields to be 0, and a batch refuses it
+ *              1 = 128, 2 = up to 512 threads; a non-zero block size requires
+ *              that pass's waves field to be 0
+ *   bits 20-21 density, bits 22-23 force: groups of 32 particles that a wave
+ *              takes one after the other, 0 = 1, 1 = 2; 1 requires that pass's
+ *              waves and block-size fields to be 0, and a batch refuses it
  *   bits 24-31 must be zero; other words are refused with SPH_ERR_ARG
  * All variants give bit-identical results.  sph_autotune times the variants
  * on the solver's current state (reps launches each), keeps the fastest and

@@ -2,18 +2,20 @@
 passes for a workload and remembers it.
 
 The library's tuner (sph_autotune / sph_batch_autotune) times every variant
-of the two neighbour passes -- LDS tile size, neighbour-list capacity and grid
-shape (one block per 256 particles, or a persistent grid of 1..8 blocks per
-CU) -- on the solver's current state and keeps the fastest; every variant
+of the two neighbour passes -- waves per block, groups per wave and grid shape
+(one block per its waves' groups of 32 particles, or a persistent grid of 1..8
+blocks per CU) -- on the solver's current state and keeps the fastest; every variant
 gives bit-identical results, so tuning never changes the simulation.  This
 module caches the chosen tune word in a JSON file keyed by the device and the
 workload's shape (kind, particle count, cell count, scene count), so a later
 run of the same workload reuses it without timing.
 
-Tune word fields (include/sph2s.h): bits 0-3 density tile, 4-7 force
-tile/list, 8-11 density grid, 12-15 force grid, 16-17 density block size,
-18-19 force block size, 20-21 density and 22-23 force particles per lane
-(particles per wavefront = 64 x particles per lane; single scenes only).
+Tune word fields (include/sph2s.h): bits 0-3 density and 4-7 force waves per
+block, 8-11 density grid, 12-15 force grid, 16-17 density block size, 18-19
+force block size, 20-21 density and 22-23 force groups per wave (single scenes
+only).  The keys and values of describe() are part of the cache file's format
+and keep their first names: the "tile", "list" and "particles_per_lane" entries
+number the variants above.
 """
 from __future__ import annotations
 
@@ -21,7 +23,7 @@ import json
 import os
 
 DENSITY_TILES = (1280, 512, 1536, 2048, 768, 1024)
-# (LDS tile, list capacity, list entry bits)
+# (variant names of the force field: tile, list capacity, list entry bits)
 FORCE_VARIANTS = ((640, 16, 16), (768, 16, 16), (768, 24, 16), (768, 8, 32), (512, 16, 16),
                   (1024, 16, 16), (512, 8, 32), (640, 24, 16), (1024, 8, 32), (512, 24, 16))
 GRID_BLOCKS_PER_CU = (None, 1, 2, 4, 8)  # None: one block per block-size particles

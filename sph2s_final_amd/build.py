@@ -22,7 +22,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIB_NAME = "libsph2s.so"
 SOURCES = ["api.hip", "radix_sort.hip", "step.hip", "two_scale.hip", "batch.hip", "adjoint.hip",
            "walls.hip", "diagnostics.hip"]
-HEADERS = ["internal.hpp", "neighbors.hpp", "pairwalk.hpp", "batch.hpp", "walls.hpp",
+HEADERS = ["internal.hpp", "neighbors.hpp", "pairtile.hpp", "pairwalk.hpp", "batch.hpp", "walls.hpp",
            "diagnostics.hpp"]
 
 

@@ -182,7 +182,7 @@ __device__ __forceinline__ bool pair_in_range(float r2, uint32_t h2_bits_m1) {
 // some lane's queue is nearly full and at the end of each staged run.
 __global__ __launch_bounds__(kBlock) void k_adj_force(
     const float4* __restrict__ tpos, const float4* __restrict__ tvel,
-    const float2* __restrict__ aux, const float* __restrict__ rho,
+    const float4* __restrict__ ixa, const float4* __restrict__ ivb, const float* __restrict__ rho,
     const uint32_t* __restrict__ i2r, const float4* __restrict__ abar,
     const uint32_t* __restrict__ cs, const uint32_t* __restrict__ ce,
     const uint4* __restrict__ bins, const SceneParams* __restrict__ scenes,
@@ -204,7 +204,7 @@ __global__ __launch_bounds__(kBlock) void k_adj_force(
     const float h = sp.p.h, h2 = sp.p.h2;
     const float4 xi = active ? tpos[s] : make_float4(0.f, 0.f, 0.f, 0.f);
     const float4 bi = active ? abar[s] : make_float4(0.f, 0.f, 0.f, 0.f);
-    const float2 ABi = active ? aux[s] : make_float2(0.f, 1.f);
+    const float2 ABi = active ? make_float2(ixa[s].w, ivb[s].w) : make_float2(0.f, 1.f);
     const Probe pr = make_probe(g, xi.x, xi.y, xi.z);
     const uint32_t h2_bits_m1 = __float_as_uint(h2) - 1u;
     float sumA = 0.f, S1 = 0.f, S2 = 0.f;
@@ -248,10 +248,8 @@ __global__ __launch_bounds__(kBlock) void k_adj_force(
     walk_stencil_staged<kBlock, kAdjForceTile, true>(
         g, pr, cs, ce, n, active, red,
         [&](uint32_t k, uint32_t j) {
-            const float4 x = tpos[j], v = tvel[j];
-            const float2 ab = aux[j];
-            tx[k] = make_float4(x.x, x.y, x.z, ab.x);
-            tv[k] = make_float4(v.x, v.y, v.z, ab.y);
+            tx[k] = ixa[j];
+            tv[k] = ivb[j];
             ta[k] = abar[j];
         },
         [&](uint32_t t0, uint32_t t1, uint32_t) {
@@ -291,10 +289,7 @@ __global__ __launch_bounds__(kBlock) void k_adj_force(
                 const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
                 const float r2 = dx * dx + dy * dy + dz * dz;
                 if (!pair_in_range(r2, h2_bits_m1)) continue;
-                const float4 vj = tvel[j];
-                const float2 ab = aux[j];
-                pair(dx, dy, dz, r2, make_float4(xj.x, xj.y, xj.z, ab.x),
-                     make_float4(vj.x, vj.y, vj.z, ab.y), abar[j]);
+                pair(dx, dy, dz, r2, ixa[j], ivb[j], abar[j]);
             }
         },
         bins);
@@ -434,7 +429,7 @@ size_t al(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
 struct RolloutSlot {
     float4 *ipos, *ivel, *accel;  // internal x-order state; accelerations at sorted slots
     float* rho;                   // sorted slots
-    float2* iaux;                 // internal order
+    float4 *ixa, *ivb;            // (x, A), (v, B), internal order
     uint32_t *perm, *i2r, *cell_start, *cell_end;
     uint4* xbins;
     hipGraphExec_t graph = nullptr;
@@ -481,7 +476,8 @@ StepBuffers slot_buffers(const sph_rollout* r, const RolloutSlot& s) {
     StepBuffers sb = r->b->buf;
     sb.ipos = s.ipos;
     sb.ivel = s.ivel;
-    sb.iaux = s.iaux;
+    sb.ixa = s.ixa;
+    sb.ivb = s.ivb;
     sb.i2r = s.i2r;
     sb.xbins = s.xbins;
     sb.accel = s.accel;
@@ -520,7 +516,7 @@ int adjoint_step(sph_rollout* r, const RolloutSlot& s) {
     hipLaunchKernelGGL(k_adj_integrate, blocks_for(n), dim3(kBlock), 0, st, s.ipos, s.ivel,
                        s.accel, s.i2r, r->gx, r->gv, b->scenes, b->buf.n_dev, r->dt, r->abar,
                        r->gxd, r->gvd);
-    hipLaunchKernelGGL(k_adj_force, blocks_for(n), dim3(kBlock), 0, st, s.ipos, s.ivel, s.iaux,
+    hipLaunchKernelGGL(k_adj_force, blocks_for(n), dim3(kBlock), 0, st, s.ipos, s.ivel, s.ixa, s.ivb,
                        s.rho, s.i2r, r->abar, s.cell_start, s.cell_end, s.xbins, b->scenes,
                        b->buf.n_dev, r->grho, r->gxd, r->gvd, r->kacc, r->macc);
     hipLaunchKernelGGL(k_adj_density, blocks_for(n), dim3(kBlock), 0, st, s.ipos, s.ivel, r->grho,
@@ -580,7 +576,7 @@ int sph_rollout_create(const sph_config* cfgs, uint32_t n_scenes, const uint32_t
     r->n_sets = (r->n_ckpt > 1) ? 2u : 1u;
     std::vector<size_t> sizes = {al(16 * N * n_stored), al(16 * N * n_stored)};
     for (uint32_t k = 0; k < K * r->n_sets; ++k)
-        for (size_t v : {16 * N, 16 * N, 16 * N, 4 * N, 8 * N, 4 * N, 4 * N, 4 * C, 4 * C,
+        for (size_t v : {16 * N, 16 * N, 16 * N, 4 * N, 16 * N, 16 * N, 4 * N, 4 * N, 4 * C, 4 * C,
                          kXBinBytes * C})
             sizes.push_back(al(v));
     for (size_t v : {16 * N, 16 * N, 16 * N, 16 * N, 16 * N, 4 * N, 8 * N, 8 * N, 16 * S})
@@ -618,7 +614,8 @@ int sph_rollout_create(const sph_config* cfgs, uint32_t n_scenes, const uint32_t
         s.ivel = static_cast<float4*>(take());
         s.accel = static_cast<float4*>(take());
         s.rho = static_cast<float*>(take());
-        s.iaux = static_cast<float2*>(take());
+        s.ixa = static_cast<float4*>(take());
+        s.ivb = static_cast<float4*>(take());
         s.perm = static_cast<uint32_t*>(take());
         s.i2r = static_cast<uint32_t*>(take());
         s.cell_start = static_cast<uint32_t*>(take());

@@ -62,6 +62,8 @@ StepParams make_step_params(const sph_config& c, uint32_t n) {
     p.spacing = c.grid.spacing;
     p.h = c.h;
     p.h2 = c.h * c.h;
+    p.inv_h = 1.0f / p.h;
+    p.inv_h2 = 1.0f / p.h2;
     p.rest_density = c.rest_density;
     p.stiffness = c.stiffness;
     const double h = c.h;
@@ -406,7 +408,7 @@ int sph_create(const sph_config* cfg, const float* pos, const float* vel, uint32
         align_up(4 * C),  align_up(4 * C),  align_up(sort_temp),                 // cells, sort temp
         align_up(8 * N),                                                         // aux
         align_up(4),                                                             // live count
-        align_up(16 * N), align_up(16 * N), align_up(8 * N),                    // ipos ivel iaux
+        align_up(16 * N), align_up(16 * N), align_up(16 * N), align_up(16 * N),  // ipos ivel ixa ivb
         align_up(4 * N),  align_up(kXBinBytes * C)};                             // i2r xbins
     size_t total = 0;
     for (size_t b : sizes) total += b;
@@ -444,9 +446,10 @@ int sph_create(const sph_config* cfg, const float* pos, const float* vel, uint32
     s->buf.n_dev = static_cast<uint32_t*>(take(13));
     s->buf.ipos = static_cast<float4*>(take(14));
     s->buf.ivel = static_cast<float4*>(take(15));
-    s->buf.iaux = static_cast<float2*>(take(16));
-    s->buf.i2r = static_cast<uint32_t*>(take(17));
-    s->buf.xbins = static_cast<uint4*>(take(18));
+    s->buf.ixa = static_cast<float4*>(take(16));
+    s->buf.ivb = static_cast<float4*>(take(17));
+    s->buf.i2r = static_cast<uint32_t*>(take(18));
+    s->buf.xbins = static_cast<uint4*>(take(19));
     s->buf.sort_temp_bytes = sort_temp;
 
     e = hipMemsetAsync(s->arena, 0, total, s->stream);

@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "batch.hpp"
+#include "pairtile.hpp"
 
 using namespace sph;
 
@@ -113,13 +114,22 @@ int batch_alloc(const sph_config* cfgs, uint32_t n_scenes, const uint32_t* count
     b->cap = make_step_params(cfgs[0], b->n);
     b->cap.num_cells = b->total_cells;
 
+    // The neighbour passes' groups of targets start anew at each scene.
+    std::vector<uint4> groups;
+    for (uint32_t s = 0; s < n_scenes; ++s)
+        for (uint32_t i = b->part_offset[s]; i < b->part_offset[s + 1]; i += kGroupTargets)
+            groups.push_back(make_uint4(i, std::min(i + kGroupTargets, b->part_offset[s + 1]), s, 0u));
+    b->buf.n_groups = static_cast<uint32_t>(groups.size());
+
     const size_t N = b->n, C = b->total_cells;
     const size_t sort_temp = radix_sort_temp_bytes(b->n);
     const size_t sizes[] = {al(16 * N), al(16 * N), al(16 * N), al(16 * N), al(4 * N),
                             al(16 * N), al(4 * N),  al(4 * N),  al(4 * N),  al(4 * C),
                             al(4 * C),  al(sort_temp), al(8 * N), al(4),
                             al(sizeof(SceneParams) * n_scenes), al(4 * (n_scenes + 1)),
-                            al(16 * N), al(16 * N), al(8 * N), al(4 * N), al(kXBinBytes * C)};
+                            al(16 * N), al(16 * N), al(16 * N), al(16 * N), al(4 * N),
+                            al(kXBinBytes * C),
+                            al(sizeof(uint4) * groups.size())};
     size_t total = 0;
     for (size_t v : sizes) total += v;
     hipError_t e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
@@ -159,9 +169,12 @@ int batch_alloc(const sph_config* cfgs, uint32_t n_scenes, const uint32_t* count
     b->part_offset_dev = static_cast<uint32_t*>(take());
     b->buf.ipos = static_cast<float4*>(take());
     b->buf.ivel = static_cast<float4*>(take());
-    b->buf.iaux = static_cast<float2*>(take());
+    b->buf.ixa = static_cast<float4*>(take());
+    b->buf.ivb = static_cast<float4*>(take());
     b->buf.i2r = static_cast<uint32_t*>(take());
     b->buf.xbins = static_cast<uint4*>(take());
+    uint4* const groups_dev = static_cast<uint4*>(take());
+    b->buf.groups = groups_dev;
 
     e = hipMemsetAsync(b->arena, 0, total, b->stream);
     if (e == hipSuccess)
@@ -169,6 +182,9 @@ int batch_alloc(const sph_config* cfgs, uint32_t n_scenes, const uint32_t* count
                            hipMemcpyHostToDevice, b->stream);
     if (e == hipSuccess)
         e = hipMemcpyAsync(b->part_offset_dev, b->part_offset.data(), 4 * (n_scenes + 1),
+                           hipMemcpyHostToDevice, b->stream);
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(groups_dev, groups.data(), sizeof(uint4) * groups.size(),
                            hipMemcpyHostToDevice, b->stream);
     if (e == hipSuccess)
         e = hipMemcpyAsync(b->buf.n_dev, &b->n, 4, hipMemcpyHostToDevice, b->stream);

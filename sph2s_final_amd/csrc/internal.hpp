@@ -35,6 +35,7 @@ struct StepParams {
     int   dx, dy, dz;       // grid dims
     float spacing;          // cell edge
     float h, h2;            // effective radius and its square
+    float inv_h, inv_h2;    // 1 / h, 1 / h2
     float rest_density, stiffness;
     float c6m;              // mass * 315/(64 pi h^9): rho = c6m * sum (h^2-r^2)^3
     float c6m_h6;           // mass * 315/(64 pi h^3): rho = c6m_h6 * sum (1 - r^2/h^2)^3
@@ -149,7 +150,8 @@ struct StepBuffers {
     // written back at the sorted slots.
     float4* ipos;       // sorted state in the internal order
     float4* ivel;
-    float2* iaux;       // aux in the internal order (density -> force)
+    float4* ixa;        // (x, A) in the internal order (density -> force)
+    float4* ivb;        // (v, B) in the internal order
     uint32_t* i2r;      // internal slot -> sorted slot
     uint4* xbins;       // per cell: cumulative counts of its kXBins x-bins (8 bits each)
     // Boundary-particle walls (NULL: none); bacc holds each sorted slot's
@@ -162,6 +164,10 @@ struct StepBuffers {
     // The reorder pass writes the sorted copies tpos/tvel even with the
     // x-order (the two-scale step's other passes read them).
     bool keep_sorted;
+    // Batched scenes: every group of up to 32 consecutive slots of one scene
+    // as (first slot, end, scene, 0); n_groups of them.
+    const uint4* groups;
+    uint32_t n_groups;
 };
 
 // Passes of one step, in launch order.
@@ -171,8 +177,8 @@ int launch_pass(int pass, const StepParams& p, const StepBuffers& b, float dt, u
 int launch_step(const StepParams& p, const StepBuffers& b, float dt, uint32_t key_bits,
                 bool write_accel, hipStream_t stream);
 // Two-scale building blocks, in the internal x-order (b.ipos set; results at
-// the sorted slots): own-set density without the A/B finalisation, the
-// internal-order copy of the finalised A/B, and the own-set acceleration
+// the sorted slots): own-set density without the A/B finalisation, the packed
+// internal state (x, A), (v, B) from the finalised A/B, and the own-set acceleration
 // (gravity included) without integration.
 struct GridView;
 int launch_density_own_x(const StepParams& p, const StepBuffers& b, hipStream_t stream);
@@ -210,13 +216,13 @@ constexpr uint32_t kNumXcds = 8;
 #endif
 constexpr uint32_t kXcdChunk = SPH_XCD_CHUNK;
 
-__device__ __forceinline__ uint32_t xcd_local_block(uint32_t b, uint32_t nblocks) {
-    if (kXcdChunk == 0) return b;
-    const uint32_t round = kNumXcds * kXcdChunk;
+__device__ __forceinline__ uint32_t xcd_local_block(uint32_t b, uint32_t nblocks,
+                                                    uint32_t chunk = kXcdChunk) {
+    const uint32_t round = kNumXcds * chunk;
     const uint32_t full = (nblocks / round) * round;
     if (b >= full) return b;
     const uint32_t x = b % kNumXcds, k = b / kNumXcds;
-    return ((k / kXcdChunk) * kNumXcds + x) * kXcdChunk + (k % kXcdChunk);
+    return ((k / chunk) * kNumXcds + x) * chunk + (k % chunk);
 }
 
 }  // namespace sph

@@ -22,6 +22,11 @@ struct GridView {
     int dx, dy, dz;
     float h;            // search radius
     float prune_h2;     // (h (1 + 1e-3))^2
+    int reach;          // cells that h spans on one axis (pairtile.hpp)
+    int span;           // cells along x that one subgroup of targets may span (pairtile.hpp)
+    float edge;         // a target this close to its cell's y or z face looks one row further
+    uint32_t mx, my;    // n / dx = (n mx) >> (31 + lx) for n < 2^31, and likewise for dy
+    uint32_t lx, ly;
     uint32_t cell_offset;  // first global cell of this grid (batched scenes share one cell array)
 };
 
@@ -39,6 +44,25 @@ __host__ __device__ inline GridView make_grid_view(float ox, float oy, float oz,
     g.h = h;
     const float ph = h * 1.001f;
     g.prune_h2 = ph * ph;
+    // Exact arithmetic reaches ceil(h / spacing) cells; cell coordinates carry
+    // the rounding of (x - o) / spacing, at most a few units in the last place
+    // of the cell index, which `edge` covers.
+    const float cells = h / spacing;
+    const int dmax = dx > dy ? (dx > dz ? dx : dz) : (dy > dz ? dy : dz);
+    g.reach = cells < 1.0f ? 1
+                           : static_cast<int>(fminf(ceilf(cells * (1.0f - 1e-6f)),
+                                                    static_cast<float>(dmax < 1 << 24 ? dmax : 1 << 24)));
+    g.span = static_cast<int>(fminf(6.0f * cells, 1e6f));
+    // Division by multiplication (l = ceil(log2 d), m = floor(2^(31 + l) / d) + 1 is
+    // exact for 31-bit dividends).
+    auto magic = [](uint32_t d, uint32_t& m, uint32_t& l) {
+        l = 0u;
+        while ((1ull << l) < d) ++l;
+        m = static_cast<uint32_t>((1ull << (31u + l)) / d + 1u);
+    };
+    magic(static_cast<uint32_t>(dx), g.mx, g.lx);
+    magic(static_cast<uint32_t>(dy), g.my, g.ly);
+    g.edge = spacing * (1e-5f + 5e-7f * static_cast<float>(dmax));
     g.cell_offset = 0u;
     return g;
 }

@@ -20,6 +20,7 @@
 // three cells is one contiguous run of sorted particles.
 #include "neighbors.hpp"
 #include "diagnostics.hpp"
+#include "pairtile.hpp"
 #include "pairwalk.hpp"
 #include "walls.hpp"
 
@@ -171,48 +172,44 @@ __global__ __launch_bounds__(kBlock) void k_xorder(const uint32_t* __restrict__ 
 }
 
 
-#ifndef SPH_DENSITY_TILE
-#define SPH_DENSITY_TILE 1280
-#endif
-#ifndef SPH_FORCE_TILE
-#define SPH_FORCE_TILE 640
-#endif
-#ifndef SPH_LIST_CAP
-#define SPH_LIST_CAP 16
-#endif
-constexpr int kDensityTile = SPH_DENSITY_TILE;
-constexpr int kForceTile = SPH_FORCE_TILE;
-constexpr int kListCap = SPH_LIST_CAP;
-constexpr int kWavesPerBlock = kBlock / 64;
-
-// Launch variants of the neighbour passes, selected at run time by the tune
-// word (StepParams::tune; 0 = the defaults above).  Every variant computes
-// bit-identical results: the tile size only decides which runs are read from
-// LDS instead of global memory, the list capacity only when queued pairs are
-// evaluated, and the grid shape only which block processes which particles.
-//   bits 0-3   density LDS tile: 1280 (default), 512, 1536, 2048, 768, 1024
-//   bits 4-7   force tile / list capacity / list entry:  640/16/u16 (default),
-//              768/16/u16, 768/24/u16, 768/8/u32, 512/16/u16, 1024/16/u16,
-//              512/8/u32, 640/24/u16, 1024/8/u32, 512/24/u16
-//   bits 8-11  density grid:       one block per block-size particles, or a
+// Launch shapes of the neighbour passes, selected at run time by the tune word
+// (StepParams::tune; 0 = the defaults).  Every shape computes bit-identical
+// results: a target's sums depend on its group of 32 alone (pairtile.hpp), and
+// the shape only decides which wave handles which group.
+//   bits 0-3   density, bits 4-7 force: waves per block (kTileWaves)
+//   bits 8-11  density grid:       one block per its waves' groups, or a
 //   bits 12-15 force grid:         persistent grid of 1, 2, 4, 8 blocks per CU
 //                                  looping over those blocks
 //   bits 16-17 density block size, bits 18-19 force block size: 256 (0), 128
-//              (1), 512 (2) threads; a non-default block size runs the pass's
-//              default tile and queue
-//   bits 20-21 density, bits 22-23 force: particles per lane, 1 (0) or 2 (1),
-//              with the default tile, queue and block size (single scenes)
-// The block size times the particles per lane decides how many targets share
-// one staged union.
+//              (1), 512 (2) threads, as far as the block's LDS goes; a non-zero
+//              field needs waves-per-block field 0
+//   bits 20-21 density, bits 22-23 force: groups taken by a wave one after the
+//              other, 1 (0) or 2 (1), with the default block (single scenes)
+//
+// Candidates in a wave's tile: a group of a resting fluid (spacing h/2, 1M
+// particles) lists about 400, the dense cells of a collapse 600 and more.  A
+// smaller tile means more waves in flight and more parts per list.  Force at
+// 1M / 30 scenes of 4096..16384: 256 slots 223 / 98 us, 192 slots 226-239 /
+// 94-99 us, 320 slots (half the waves) 252 / 112 us; density 320 slots 144 / 67,
+// 256 slots 149 / 66, 384 slots 152 / 68 us.
+constexpr uint32_t kDensityCap = 320, kForceCap = 256;
+typedef PairTile<kDensityCap, false> DensityTile;
+typedef PairTile<kForceCap, true> ForceTile;
+// Waves share nothing but the launch: 2 and 4 waves are within 3% of each other
+// on every size, the rest is left to the tuner.
+constexpr uint32_t kTileWaves[] = {4, 1, 2, 3, 5, 6, 4, 4, 4, 4};
+constexpr uint32_t kMaxBlockLds = 64u << 10;
+// Groups in a row that one XCD takes (32, 128 and 512: within 2%).
+constexpr uint32_t kXcdChunkGroups = 128;
 constexpr uint32_t kPersistPerCu[] = {0, 1, 2, 4, 8};
+constexpr int kWavesPerBlock = kBlock / 64;
 const SceneParams* const kNoScenes = nullptr;
 
-// Internal x-order of a neighbour pass (kX): the pass reads the internal-order
+// Internal x-order of a neighbour pass: the pass reads the internal-order
 // state, trims rows with the cells' x-bins and writes results at i2r[slot].
 struct XOrder {
     const uint32_t* i2r;
     const uint4* bins;
-    float2* iaux;  // density: internal-order copy of aux for the force pass
     const float4* bacc;  // force: boundary acceleration per sorted slot (or NULL)
     // force: device error word; the integration ORs kDevErrNonFinite into it
     // when it writes a NaN or infinite position or velocity (or NULL).
@@ -221,31 +218,33 @@ struct XOrder {
 constexpr uint32_t kNumCus = 256;
 
 struct LaunchShape {
-    dim3 grid;
-    uint32_t nvb;  // blocks of `block` particles to cover
+    dim3 grid, block;
+    uint32_t nvb;     // blocks of `block` waves to cover
+    uint32_t per;     // groups per wave
+    uint32_t lds;     // bytes of LDS per block
+    uint32_t chunk;   // consecutive blocks that one XCD takes
 };
 
-inline LaunchShape launch_shape(uint32_t cap_n, uint32_t persist_idx, uint32_t block = kBlock) {
-    const uint32_t nvb = cap_n ? (cap_n + block - 1) / block : 1u;
-    uint32_t g = nvb;
+inline LaunchShape launch_shape(uint32_t groups, uint32_t tile_bytes, uint32_t waves_idx,
+                                uint32_t persist_idx, uint32_t block_idx, uint32_t per) {
+    LaunchShape s;
+    uint32_t waves = block_idx == 1 ? 2u : block_idx == 2 ? 8u : kTileWaves[std::min(waves_idx, 9u)];
+    waves = std::min(waves, kMaxBlockLds / tile_bytes);
+    s.lds = waves * tile_bytes;
+    s.per = per;
+    s.chunk = std::max(1u, kXcdChunkGroups / (waves * per));
+    s.nvb = std::max(1u, (groups + waves * per - 1) / (waves * per));
+    s.block = dim3(64u * waves);
+    uint32_t g = s.nvb;
     if (persist_idx > 0 && persist_idx < 5) {
-        g = std::min(nvb, kPersistPerCu[persist_idx] * kNumCus);
+        g = std::min(s.nvb, kPersistPerCu[persist_idx] * kNumCus);
         // A multiple of the XCD count keeps each virtual block on the XCD the
         // chunked mapping assigns it to.
         if (g > kNumXcds) g -= g % kNumXcds;
     }
-    return {dim3(g), nvb};
+    s.grid = dim3(g);
+    return s;
 }
-
-// The neighbour passes walk the nine grid rows (cy + dy, cz + dz),
-// dy, dz in {-1, 0, 1}, as block-wide phases.  In each phase every lane finds
-// its candidate run in that row (neighbors.hpp), the block takes the union of
-// the runs of its 256 consecutive sorted targets -- one contiguous index range
-// when the targets share a grid row -- and loads it into LDS with coalesced
-// reads; each lane then scans its own run out of LDS.  A run that lies outside
-// the loaded range (targets spanning distant rows, or a range larger than the
-// tile) is read from global memory instead, and so are the rare extra rows a
-// reference stencil reaches when rounding puts a bound two cells away.
 
 // The pair arithmetic below is written with explicit fused multiply-adds and
 // contraction off, so every kernel that evaluates a pair rounds it the same
@@ -259,207 +258,126 @@ __device__ __forceinline__ float dist2(float dx, float dy, float dz) {
 // Poly6 weight in units of h^2: a = 1 - r^2 / h^2 clamped to [0, 1] (one
 // fused multiply-add with the clamp modifier), so (h^2 - r^2)^3 = h^6 a^3 for
 // r < h and the term is 0 otherwise; a = 1 for r = 0.
-__device__ __forceinline__ float poly6_unit(const float4& xi, const float4& xj, float inv_h2) {
+__device__ __forceinline__ float poly6_unit(const float4& xi, const v4f& xj, float inv_h2) {
 #pragma clang fp contract(off)
     const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
     const float r2 = dist2(dx, dy, dz);
     return __builtin_amdgcn_fmed3f(__builtin_fmaf(-r2, inv_h2, 1.0f), 0.0f, 1.0f);
 }
 
-// Sum of a^3 over a run of m candidates (poly6_unit), added one at a time in
-// index order (a^2 * a + sum as one fused operation), whether the run is read
-// from global memory or staged in LDS (kQuad: LDS, read in 16-byte elements).
-constexpr int kScanGroup = 8;  // force scan: candidates loaded together before use
+// One group of targets: slots [start, end) of the internal order, all of one
+// scene.  Single scenes are cut every 32 slots; a batch
+// starts anew at each scene (its table of groups), so a scene's groups, and
+// with them its sums, are those of the scene alone.
+struct GroupRange {
+    uint32_t start, end, scene;
+};
 
-template <bool kQuad, class Load>
-__device__ __forceinline__ float poly6_run(const float4& xi, float inv_h2, uint32_t m,
-                                           Load&& load) {
-#pragma clang fp contract(off)
-    float rs = 0.0f;
-    auto add = [&](const float4& q) {
-        if (kQuad) keep_lds_quad(q);
-        const float a = poly6_unit(xi, q, inv_h2);
-        rs = __builtin_fmaf(a * a, a, rs);
-    };
-    uint32_t k = 0;
-    for (; k + 8 <= m; k += 8) {
-        float4 q[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) q[u] = load(k + u);
-#pragma unroll
-        for (int u = 0; u < 8; ++u) add(q[u]);
+template <bool kBatched>
+__device__ __forceinline__ GroupRange group_range(uint32_t group, uint32_t n,
+                                                  const uint4* __restrict__ groups,
+                                                  uint32_t n_groups) {
+    GroupRange r{0u, 0u, 0u};
+    if (kBatched) {
+        if (group < n_groups) {
+            const uint4 v = groups[group];
+            r.start = uniform_u32(v.x);
+            r.end = min(uniform_u32(v.y), n);
+            r.scene = uniform_u32(v.z);
+        }
+    } else if (group < n_groups) {
+        r.start = group * kGroupTargets;
+        r.end = min(r.start + kGroupTargets, n);
     }
-    for (; k + 4 <= m; k += 4) {
-        const float4 q0 = load(k), q1 = load(k + 1), q2 = load(k + 2), q3 = load(k + 3);
-        add(q0);
-        add(q1);
-        add(q2);
-        add(q3);
-    }
-    for (; k < m; ++k) add(load(k));
-    return rs;
+    return r;
 }
+
+// The group's targets: positions, and cells from the sorted keys (a cell's
+// slots are the same in the sorted and the internal order).
+__device__ __forceinline__ GroupTargets load_targets(const GridView& g, const GroupRange& r,
+                                                     const float4* __restrict__ tpos,
+                                                     const uint32_t* __restrict__ skeys,
+                                                     uint32_t& s) {
+    GroupTargets t;
+    s = r.start + (threadIdx.x & 31u);
+    t.active = s < r.end;
+    const uint32_t at = t.active ? s : r.start;
+    t.x = tpos[at];
+    t.key = skeys[at] - g.cell_offset;
+    return t;
+}
+
+// The sum of both lane halves' partial sums of a target.
+__device__ __forceinline__ double both_halves(double v) { return v + __shfl_xor(v, 32); }
+__device__ __forceinline__ float both_halves(float v) { return v + __shfl_xor(v, 32); }
 
 // computeDensitiesPressuresD + computeDensityCell (Solver.cu:198-229,536-599):
 // rho_i = m c6 sum_{r_ij < h} (h^2 - r_ij^2)^3, self included, evaluated as
-// (m c6 h^6) sum a^3 with a = 1 - r_ij^2 / h^2 (poly6_run).  Each run is
-// summed in plain FP32 and the run sums are combined with Kahan compensation
-// (with kKahan).  Also emits the per-particle factors the force pass needs for
-// every neighbour j: A_j = k (rho_j - rho0) / rho_j^2 and B_j = 1 / rho_j.
-// Batched scenes (kBatched): each particle's scene id is in tvel[s].w and its
-// constants come from scenes[id]; runs never leave a scene because each
-// scene's cells occupy their own range of the global cell array.
-template <bool kBatched>
-__device__ __forceinline__ void scene_constants(const SceneParams* __restrict__ scenes,
-                                                const float4* __restrict__ tvel, uint32_t s,
-                                                bool active, StepParams& p, GridView& g) {
-    if (kBatched) {
-        const uint32_t sc = active ? __float_as_uint(tvel[s].w) : 0u;
-        p = scenes[sc].p;
-        g = scenes[sc].g;
-    }
-}
-
-// kP targets per lane (particles per wavefront 64 kP): the block covers
-// the kP kB consecutive targets block0 + q kB + lane, q < kP, stages one union
-// of all their runs per row and scans each lane's targets in turn against it.
-// Each target's sums are taken exactly as with one target per lane.
-template <bool kKahan, bool kFinalize, bool kBatched, int kTile, bool kX, int kB, int kP>
-__device__ __forceinline__ void density_block(uint32_t block0, uint32_t n, float4* tile,
-                                              uint32_t* red, const float4* __restrict__ tpos,
-                                              const uint32_t* __restrict__ cs,
-                                              const uint32_t* __restrict__ ce,
-                                              const StepParams& p_in, const GridView& g_in,
-                                              float* __restrict__ rho, float2* __restrict__ aux,
-                                              const float4* __restrict__ tvel,
-                                              const SceneParams* __restrict__ scenes,
-                                              const XOrder& xo) {
-    static_assert(kP == 1 || !kBatched, "batched scenes run one target per lane");
-    StepParams p = p_in;
-    GridView g = g_in;
-    uint32_t s[kP];
-    bool active[kP];
-    float4 xi[kP];
-    Probe pr[kP];
-    float sum[kP], comp[kP];
-#pragma unroll
-    for (int q = 0; q < kP; ++q) {
-        s[q] = block0 + q * kB + threadIdx.x;
-        active[q] = s[q] < n;
-        if (kBatched) scene_constants<kBatched>(scenes, tvel, s[q], active[q], p, g);
-        xi[q] = active[q] ? tpos[s[q]] : make_float4(0.f, 0.f, 0.f, 0.f);
-        pr[q] = make_probe(g, xi[q].x, xi[q].y, xi[q].z);
-        sum[q] = 0.0f;
-        comp[q] = 0.0f;
-    }
-    const float inv_h2 = 1.0f / p.h2;
-    auto accumulate = [&](int q, float rs) {
-        if (kKahan) {
-            const float y = rs - comp[q];
-            const float t = sum[q] + y;
-            comp[q] = (t - sum[q]) - y;
-            sum[q] = t;
-        } else {
-            sum[q] += rs;
-        }
-    };
-    for (int dz = -1; dz <= 1; ++dz) {
-        for (int dy = -1; dy <= 1; ++dy) {
-            uint32_t b[kP], e[kP];
-            uint32_t lb = kEmptyCell, le = 0u;
-#pragma unroll
-            for (int q = 0; q < kP; ++q) {
-                b[q] = kEmptyCell;
-                e[q] = 0u;
-                if (active[q])
-                    probe_row<kX>(g, pr[q], cs, ce, xo.bins, n, pr[q].cy + dy, pr[q].cz + dz,
-                                  b[q], e[q]);
-                lb = min(lb, b[q]);
-                le = max(le, e[q]);
-            }
-            uint32_t ub, ue;
-            block_run_union<kB>(lb, le, red, ub, ue);
-            // Loaded range [ub, seg_e); empty when every lane's run is empty.
-            const uint32_t seg_n = (ue > ub) ? min(ue - ub, static_cast<uint32_t>(kTile)) : 0u;
-            const uint32_t seg_e = ub + seg_n;
-            __syncthreads();
-            for (uint32_t k = threadIdx.x; k < seg_n; k += kB) tile[k] = tpos[ub + k];
-            __syncthreads();
-#pragma unroll
-            for (int q = 0; q < kP; ++q) {
-                const bool staged = b[q] < e[q] && b[q] >= ub && e[q] <= seg_e;
-                if (staged) {
-                    const float4* t = tile + (b[q] - ub);
-                    accumulate(q, poly6_run<true>(xi[q], inv_h2, e[q] - b[q],
-                                                  [&](uint32_t k) { return t[k]; }));
-                }
-                if (b[q] < e[q] && !staged) {
-                    const float4* t = tpos + b[q];
-                    accumulate(q, poly6_run<false>(xi[q], inv_h2, e[q] - b[q],
-                                                   [&](uint32_t k) { return t[k]; }));
-                }
-            }
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < kP; ++q) {
-        if (!active[q]) continue;
-        for (int rz = pr[q].sz; rz <= pr[q].ez; ++rz)
-            for (int ry = pr[q].sy; ry <= pr[q].ey; ++ry) {
-                if (abs(ry - pr[q].cy) <= 1 && abs(rz - pr[q].cz) <= 1) continue;
-                uint32_t b, e;
-                probe_row<kX>(g, pr[q], cs, ce, xo.bins, n, ry, rz, b, e);
-                if (b < e) {
-                    const float4* t = tpos + b;
-                    accumulate(q, poly6_run<false>(xi[q], inv_h2, e - b,
-                                                   [&](uint32_t k) { return t[k]; }));
-                }
-            }
-        const float r = p.c6m_h6 * sum[q];
-        const uint32_t o = kX ? xo.i2r[s[q]] : s[q];
-        rho[o] = r;
-        if (kFinalize) {
-            const float inv = __builtin_amdgcn_rcpf(r);
-            const float2 ab = make_float2(p.stiffness * (r - p.rest_density) * inv * inv, inv);
-            aux[o] = ab;
-            if (kX) xo.iaux[s[q]] = ab;
-        }
-    }
-}
-
-// Occupancy targets of the neighbour passes (waves per SIMD): the density
-// pass fits 6 waves in 84 VGPRs, the force pass 5 in 102 with the
-// 640-candidate tile (LDS 28.8 KB per block); the hints make the compiler
-// allocate within those budgets.  Batched scenes take the same targets (left
-// to itself the compiler gave their force pass 116 VGPRs, 4 waves; with the
-// hints the batch step went from 1.92-1.96 to 1.89 ms).  The tension and
-// two-scale own-set forces keep the compiler's choice (94 VGPRs for the
-// latter, 5 waves already).
-constexpr int density_waves(bool /*batched*/, int ppl = 1) { return ppl == 1 ? 6 : 4; }
-constexpr int force_waves(bool /*batched*/, bool tension, bool integrate, int ppl = 1) {
-    return (!tension && integrate) ? (ppl == 1 ? 5 : 4) : 1;
-}
-
-template <bool kKahan, bool kFinalize, bool kBatched, int kTile, bool kX, int kB, int kP>
-__global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(density_waves(kBatched, kP))))
-void k_density(const float4* __restrict__ tpos,
-                                                    const uint32_t* __restrict__ cs,
-                                                    const uint32_t* __restrict__ ce,
-                                                    StepParams p_in, GridView g_in,
-                                                    const uint32_t* __restrict__ n_dev,
-                                                    float* __restrict__ rho,
-                                                    float2* __restrict__ aux,
-                                                    const float4* __restrict__ tvel,
-                                                    const SceneParams* __restrict__ scenes,
-                                                    XOrder xo, uint32_t nvb) {
-    __shared__ float4 tile[kTile];
-    __shared__ uint32_t red[2 * (kB / 64)];
+// (m c6 h^6) sum a^3 with a = 1 - r_ij^2 / h^2 (poly6_unit).  Terms are added in
+// FP32, with kKahan at most nine in a row, whose sums are added in FP64.
+// Also emits the per-particle factors the force pass needs for every
+// neighbour j: A_j = k (rho_j - rho0) / rho_j^2 and B_j = 1 / rho_j, packed
+// with the state as (x, A) and (v, B), which the force pass copies to LDS as
+// they lie.  Bound by VALU issue.
+// Against one lane per target with a block-staged tile per grid row (us, before
+// -> now): 4096 particles 29 -> 18, 30 scenes of 4096..16384 72 -> 67, one
+// million 138 -> 144.
+// Batched scenes (kBatched): a group's constants come from scenes[id]; runs
+// never leave a scene because each scene's cells occupy their own range of the
+// global cell array.
+template <bool kKahan, bool kFinalize, bool kBatched>
+__global__ __launch_bounds__(512) void k_density(
+    const float4* __restrict__ ipos, const float4* __restrict__ ivel,
+    const uint32_t* __restrict__ skeys, const uint32_t* __restrict__ cs,
+    const uint32_t* __restrict__ ce, StepParams p_in, GridView g_in,
+    const uint32_t* __restrict__ n_dev, float* __restrict__ rho, float2* __restrict__ aux,
+    float4* __restrict__ ixa, float4* __restrict__ ivb, const SceneParams* __restrict__ scenes,
+    const uint4* __restrict__ groups, uint32_t n_groups, XOrder xo, LaunchShape sh) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    const uint32_t wave = uniform_u32(threadIdx.x >> 6), waves = blockDim.x >> 6;
+    const uint32_t tile = lds_address(lds) + wave * DensityTile::kBytes;
     const uint32_t n = *n_dev;
-    for (uint32_t vb = blockIdx.x; vb < nvb; vb += gridDim.x) {
-        const uint32_t block0 = xcd_local_block(vb, nvb) * (kB * kP);
-        if (block0 < n)  // block-uniform
-            density_block<kKahan, kFinalize, kBatched, kTile, kX, kB, kP>(
-                block0, n, tile, red, tpos, cs, ce, p_in, g_in, rho, aux, tvel, scenes, xo);
+    for (uint32_t vb = blockIdx.x; vb < sh.nvb; vb += gridDim.x) {
+        const uint32_t first = (xcd_local_block(vb, sh.nvb, sh.chunk) * waves + wave) * sh.per;
+        for (uint32_t group = first; group < first + sh.per; ++group) {
+            const GroupRange gr = group_range<kBatched>(group, n, groups, n_groups);
+            if (gr.start >= gr.end) continue;
+            const StepParams& p = kBatched ? scenes[gr.scene].p : p_in;
+            const GridView& g = kBatched ? scenes[gr.scene].g : g_in;
+            uint32_t s;
+            const GroupTargets t = load_targets(g, gr, ipos, skeys, s);
+            const float4 xi = target_position(t);
+            const float inv_h2 = p.inv_h2;
+            // What the end needs, loaded before the walk.
+            const uint32_t o = xo.i2r[t.active ? s : gr.start];
+            const float4 v = kFinalize ? ivel[t.active ? s : gr.start] : t.x;
+            double sum64 = 0.0;
+            float sum32 = 0.0f;
+            walk_group<kDensityCap, false>(
+                g, t, p.inv_h, cs, ce, xo.bins, n, ipos, nullptr, tile, [&](const v4f& x) {
+#pragma clang fp contract(off)
+                    const float a = poly6_unit(xi, x, inv_h2);
+                    sum32 = __builtin_fmaf(a * a, a, sum32);
+                },
+                [&] {
+                    if (kKahan) {
+                        sum64 += static_cast<double>(sum32);
+                        sum32 = 0.0f;
+                    }
+                });
+            const float r = p.c6m_h6 * (kKahan ? static_cast<float>(both_halves(sum64))
+                                               : both_halves(sum32));
+            if (t.active && (threadIdx.x & 32u) == 0u) {
+                rho[o] = r;
+                if (kFinalize) {
+                    const float inv = __builtin_amdgcn_rcpf(r);
+                    const float A = p.stiffness * (r - p.rest_density) * inv * inv;
+                    ixa[s] = make_float4(t.x.x, t.x.y, t.x.z, A);
+                    ivb[s] = make_float4(v.x, v.y, v.z, inv);
+                    if (aux) aux[o] = make_float2(A, inv);
+                }
+            }
+        }
     }
 }
 
@@ -471,14 +389,17 @@ struct PairSums {
     float Vx = 0.f, Vy = 0.f, Vz = 0.f;
     float Tx = 0.f, Ty = 0.f, Tz = 0.f;
 
-    // xa = (x_j, A_j), vb = (v_j, B_j); requires 0 < r_ij < h.
+    // xa = (x_j, A_j), vb = (v_j, B_j), x_j finite.  Branch-free: out of range
+    // (h - r) clamps to 0, and at r = 0 it is 0 too (0 * inf is a NaN, which
+    // the clamp takes to 0), with 1 / r held finite, so such a pair adds 0.
     __device__ __forceinline__ void add(const float4& xi, const float4& vi, float ai, float h,
-                                        float h2, const float4& xa, const float4& vb) {
+                                        float h2, const v4f& xa, const v4f& vb) {
 #pragma clang fp contract(off)
         const float dx = xi.x - xa.x, dy = xi.y - xa.y, dz = xi.z - xa.z;
         const float r2 = dist2(dx, dy, dz);
-        const float inv_r = __builtin_amdgcn_rsqf(r2);
-        const float hr = __builtin_fmaf(-r2, inv_r, h);
+        const float rs = __builtin_amdgcn_rsqf(r2);
+        const float hr = __builtin_amdgcn_fmed3f(__builtin_fmaf(-r2, rs, h), 0.0f, h);
+        const float inv_r = __builtin_amdgcn_fmed3f(rs, 0.0f, 2e19f);
         const float tpr = (ai + xa.w) * hr * hr * inv_r;
         Px = __builtin_fmaf(tpr, dx, Px);
         Py = __builtin_fmaf(tpr, dy, Py);
@@ -488,7 +409,7 @@ struct PairSums {
         Vy = __builtin_fmaf(tvs, vb.y - vi.y, Vy);
         Vz = __builtin_fmaf(tvs, vb.z - vi.z, Vz);
         if (kTension) {
-            const float a = h2 - r2;
+            const float a = __builtin_amdgcn_fmed3f(h2 - r2, 0.0f, h2);
             const float w = a * a * a;
             Tx = __builtin_fmaf(w, dx, Tx);
             Ty = __builtin_fmaf(w, dy, Ty);
@@ -557,188 +478,226 @@ __device__ __forceinline__ void force_finish(const PairSums<kTension>& S, const 
 // which is f_i / rho_i of Solver.cu:231-309,601-711 with rho_i factored out,
 // fused with integrateD (Solver.cu:713-755) and the wall clamp.
 //
-// Candidates are tested as they are scanned; in-range ones are appended to
-// the lane's column of an LDS list (list[k][lane], conflict-free for any k)
-// and their pair terms are evaluated when some lane's column is full and at
-// the end of every phase, so the pair body runs for neighbours only.  The
-// tile holds (x, y, z, A_j) and (vx, vy, vz, B_j) per candidate.
-// With kIntegrate = false (two-scale own-set pass) the kernel only writes the
-// acceleration, gravity included, to accel.
-template <bool kTension, bool kIntegrate, bool kBatched, int kTile, int kCap, class TList,
-          bool kX, int kB, int kP>
-__device__ __forceinline__ void force_block(uint32_t block0, uint32_t n, float4* tp, float4* tv,
-                                            TList (*list)[kB], uint32_t* red,
-                                            const float4* __restrict__ tpos,
-                                            const float4* __restrict__ tvel,
-                                            const float2* __restrict__ aux,
-                                            const uint32_t* __restrict__ cs,
-                                            const uint32_t* __restrict__ ce,
-                                            const StepParams& p_in, const GridView& g_in,
-                                            float dt, float4* __restrict__ pos,
-                                            float4* __restrict__ vel,
-                                            float4* __restrict__ accel,
-                                            const SceneParams* __restrict__ scenes,
-                                            const XOrder& xo) {
-    static_assert(kP == 1 || !kBatched, "batched scenes run one target per lane");
-    StepParams p = p_in;
-    GridView g = g_in;
-    uint32_t s[kP];
-    bool active[kP];
-    float4 xi[kP], vi[kP];
-    float2 ai[kP];
-    Probe pr[kP];
-    PairSums<kTension> S[kP];
-#pragma unroll
-    for (int q = 0; q < kP; ++q) {
-        s[q] = block0 + q * kB + threadIdx.x;
-        active[q] = s[q] < n;
-        if (kBatched) scene_constants<kBatched>(scenes, tvel, s[q], active[q], p, g);
-        xi[q] = active[q] ? tpos[s[q]] : make_float4(0.f, 0.f, 0.f, 0.f);
-        vi[q] = active[q] ? tvel[s[q]] : make_float4(0.f, 0.f, 0.f, 0.f);
-        ai[q] = active[q] ? aux[s[q]] : make_float2(0.f, 1.f);
-        pr[q] = make_probe(g, xi[q].x, xi[q].y, xi[q].z);
+// With kIntegrate = false (two-scale own-set pass, XSPH) the kernel only writes
+// the acceleration, gravity included, to accel.
+//
+// Bound by VALU issue.  A queue of hits per lane, filled by distance tests on a
+// block-staged tile, spent most of its time on lanes waiting for the slowest
+// and on block barriers; two lanes per target with the matrix filter's masks
+// take (us, before -> now): 4096 particles 50 -> 21, 30 scenes of 4096..16384
+// 116 -> 98, one million 320 -> 223.
+template <bool kTension, bool kIntegrate, bool kBatched>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_force(
+    const float4* __restrict__ ipos, const float4* __restrict__ ivel,
+    const float4* __restrict__ ixa, const float4* __restrict__ ivb,
+    const uint32_t* __restrict__ skeys, const uint32_t* __restrict__ cs,
+    const uint32_t* __restrict__ ce, StepParams p_in, GridView g_in,
+    const uint32_t* __restrict__ n_dev, float dt, float4* __restrict__ pos,
+    float4* __restrict__ vel, float4* __restrict__ accel, const SceneParams* __restrict__ scenes,
+    const uint4* __restrict__ groups, uint32_t n_groups, XOrder xo, LaunchShape sh) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    const uint32_t wave = uniform_u32(threadIdx.x >> 6), waves = blockDim.x >> 6;
+    const uint32_t tile = lds_address(lds) + wave * ForceTile::kBytes;
+    const uint32_t n = *n_dev;
+    for (uint32_t vb = blockIdx.x; vb < sh.nvb; vb += gridDim.x) {
+        const uint32_t first = (xcd_local_block(vb, sh.nvb, sh.chunk) * waves + wave) * sh.per;
+        for (uint32_t group = first; group < first + sh.per; ++group) {
+            const GroupRange gr = group_range<kBatched>(group, n, groups, n_groups);
+            if (gr.start >= gr.end) continue;
+            const StepParams& p = kBatched ? scenes[gr.scene].p : p_in;
+            const GridView& g = kBatched ? scenes[gr.scene].g : g_in;
+            uint32_t s;
+            const GroupTargets t = load_targets(g, gr, ixa, skeys, s);
+            const float4 xi = target_position(t);
+            // What the end needs, loaded before the walk; the id and tag words
+            // come with the unpacked state.
+            const uint32_t at = t.active ? s : gr.start;
+            const float4 vi = ivb[at];
+            const uint32_t o = xo.i2r[at];
+            const float id = kIntegrate ? ipos[at].w : 0.0f, tag = kIntegrate ? ivel[at].w : 0.0f;
+            PairSums<kTension> S;
+            walk_group<kForceCap, true>(
+                g, t, p.inv_h, cs, ce, xo.bins, n, ixa, ivb, tile,
+                [&](const v4f& x, const v4f& v) { S.add(xi, vi, t.x.w, p.h, p.h2, x, v); }, [] {});
+            S.Px = both_halves(S.Px);
+            S.Py = both_halves(S.Py);
+            S.Pz = both_halves(S.Pz);
+            S.Vx = both_halves(S.Vx);
+            S.Vy = both_halves(S.Vy);
+            S.Vz = both_halves(S.Vz);
+            if (kTension) {
+                S.Tx = both_halves(S.Tx);
+                S.Ty = both_halves(S.Ty);
+                S.Tz = both_halves(S.Tz);
+            }
+            if (t.active && (threadIdx.x & 32u) == 0u) {
+                float4 x = t.x, v = vi;
+                x.w = id;
+                v.w = tag;
+                force_finish<kTension, kIntegrate>(S, p, x, v, make_float2(t.x.w, vi.w), o, xo.bacc,
+                                                   dt, pos, vel, accel, xo.err);
+            }
+        }
     }
-    uint32_t cnt = 0;
+}
 
-    auto pair = [&](int q, const float4& xa, const float4& vb) {
-        S[q].add(xi[q], vi[q], ai[q].x, p.h, p.h2, xa, vb);
+// ---- walled scenes ---------------------------------------------------------
+// One lane per target and the sums in row order: density in plain FP32 per grid
+// row with the rows' sums combined by Kahan compensation, force in one chain.
+// A boundary particle's push rises so steeply that the last bits of a velocity
+// grow by 10^4 within four steps (200,000 particles in the reference's tank:
+// largest velocity difference, over the RMS velocity, of the same sums in the
+// group walk's order 3e-4 to 1.6e-3, by the initial jitter), so scenes with
+// walls keep this order of additions and with it their trajectories.  The group
+// walk would take the four steps from 826 to 739 us.
+constexpr int kRowDensityTile = 1280, kRowForceTile = 640, kRowList = 16, kRowScan = 8;
+
+__device__ __forceinline__ v4f as_v4f(const float4& q) { return v4f{q.x, q.y, q.z, q.w}; }
+
+template <bool kKahan>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) void k_density_rows(
+    const float4* __restrict__ ipos, const float4* __restrict__ ivel,
+    const uint32_t* __restrict__ cs, const uint32_t* __restrict__ ce, StepParams p, GridView g,
+    const uint32_t* __restrict__ n_dev, float* __restrict__ rho, float4* __restrict__ ixa,
+    float4* __restrict__ ivb, XOrder xo) {
+    __shared__ float4 tile[kRowDensityTile];
+    __shared__ uint32_t red[2 * kWavesPerBlock];
+    const uint32_t n = *n_dev;
+    const uint32_t s = xcd_local_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
+    const bool active = s < n;
+    const float4 xi = active ? ipos[s] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const Probe pr = make_probe(g, xi.x, xi.y, xi.z);
+    const float inv_h2 = p.inv_h2;
+    float sum = 0.0f, comp = 0.0f;
+    auto row = [&](uint32_t m, auto&& load) {
+#pragma clang fp contract(off)
+        float rs = 0.0f;
+        auto add = [&](const float4& q) {
+            const float a = poly6_unit(xi, as_v4f(q), inv_h2);
+            rs = __builtin_fmaf(a * a, a, rs);
+        };
+        uint32_t k = 0;
+        for (; k + 8 <= m; k += 8) {
+            float4 q[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) q[u] = load(k + u);
+#pragma unroll
+            for (int u = 0; u < 8; ++u) add(q[u]);
+        }
+        for (; k < m; ++k) add(load(k));
+        if (kKahan) {
+            const float y = rs - comp;
+            const float t = sum + y;
+            comp = (t - sum) - y;
+            sum = t;
+        } else {
+            sum += rs;
+        }
+    };
+    walk_stencil_staged<kBlock, kRowDensityTile, true>(
+        g, pr, cs, ce, n, active, red, [&](uint32_t k, uint32_t j) { tile[k] = ipos[j]; },
+        [&](uint32_t t0, uint32_t t1, uint32_t) {
+            row(t1 - t0, [&](uint32_t k) {
+                const float4 q = tile[t0 + k];
+                keep_lds_quad(q);
+                return q;
+            });
+        },
+        [&](uint32_t b, uint32_t e) { row(e - b, [&](uint32_t k) { return ipos[b + k]; }); },
+        xo.bins);
+    if (!active) return;
+    const float r = p.c6m_h6 * sum;
+    const float inv = __builtin_amdgcn_rcpf(r);
+    const float4 v = ivel[s];
+    rho[xo.i2r[s]] = r;
+    ixa[s] = make_float4(xi.x, xi.y, xi.z, p.stiffness * (r - p.rest_density) * inv * inv);
+    ivb[s] = make_float4(v.x, v.y, v.z, inv);
+}
+
+// In-range candidates are appended to the lane's column of an LDS list, and
+// their pair terms evaluated, in order, when some lane's column is full and at
+// the end of every row.
+template <bool kTension>
+__global__ __launch_bounds__(kBlock) void k_force_rows(
+    const float4* __restrict__ ipos, const float4* __restrict__ ivel,
+    const float4* __restrict__ ixa, const float4* __restrict__ ivb,
+    const uint32_t* __restrict__ cs, const uint32_t* __restrict__ ce, StepParams p, GridView g,
+    const uint32_t* __restrict__ n_dev, float dt, float4* __restrict__ pos,
+    float4* __restrict__ vel, float4* __restrict__ accel, XOrder xo) {
+    __shared__ float4 tp[kRowForceTile + kRowScan];
+    __shared__ float4 tv[kRowForceTile + kRowScan];
+    __shared__ uint16_t list[kRowList][kBlock];
+    __shared__ uint32_t red[2 * kWavesPerBlock];
+    const uint32_t n = *n_dev;
+    const uint32_t s = xcd_local_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
+    const bool active = s < n;
+    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+    const float4 xi = active ? ixa[s] : zero, vi = active ? ivb[s] : zero;
+    const Probe pr = make_probe(g, xi.x, xi.y, xi.z);
+    PairSums<kTension> S;
+    uint32_t cnt = 0;
+    auto pair = [&](const float4& x, const float4& v) {
+        S.add(xi, vi, xi.w, p.h, p.h2, as_v4f(x), as_v4f(v));
     };
     // 0 < r2 < h2 as one unsigned compare: r2 >= +0 is a sum of squares, and
     // for non-negative floats the bit patterns order like the values.
     const uint32_t h2_bits_m1 = __float_as_uint(p.h2) - 1u;
-    auto in_range = [&](int q, const float4& xj) {
-        const float dx = xi[q].x - xj.x, dy = xi[q].y - xj.y, dz = xi[q].z - xj.z;
-        const float r2 = dist2(dx, dy, dz);
-        return __float_as_uint(r2) - 1u < h2_bits_m1;
+    auto in_range = [&](const float4& q) {
+        return __float_as_uint(dist2(xi.x - q.x, xi.y - q.y, xi.z - q.z)) - 1u < h2_bits_m1;
     };
-    // Queued pairs in queue order; two list entries are fetched per step so
-    // their tile reads overlap.
-    auto flush = [&](int q) {
+    // Two list entries are fetched per step so their tile reads overlap.
+    auto flush = [&]() {
         uint32_t k = 0;
         for (; k + 2 <= cnt; k += 2) {
             const uint32_t t0 = list[k][threadIdx.x], t1 = list[k + 1][threadIdx.x];
             const float4 a0 = tp[t0], b0 = tv[t0], a1 = tp[t1], b1 = tv[t1];
-            pair(q, a0, b0);
-            pair(q, a1, b1);
+            pair(a0, b0);
+            pair(a1, b1);
         }
         if (k < cnt) {
             const uint32_t t0 = list[k][threadIdx.x];
-            pair(q, tp[t0], tv[t0]);
+            pair(tp[t0], tv[t0]);
         }
         cnt = 0;
     };
-    auto global_run = [&](int q, uint32_t b, uint32_t e) {
-        for (uint32_t j = b; j < e; ++j) {
-            const float4 xj = tpos[j];
-            if (in_range(q, xj)) {
-                const float4 vj = tvel[j];
-                const float2 aj = aux[j];
-                pair(q, make_float4(xj.x, xj.y, xj.z, aj.x), make_float4(vj.x, vj.y, vj.z, aj.y));
-            }
-        }
-    };
-
-    for (int dz = -1; dz <= 1; ++dz) {
-        for (int dy = -1; dy <= 1; ++dy) {
-            uint32_t b[kP], e[kP];
-            uint32_t lb = kEmptyCell, le = 0u;
+    walk_stencil_staged<kBlock, kRowForceTile, true, kRowScan>(
+        g, pr, cs, ce, n, active, red,
+        [&](uint32_t k, uint32_t j) {
+            tp[k] = ixa[j];
+            tv[k] = ivb[j];
+        },
+        [&](uint32_t t0, uint32_t t1, uint32_t) {
+            // Whole groups of candidates are loaded before any test (the tile is
+            // padded); every candidate's index is written at the queue tail and
+            // the tail advances only for in-range ones.
+            for (uint32_t t = t0; t < t1; t += kRowScan) {
+                float4 c[kRowScan];
 #pragma unroll
-            for (int q = 0; q < kP; ++q) {
-                b[q] = kEmptyCell;
-                e[q] = 0u;
-                if (active[q])
-                    probe_row<kX>(g, pr[q], cs, ce, xo.bins, n, pr[q].cy + dy, pr[q].cz + dz,
-                                  b[q], e[q]);
-                lb = min(lb, b[q]);
-                le = max(le, e[q]);
-            }
-            uint32_t ub, ue;
-            block_run_union<kB>(lb, le, red, ub, ue);
-            const uint32_t seg_n = (ue > ub) ? min(ue - ub, static_cast<uint32_t>(kTile)) : 0u;
-            const uint32_t seg_e = ub + seg_n;
-            __syncthreads();
-            for (uint32_t k = threadIdx.x; k < seg_n; k += kB) {
-                const float4 x = tpos[ub + k];
-                const float4 v = tvel[ub + k];
-                const float2 a = aux[ub + k];
-                tp[k] = make_float4(x.x, x.y, x.z, a.x);
-                tv[k] = make_float4(v.x, v.y, v.z, a.y);
-            }
-            __syncthreads();
-            constexpr int kG = kCap >= 16 ? kScanGroup : kScanGroup / 2;
+                for (int u = 0; u < kRowScan; ++u) c[u] = tp[t + u];
 #pragma unroll
-            for (int q = 0; q < kP; ++q) {
-                const bool staged = b[q] < e[q] && b[q] >= ub && e[q] <= seg_e;
-                if (staged) {
-                    // Whole groups of candidates are loaded before any test (the
-                    // tile is padded); every candidate's index is written at the
-                    // queue tail and the tail advances only for in-range ones.
-                    const uint32_t t0 = b[q] - ub, t1 = e[q] - ub;
-                    for (uint32_t t = t0; t < t1; t += kG) {
-                        float4 c[kG];
-#pragma unroll
-                        for (int u = 0; u < kG; ++u) c[u] = tp[t + u];
-#pragma unroll
-                        for (int u = 0; u < kG; ++u) {
-                            keep_lds_quad(c[u]);
-                            const bool hit = (t + u < t1) & in_range(q, c[u]);  // no short circuit
-                            list[cnt][threadIdx.x] = static_cast<TList>(t + u);
-                            cnt += hit ? 1u : 0u;
-                        }
-                        if (__ballot(cnt > kCap - kG) != 0ull) flush(q);
-                    }
+                for (int u = 0; u < kRowScan; ++u) {
+                    keep_lds_quad(c[u]);
+                    const bool hit = (t + u < t1) & in_range(c[u]);  // no short circuit
+                    list[cnt][threadIdx.x] = static_cast<uint16_t>(t + u);
+                    cnt += hit ? 1u : 0u;
                 }
-                if (b[q] < e[q] && !staged) global_run(q, b[q], e[q]);
-                flush(q);
+                if (__ballot(cnt > kRowList - kRowScan) != 0ull) flush();
             }
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < kP; ++q) {
-        if (!active[q]) continue;
-        for (int rz = pr[q].sz; rz <= pr[q].ez; ++rz)
-            for (int ry = pr[q].sy; ry <= pr[q].ey; ++ry) {
-                if (abs(ry - pr[q].cy) <= 1 && abs(rz - pr[q].cz) <= 1) continue;
-                uint32_t b, e;
-                probe_row<kX>(g, pr[q], cs, ce, xo.bins, n, ry, rz, b, e);
-                global_run(q, b, e);
+            flush();
+        },
+        [&](uint32_t b, uint32_t e) {
+            for (uint32_t j = b; j < e; ++j) {
+                const float4 x = ixa[j];
+                if (in_range(x)) pair(x, ivb[j]);
             }
-        const uint32_t o = kX ? xo.i2r[s[q]] : s[q];
-        force_finish<kTension, kIntegrate>(S[q], p, xi[q], vi[q], ai[q], o, xo.bacc, dt, pos,
-                                           vel, accel, xo.err);
-    }
-}
-
-template <bool kTension, bool kIntegrate, bool kBatched, int kTile, int kCap, class TList,
-          bool kX, int kB, int kP>
-__global__ __launch_bounds__(kB)
-__attribute__((amdgpu_waves_per_eu(force_waves(kBatched, kTension, kIntegrate, kP))))
-void k_force(const float4* __restrict__ tpos,
-                                                  const float4* __restrict__ tvel,
-                                                  const float2* __restrict__ aux,
-                                                  const uint32_t* __restrict__ cs,
-                                                  const uint32_t* __restrict__ ce,
-                                                  StepParams p_in, GridView g_in,
-                                                  const uint32_t* __restrict__ n_dev,
-                                                  float dt, float4* __restrict__ pos,
-                                                  float4* __restrict__ vel,
-                                                  float4* __restrict__ accel,
-                                                  const SceneParams* __restrict__ scenes,
-                                                  XOrder xo, uint32_t nvb) {
-    static_assert(kCap >= kScanGroup, "a scan group queues up to kCap / 2 candidates");
-    static_assert(kTile + kScanGroup <= 65536 || sizeof(TList) == 4, "list entries index the tile");
-    __shared__ float4 tp[kTile + kScanGroup];  // padded for whole-group loads
-    __shared__ float4 tv[kTile];
-    __shared__ TList list[kCap][kB];
-    __shared__ uint32_t red[2 * (kB / 64)];
-    const uint32_t n = *n_dev;
-    for (uint32_t vb = blockIdx.x; vb < nvb; vb += gridDim.x) {
-        const uint32_t block0 = xcd_local_block(vb, nvb) * (kB * kP);
-        if (block0 < n)  // block-uniform
-            force_block<kTension, kIntegrate, kBatched, kTile, kCap, TList, kX, kB, kP>(
-                block0, n, tp, tv, list, red, tpos, tvel, aux, cs, ce, p_in, g_in, dt, pos, vel,
-                accel, scenes, xo);
-    }
+        },
+        xo.bins);
+    if (!active) return;
+    float4 x = xi, v = vi;
+    x.w = ipos[s].w;
+    v.w = ivel[s].w;
+    force_finish<kTension, true>(S, p, x, v, make_float2(xi.w, vi.w), xo.i2r[s], xo.bacc, dt, pos,
+                                 vel, accel, xo.err);
 }
 
 // XSPH integrator (integrateXSPHD, SINGLE_SCALE/Solver.cu:346-395, 757-853,
@@ -823,82 +782,38 @@ __global__ __launch_bounds__(kBlock) void k_xsph_integrate(
     vel[s] = make_float4(vx, vy, vz, vi.w);
 }
 
-// Variant dispatch.  Only the passes of the single-scale and batched steps
-// (density with aux, force with integration and no tension) are tunable; the
-// other instantiations use the defaults.  The single-scale and batched passes
-// (density with aux, force with integration) run in the internal x-order; the
-// two-scale own-set passes (neither) in the sorted order.
-// Block size of a tunable pass from its tune-word bits: 0 = 256, 1 = 128,
-// 2 = 512 threads; 3 is invalid, refused by tune_word_valid.
-
-template <bool kKahan, bool kFinalize, bool kBatched, bool kX = kFinalize, class... A>
-void launch_density(uint32_t tune, uint32_t cap_n, hipStream_t st, A... args) {
-    // The step's density pass and the two-scale own-set pass (x-order, no
-    // finalisation) take the tune word.
-    constexpr bool kTunable = kFinalize || kX;
-    const uint32_t v = kTunable ? (tune & 0xFu) : 0u;
-    const uint32_t bv = kTunable ? ((tune >> 16) & 0x3u) : 0u;
-    const uint32_t pv = (kTunable && !kBatched) ? ((tune >> 20) & 0x3u) : 0u;
-    const uint32_t persist = kTunable ? ((tune >> 8) & 0xFu) : 0u;
-#define SPH_DENSITY_VARIANT(TILE, B, P)                                                         \
-    do {                                                                                        \
-        const LaunchShape sh = launch_shape(cap_n, persist, (B) * (P));                         \
-        hipLaunchKernelGGL((k_density<kKahan, kFinalize, kBatched, TILE, kX, B, P>), sh.grid,  \
-                           dim3(B), 0, st, args..., sh.nvb);                                    \
-    } while (0)
-    if constexpr (kTunable) {
-        if constexpr (!kBatched)
-            if (pv == 1) { SPH_DENSITY_VARIANT(kDensityTile, kBlock, 2); return; }
-        if (bv == 1) { SPH_DENSITY_VARIANT(kDensityTile, 128, 1); return; }
-        if (bv == 2) { SPH_DENSITY_VARIANT(kDensityTile, 512, 1); return; }
-        switch (v) {
-            case 1: SPH_DENSITY_VARIANT(512, kBlock, 1); return;
-            case 2: SPH_DENSITY_VARIANT(1536, kBlock, 1); return;
-            case 3: SPH_DENSITY_VARIANT(2048, kBlock, 1); return;
-            case 4: SPH_DENSITY_VARIANT(768, kBlock, 1); return;
-            case 5: SPH_DENSITY_VARIANT(1024, kBlock, 1); return;
-            default: break;
-        }
-    }
-    SPH_DENSITY_VARIANT(kDensityTile, kBlock, 1);
-#undef SPH_DENSITY_VARIANT
+// Launches.  All density and force passes run in the internal x-order.  The
+// group passes take the tune word (the tension forms run the default shape);
+// walled scenes have one shape.
+inline uint32_t group_count(uint32_t cap_n, uint32_t n_groups) {
+    return n_groups ? n_groups : (cap_n + kGroupTargets - 1) / kGroupTargets;
 }
 
-template <bool kTension, bool kIntegrate, bool kBatched, bool kX = kIntegrate, class... A>
-void launch_force(uint32_t tune, uint32_t cap_n, hipStream_t st, A... args) {
-    // The step's force pass and the two-scale own-set pass (x-order, no
-    // integration) take the tune word; the tension forms run the default.
-    constexpr bool kTunable = !kTension && (kIntegrate || kX);
-    const uint32_t v = kTunable ? ((tune >> 4) & 0xFu) : 0u;
-    const uint32_t bv = kTunable ? ((tune >> 18) & 0x3u) : 0u;
-    const uint32_t pv = (kTunable && !kBatched) ? ((tune >> 22) & 0x3u) : 0u;
-    const uint32_t persist = kTunable ? ((tune >> 12) & 0xFu) : 0u;
-#define SPH_FORCE_VARIANT(TILE, CAP, TLIST, B, P)                                               \
-    do {                                                                                        \
-        const LaunchShape sh = launch_shape(cap_n, persist, (B) * (P));                         \
-        hipLaunchKernelGGL((k_force<kTension, kIntegrate, kBatched, TILE, CAP, TLIST, kX, B, P>), \
-                           sh.grid, dim3(B), 0, st, args..., sh.nvb);                           \
-    } while (0)
-    if constexpr (kTunable) {
-        if constexpr (!kBatched)
-            if (pv == 1) { SPH_FORCE_VARIANT(kForceTile, kListCap, uint16_t, kBlock, 2); return; }
-        if (bv == 1) { SPH_FORCE_VARIANT(kForceTile, kListCap, uint16_t, 128, 1); return; }
-        if (bv == 2) { SPH_FORCE_VARIANT(kForceTile, kListCap, uint16_t, 512, 1); return; }
-        switch (v) {
-            case 1: SPH_FORCE_VARIANT(768, 16, uint16_t, kBlock, 1); return;
-            case 2: SPH_FORCE_VARIANT(768, 24, uint16_t, kBlock, 1); return;
-            case 3: SPH_FORCE_VARIANT(768, 8, uint32_t, kBlock, 1); return;
-            case 4: SPH_FORCE_VARIANT(512, 16, uint16_t, kBlock, 1); return;
-            case 5: SPH_FORCE_VARIANT(1024, 16, uint16_t, kBlock, 1); return;
-            case 6: SPH_FORCE_VARIANT(512, 8, uint32_t, kBlock, 1); return;
-            case 7: SPH_FORCE_VARIANT(640, 24, uint16_t, kBlock, 1); return;
-            case 8: SPH_FORCE_VARIANT(1024, 8, uint32_t, kBlock, 1); return;
-            case 9: SPH_FORCE_VARIANT(512, 24, uint16_t, kBlock, 1); return;
-            default: break;
-        }
-    }
-    SPH_FORCE_VARIANT(kForceTile, kListCap, uint16_t, kBlock, 1);
-#undef SPH_FORCE_VARIANT
+template <bool kKahan, bool kFinalize, bool kBatched>
+void launch_density(uint32_t tune, uint32_t cap_n, hipStream_t st, const StepBuffers& b,
+                    const StepParams& p, const GridView& g, float2* aux, const SceneParams* scenes,
+                    const XOrder& xo) {
+    const uint32_t n_groups = group_count(cap_n, kBatched ? b.n_groups : 0u);
+    const LaunchShape sh =
+        launch_shape(n_groups, DensityTile::kBytes, tune & 0xFu, (tune >> 8) & 0xFu,
+                     (tune >> 16) & 0x3u, kBatched ? 1u : 1u + ((tune >> 20) & 1u));
+    hipLaunchKernelGGL((k_density<kKahan, kFinalize, kBatched>), sh.grid, sh.block, sh.lds, st,
+                       b.ipos, b.ivel, b.skeys, b.cell_start, b.cell_end, p, g, b.n_dev, b.rho, aux,
+                       b.ixa, b.ivb, scenes, b.groups, n_groups, xo, sh);
+}
+
+template <bool kTension, bool kIntegrate, bool kBatched>
+void launch_force(uint32_t tune, uint32_t cap_n, hipStream_t st, const StepBuffers& b,
+                  const StepParams& p, const GridView& g, float dt, float4* pos, float4* vel,
+                  float4* accel, const SceneParams* scenes, const XOrder& xo) {
+    if (kTension) tune = 0u;
+    const uint32_t n_groups = group_count(cap_n, kBatched ? b.n_groups : 0u);
+    const LaunchShape sh =
+        launch_shape(n_groups, ForceTile::kBytes, (tune >> 4) & 0xFu, (tune >> 12) & 0xFu,
+                     (tune >> 18) & 0x3u, kBatched ? 1u : 1u + ((tune >> 22) & 1u));
+    hipLaunchKernelGGL((k_force<kTension, kIntegrate, kBatched>), sh.grid, sh.block, sh.lds, st,
+                       b.ipos, b.ivel, b.ixa, b.ivb, b.skeys, b.cell_start, b.cell_end, p, g,
+                       b.n_dev, dt, pos, vel, accel, scenes, b.groups, n_groups, xo, sh);
 }
 
 __global__ void k_pack_state(const float* __restrict__ pxyz, const float* __restrict__ vxyz,
@@ -922,6 +837,11 @@ __global__ void k_export_aos(const float4* __restrict__ src, uint32_t n, float* 
 }
 
 inline dim3 blocks_for(uint32_t n) { return dim3((n + kBlock - 1) / kBlock); }
+
+// Whether a step's sums are taken in row order (k_density_rows).
+inline bool row_order(const StepParams& p, const StepBuffers& b) {
+    return b.walls && b.bacc && !(p.flags & SPH_FLAG_XSPH);
+}
 
 }  // namespace
 
@@ -970,14 +890,22 @@ int launch_pass(int pass, const StepParams& p, const StepBuffers& b, float dt,
         }
         case kPassDensity:
             if (!b.ipos) return set_error(SPH_ERR_INVALID_ARGUMENT, "step buffers lack the x-order");
-            if (p.flags & SPH_FLAG_KAHAN)
-                launch_density<true, true, false>(p.tune, p.n, stream, b.ipos, b.cell_start,
-                                                  b.cell_end, p, g, b.n_dev, b.rho, b.aux, b.ivel,
-                                                  kNoScenes, XOrder{b.i2r, b.xbins, b.iaux});
+            if (row_order(p, b)) {
+                hipLaunchKernelGGL((p.flags & SPH_FLAG_KAHAN) ? k_density_rows<true>
+                                                              : k_density_rows<false>,
+                                   blocks_for(p.n), dim3(kBlock), 0, stream, b.ipos, b.ivel,
+                                   b.cell_start, b.cell_end, p, g, b.n_dev, b.rho, b.ixa, b.ivb,
+                                   XOrder{b.i2r, b.xbins});
+                break;
+            }
+            // Only the XSPH pass reads A, B in the sorted order.
+            if (float2* const aux = (p.flags & SPH_FLAG_XSPH) ? b.aux : nullptr;
+                p.flags & SPH_FLAG_KAHAN)
+                launch_density<true, true, false>(p.tune, p.n, stream, b, p, g, aux, kNoScenes,
+                                                 XOrder{b.i2r, b.xbins});
             else
-                launch_density<false, true, false>(p.tune, p.n, stream, b.ipos, b.cell_start,
-                                                   b.cell_end, p, g, b.n_dev, b.rho, b.aux, b.ivel,
-                                                   kNoScenes, XOrder{b.i2r, b.xbins, b.iaux});
+                launch_density<false, true, false>(p.tune, p.n, stream, b, p, g, aux, kNoScenes,
+                                                 XOrder{b.i2r, b.xbins});
             break;
         case kPassForce: {
             float4* acc = write_accel ? b.accel : nullptr;
@@ -995,32 +923,32 @@ int launch_pass(int pass, const StepParams& p, const StepBuffers& b, float dt,
             if (p.flags & SPH_FLAG_XSPH) {
                 // Accelerations of every particle first (sorted order), then
                 // the XSPH integration, which reads its neighbours' ones.
-                const XOrder xa{nullptr, nullptr, nullptr, walls ? b.bacc : nullptr};
+                const XOrder xa{b.i2r, b.xbins, walls ? b.bacc : nullptr};
                 float4* const no_state = nullptr;
                 if (p.tens != 0.0f)
-                    launch_force<true, false, false>(0u, p.n, stream, b.tpos, b.tvel, b.aux,
-                                                     b.cell_start, b.cell_end, p, g, b.n_dev, 0.0f,
-                                                     no_state, no_state, b.accel, kNoScenes, xa);
+                    launch_force<true, false, false>(p.tune, p.n, stream, b, p, g, 0.0f, no_state,
+                                                    no_state, b.accel, kNoScenes, xa);
                 else
-                    launch_force<false, false, false>(0u, p.n, stream, b.tpos, b.tvel, b.aux,
-                                                      b.cell_start, b.cell_end, p, g, b.n_dev,
-                                                      0.0f, no_state, no_state, b.accel, kNoScenes,
-                                                      xa);
+                    launch_force<false, false, false>(p.tune, p.n, stream, b, p, g, 0.0f, no_state,
+                                                    no_state, b.accel, kNoScenes, xa);
                 hipLaunchKernelGGL(k_xsph_integrate, blocks_for(p.n), dim3(kBlock), 0, stream,
                                    b.tpos, b.tvel, b.aux, b.accel, b.cell_start, b.cell_end, p, g,
                                    b.n_dev, dt, b.pos, b.vel);
                 break;
             }
-            const XOrder xo{b.i2r, b.xbins, nullptr, walls ? b.bacc : nullptr,
+            const XOrder xo{b.i2r, b.xbins, walls ? b.bacc : nullptr,
                             radix_sort_error_word(b.sort_temp)};
-            if (p.tens != 0.0f)
-                launch_force<true, true, false>(p.tune, p.n, stream, b.ipos, b.ivel, b.iaux,
-                                                b.cell_start, b.cell_end, p, g, b.n_dev, dt, b.pos,
-                                                b.vel, acc, kNoScenes, xo);
+            if (row_order(p, b))
+                hipLaunchKernelGGL((p.tens != 0.0f) ? k_force_rows<true> : k_force_rows<false>,
+                                   blocks_for(p.n), dim3(kBlock), 0, stream, b.ipos, b.ivel, b.ixa,
+                                   b.ivb, b.cell_start, b.cell_end, p, g, b.n_dev, dt, b.pos, b.vel,
+                                   acc, xo);
+            else if (p.tens != 0.0f)
+                launch_force<true, true, false>(p.tune, p.n, stream, b, p, g, dt, b.pos, b.vel, acc,
+                                               kNoScenes, xo);
             else
-                launch_force<false, true, false>(p.tune, p.n, stream, b.ipos, b.ivel, b.iaux,
-                                                 b.cell_start, b.cell_end, p, g, b.n_dev, dt,
-                                                 b.pos, b.vel, acc, kNoScenes, xo);
+                launch_force<false, true, false>(p.tune, p.n, stream, b, p, g, dt, b.pos, b.vel, acc,
+                                               kNoScenes, xo);
             break;
         }
         default:
@@ -1047,36 +975,52 @@ int launch_density_own_x(const StepParams& p, const StepBuffers& b, hipStream_t 
     if (p.n == 0) return SPH_OK;
     if (!b.ipos) return set_error(SPH_ERR_INVALID_ARGUMENT, "step buffers lack the x-order");
     const GridView g = make_grid_view(p.ox, p.oy, p.oz, p.spacing, p.dx, p.dy, p.dz, p.h);
-    const XOrder xo{b.i2r, b.xbins, nullptr};
+    const XOrder xo{b.i2r, b.xbins};
     if (p.flags & SPH_FLAG_KAHAN)
-        launch_density<true, false, false, true>(p.tune, p.n, stream, b.ipos, b.cell_start,
-                                                 b.cell_end, p, g, b.n_dev, b.rho, b.aux, b.ivel,
-                                                 kNoScenes, xo);
+        launch_density<true, false, false>(p.tune, p.n, stream, b, p, g, nullptr, kNoScenes, xo);
     else
-        launch_density<false, false, false, true>(p.tune, p.n, stream, b.ipos, b.cell_start,
-                                                  b.cell_end, p, g, b.n_dev, b.rho, b.aux,
-                                                  b.ivel, kNoScenes, xo);
+        launch_density<false, false, false>(p.tune, p.n, stream, b, p, g, nullptr, kNoScenes, xo);
     SPH_HIP(hipGetLastError());
     return SPH_OK;
 }
 
+// The packed internal state of the force pass from the final A, B: (x, A) and
+// (v, B).
 __global__ __launch_bounds__(kBlock) void k_gather_aux(const float2* __restrict__ aux,
                                                        const uint32_t* __restrict__ i2r,
                                                        const uint32_t* __restrict__ n_dev,
-                                                       float2* __restrict__ iaux) {
+                                                       const float4* __restrict__ ipos,
+                                                       const float4* __restrict__ ivel,
+                                                       float4* __restrict__ ixa,
+                                                       float4* __restrict__ ivb) {
     const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
-    if (s < *n_dev) iaux[s] = aux[i2r[s]];
+    if (s >= *n_dev) return;
+    const float4 x = ipos[s], v = ivel[s];
+    const float2 a = aux[i2r[s]];
+    ixa[s] = make_float4(x.x, x.y, x.z, a.x);
+    ivb[s] = make_float4(v.x, v.y, v.z, a.y);
 }
 
 int launch_gather_aux(const StepParams& p, const StepBuffers& b, hipStream_t stream) {
-    return launch_gather_x(b.aux, b.i2r, b.n_dev, p.n, b.iaux, stream);
+    if (p.n == 0) return SPH_OK;
+    hipLaunchKernelGGL(k_gather_aux, blocks_for(p.n), dim3(kBlock), 0, stream, b.aux, b.i2r,
+                       b.n_dev, b.ipos, b.ivel, b.ixa, b.ivb);
+    SPH_HIP(hipGetLastError());
+    return SPH_OK;
+}
+
+__global__ __launch_bounds__(kBlock) void k_gather_x(const float2* __restrict__ src,
+                                                     const uint32_t* __restrict__ i2r,
+                                                     const uint32_t* __restrict__ n_dev,
+                                                     float2* __restrict__ dst) {
+    const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
+    if (s < *n_dev) dst[s] = src[i2r[s]];
 }
 
 int launch_gather_x(const float2* src, const uint32_t* i2r, const uint32_t* n_dev, uint32_t cap,
                     float2* dst, hipStream_t stream) {
     if (cap == 0) return SPH_OK;
-    hipLaunchKernelGGL(k_gather_aux, blocks_for(cap), dim3(kBlock), 0, stream, src, i2r, n_dev,
-                       dst);
+    hipLaunchKernelGGL(k_gather_x, blocks_for(cap), dim3(kBlock), 0, stream, src, i2r, n_dev, dst);
     SPH_HIP(hipGetLastError());
     return SPH_OK;
 }
@@ -1086,15 +1030,13 @@ int launch_force_own_x(const StepParams& p, const GridView& g, const StepBuffers
     if (p.n == 0) return SPH_OK;
     if (!b.ipos) return set_error(SPH_ERR_INVALID_ARGUMENT, "step buffers lack the x-order");
     float4* const no_state = nullptr;
-    const XOrder xo{b.i2r, b.xbins, nullptr, nullptr};
+    const XOrder xo{b.i2r, b.xbins};
     if (p.tens != 0.0f)
-        launch_force<true, false, false, true>(p.tune, p.n, stream, b.ipos, b.ivel, b.iaux,
-                                               b.cell_start, b.cell_end, p, g, b.n_dev, 0.0f,
-                                               no_state, no_state, accel_own, kNoScenes, xo);
+        launch_force<true, false, false>(p.tune, p.n, stream, b, p, g, 0.0f, no_state, no_state,
+                                        accel_own, kNoScenes, xo);
     else
-        launch_force<false, false, false, true>(p.tune, p.n, stream, b.ipos, b.ivel, b.iaux,
-                                                b.cell_start, b.cell_end, p, g, b.n_dev, 0.0f,
-                                                no_state, no_state, accel_own, kNoScenes, xo);
+        launch_force<false, false, false>(p.tune, p.n, stream, b, p, g, 0.0f, no_state, no_state,
+                                        accel_own, kNoScenes, xo);
     SPH_HIP(hipGetLastError());
     return SPH_OK;
 }
@@ -1198,26 +1140,22 @@ int launch_batch_pass(int pass, const StepParams& cap, const StepBuffers& b,
         case kPassDensity:
             if (!b.ipos) return set_error(SPH_ERR_INVALID_ARGUMENT, "step buffers lack the x-order");
             if (kahan)
-                launch_density<true, true, true>(cap.tune, cap.n, stream, b.ipos, b.cell_start,
-                                                 b.cell_end, cap, g0, b.n_dev, b.rho, b.aux,
-                                                 b.ivel, scenes, XOrder{b.i2r, b.xbins, b.iaux});
+                launch_density<true, true, true>(cap.tune, cap.n, stream, b, cap, g0, nullptr, scenes,
+                                                XOrder{b.i2r, b.xbins});
             else
-                launch_density<false, true, true>(cap.tune, cap.n, stream, b.ipos, b.cell_start,
-                                                  b.cell_end, cap, g0, b.n_dev, b.rho, b.aux,
-                                                  b.ivel, scenes, XOrder{b.i2r, b.xbins, b.iaux});
+                launch_density<false, true, true>(cap.tune, cap.n, stream, b, cap, g0, nullptr, scenes,
+                                                XOrder{b.i2r, b.xbins});
             break;
         case kPassForce: {
             if (!b.ipos) return set_error(SPH_ERR_INVALID_ARGUMENT, "step buffers lack the x-order");
             float4* acc = write_accel ? b.accel : nullptr;
-            const XOrder xo{b.i2r, b.xbins, nullptr, nullptr, radix_sort_error_word(b.sort_temp)};
+            const XOrder xo{b.i2r, b.xbins, nullptr, radix_sort_error_word(b.sort_temp)};
             if (tension)
-                launch_force<true, true, true>(cap.tune, cap.n, stream, b.ipos, b.ivel, b.iaux,
-                                               b.cell_start, b.cell_end, cap, g0, b.n_dev, dt,
-                                               b.pos, b.vel, acc, scenes, xo);
+                launch_force<true, true, true>(cap.tune, cap.n, stream, b, cap, g0, dt, b.pos, b.vel, acc,
+                                              scenes, xo);
             else
-                launch_force<false, true, true>(cap.tune, cap.n, stream, b.ipos, b.ivel, b.iaux,
-                                                b.cell_start, b.cell_end, cap, g0, b.n_dev, dt,
-                                                b.pos, b.vel, acc, scenes, xo);
+                launch_force<false, true, true>(cap.tune, cap.n, stream, b, cap, g0, dt, b.pos, b.vel, acc,
+                                              scenes, xo);
             break;
         }
         default:

@@ -717,7 +717,8 @@ __global__ __launch_bounds__(kBlock) void k_blend_density(
 template <bool kTension>
 __global__ __launch_bounds__(kBlock) void k_blend_force_integrate(
     const float4* __restrict__ ipos_a, const float4* __restrict__ ivel_a,
-    const float2* __restrict__ iaux_a, const float2* __restrict__ ibl_a,
+    const float4* __restrict__ ixa_a, const float4* __restrict__ ivb_a,
+    const float2* __restrict__ ibl_a,
     const uint32_t* __restrict__ cs_a, const uint32_t* __restrict__ ce_a,
     const uint4* __restrict__ bins_a, const uint32_t* __restrict__ i2r_a,
     const uint32_t* __restrict__ n_a, GridView ga, StepParams pa, CrossParams c,
@@ -733,7 +734,7 @@ __global__ __launch_bounds__(kBlock) void k_blend_force_integrate(
     const bool active = s < na;
     const float4 xi = active ? ipos_a[s] : make_float4(0.f, 0.f, 0.f, 0.f);
     const float4 vi = active ? ivel_a[s] : make_float4(0.f, 0.f, 0.f, 0.f);
-    const float2 ai = active ? iaux_a[s] : make_float2(0.f, 1.f);
+    const float2 ai = active ? make_float2(ixa_a[s].w, ivb_a[s].w) : make_float2(0.f, 1.f);
     const Probe pr = make_probe(ga, xi.x, xi.y, xi.z);
     float Px = 0.f, Py = 0.f, Pz = 0.f, Vx = 0.f, Vy = 0.f, Vz = 0.f, Tx = 0.f, Ty = 0.f,
           Tz = 0.f;
@@ -764,10 +765,8 @@ __global__ __launch_bounds__(kBlock) void k_blend_force_integrate(
     walk_stencil_staged<kBlock, kBlendForceTile, true>(
         ga, pr, cs_a, ce_a, na, active, red,
         [&](uint32_t k, uint32_t j) {
-            const float4 x = ipos_a[j], v = ivel_a[j];
-            const float2 a = iaux_a[j];
-            tx[k] = make_float4(x.x, x.y, x.z, a.x);
-            tv[k] = make_float4(v.x, v.y, v.z, a.y);
+            tx[k] = ixa_a[j];
+            tv[k] = ivb_a[j];
             tl[k] = ibl_a[j].x;
         },
         [&](uint32_t t0, uint32_t t1, uint32_t) {
@@ -778,12 +777,7 @@ __global__ __launch_bounds__(kBlock) void k_blend_force_integrate(
             }
         },
         [&](uint32_t b, uint32_t e) {
-            for (uint32_t j = b; j < e; ++j) {
-                const float4 x = ipos_a[j], v = ivel_a[j];
-                const float2 a = iaux_a[j];
-                pair(make_float4(x.x, x.y, x.z, a.x), make_float4(v.x, v.y, v.z, a.y),
-                     ibl_a[j].x);
-            }
+            for (uint32_t j = b; j < e; ++j) pair(ixa_a[j], ivb_a[j], ibl_a[j].x);
         },
         bins_a);
     if (!active) return;
@@ -1607,14 +1601,14 @@ int launch_blended_passes(sph_two_scale* t, const StepParams* P, const GridView*
         if (rc != SPH_OK) return rc;
         if (P[r].tens != 0.0f)
             hipLaunchKernelGGL(k_blend_force_integrate<true>, blocks_for(A.cap), dim3(kBlock), 0,
-                               s, A.buf.ipos, A.buf.ivel, A.buf.iaux, A.iblend, A.buf.cell_start,
-                               A.buf.cell_end, A.buf.xbins, A.buf.i2r, A.buf.n_dev, G[r], P[r], c,
+                               s, A.buf.ipos, A.buf.ivel, A.buf.ixa, A.buf.ivb, A.iblend,
+                               A.buf.cell_start, A.buf.cell_end, A.buf.xbins, A.buf.i2r, A.buf.n_dev, G[r], P[r], c,
                                A.accel, wall_acc(t, r), dt, inc, A.buf.pos, A.buf.vel, A.nblend,
                                acc);
         else
             hipLaunchKernelGGL(k_blend_force_integrate<false>, blocks_for(A.cap), dim3(kBlock), 0,
-                               s, A.buf.ipos, A.buf.ivel, A.buf.iaux, A.iblend, A.buf.cell_start,
-                               A.buf.cell_end, A.buf.xbins, A.buf.i2r, A.buf.n_dev, G[r], P[r], c,
+                               s, A.buf.ipos, A.buf.ivel, A.buf.ixa, A.buf.ivb, A.iblend,
+                               A.buf.cell_start, A.buf.cell_end, A.buf.xbins, A.buf.i2r, A.buf.n_dev, G[r], P[r], c,
                                A.accel, wall_acc(t, r), dt, inc, A.buf.pos, A.buf.vel, A.nblend,
                                acc);
     }
@@ -2025,7 +2019,8 @@ int sph2_create(const sph_config* cfg, const float region_lo[3], const float reg
         add(4ull * kWalkSegments * walk_segment_cap(S.cap));  // walk list segments
         add(16 * N);                               // ipos
         add(16 * N);                               // ivel
-        add(8 * N);                                // iaux
+        add(16 * N);                               // ixa
+        add(16 * N);                               // ivb
         add(4 * N);                                // i2r
         add(kXBinBytes * C);                       // xbins
         add(8 * N);                                // iblend
@@ -2091,7 +2086,8 @@ int sph2_create(const sph_config* cfg, const float region_lo[3], const float reg
         S.walk = static_cast<uint32_t*>(take());
         S.buf.ipos = static_cast<float4*>(take());
         S.buf.ivel = static_cast<float4*>(take());
-        S.buf.iaux = static_cast<float2*>(take());
+        S.buf.ixa = static_cast<float4*>(take());
+        S.buf.ivb = static_cast<float4*>(take());
         S.buf.i2r = static_cast<uint32_t*>(take());
         S.buf.xbins = static_cast<uint4*>(take());
         S.iblend = static_cast<float2*>(take());
