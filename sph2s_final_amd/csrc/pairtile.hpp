@@ -287,8 +287,10 @@ __device__ __forceinline__ void walk_group(const GridView& g, const GroupTargets
     typedef PairTile<kCap, kVelocity> T;
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t half = lane >> 5;
-    // Row m of a filter product reads slot 2 r + q of its 32, where (q, r) are
-    // the lane half and accumulator that receive row m: a lane's 32 mask bits
+    // A lane half converts 32 of 64 candidates; the first product takes the lower
+    // half's (the upper half's target operand is 0), the second the upper's.
+    // Row m of a product reads slot 2 r + q of its 32, where (q, r) are the lane
+    // half and accumulator that receive row m: a lane's 32 mask bits
     // are the even (half 0) or odd slots of 64, so a target's hits, which lie
     // together along a row, fall evenly on its two lanes.
     const uint32_t m = lane & 31u;
@@ -299,19 +301,20 @@ __device__ __forceinline__ void walk_group(const GridView& g, const GroupTargets
         // Fills a tile to whole words: out of the members' range, yet finite in
         // FP16 (an infinity would make the products NaN, and its sign a hit).
         const v4f far = {s.ox + 100.0f * __builtin_amdgcn_rcpf(inv_h), s.oy, s.oz, 0.0f};
-        // Target operands of the filter, in units of h: columns
-        // (-2 x, -2 y, -2 z, c) and (1, c', 0, 0) against rows (x, y, z, 1) and
-        // (|x|^2, 1, 0, 0), with c + c' = |x|^2 - 1 - margin.
+        // Target operands of the filter, in units of h: columns (-2 x, -2 y, -2 z, 1)
+        // against rows (x, y, z, |x|^2), added to the column's |x|^2 - 1 - margin.
         const float sx = -s.ox * inv_h, sy = -s.oy * inv_h, sz = -s.oz * inv_h;
         const float ix = __builtin_fmaf(t.x.x, inv_h, sx), iy = __builtin_fmaf(t.x.y, inv_h, sy),
                     iz = __builtin_fmaf(t.x.z, inv_h, sz);
         const float qi = ix * ix + iy * iy + iz * iz;
-        const float ci = s.member && qi < 1e4f ? qi - 1.0f - group_margin(qi) : 6e4f;
-        const _Float16 c_hi = static_cast<_Float16>(ci);
-        const _Float16 c_lo = static_cast<_Float16>(ci - static_cast<float>(c_hi));
-        const v4h col = half ? v4h{1, c_lo, 0, 0}
-                             : v4h{static_cast<_Float16>(-2.0f * ix), static_cast<_Float16>(-2.0f * iy),
-                                   static_cast<_Float16>(-2.0f * iz), c_hi};
+        const float ci = s.member && qi < 1e4f ? qi - 1.0f - group_margin(qi) : 1e30f;
+        const v4h none = {0, 0, 0, 0},
+                  col = {static_cast<_Float16>(-2.0f * ix), static_cast<_Float16>(-2.0f * iy),
+                         static_cast<_Float16>(-2.0f * iz), 1},
+                  cols[2] = {half ? none : col, half ? col : none};
+        v16f base;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) base[r] = ci;
         const uint32_t rows = static_cast<uint32_t>(s.ny) * static_cast<uint32_t>(s.nz);
         for (uint32_t row0 = 0; row0 < rows; row0 += 64u) {
             uint32_t rb = 0u, re = 0u;
@@ -364,25 +367,27 @@ __device__ __forceinline__ void walk_group(const GridView& g, const GroupTargets
                 wait_vmem();
                 wave_sync();
                 for (uint32_t w = 0; w < words; ++w) {
+                    const uint32_t at = tile + 16u * (64u * w + 32u * half + slot_of_row);
+                    const v4f x = lds_read<v4f>(at);
+                    keep4(x);
+                    float dx = __builtin_fmaf(x.x, inv_h, sx), dy = __builtin_fmaf(x.y, inv_h, sy),
+                          dz = __builtin_fmaf(x.z, inv_h, sz);
+                    float q = dx * dx + dy * dy + dz * dz;
+                    if (__ballot(!(q < kFar2)) != 0ull && !(q < kFar2)) {
+                        lds_write<v4f>(at, far);
+                        dx = 100.0f;
+                        dy = dz = 0.0f;
+                        q = 1e4f;
+                    }
+                    const v2h xy = __builtin_amdgcn_cvt_pkrtz(dx, dy),
+                              zq = __builtin_amdgcn_cvt_pkrtz(dz, q);
+                    const v4h rows8 = {static_cast<_Float16>(xy.x), static_cast<_Float16>(xy.y),
+                                       static_cast<_Float16>(zq.x), static_cast<_Float16>(zq.y)};
                     uint32_t bits = 0u;
 #pragma unroll
-                    for (uint32_t T2 = 0; T2 < 2; ++T2) {
-                        const uint32_t at = tile + 16u * (64u * w + 32u * T2 + slot_of_row);
-                        const v4f x = lds_read<v4f>(at);
-                        keep4(x);
-                        const float dx = __builtin_fmaf(x.x, inv_h, sx),
-                                    dy = __builtin_fmaf(x.y, inv_h, sy),
-                                    dz = __builtin_fmaf(x.z, inv_h, sz);
-                        const float q = dx * dx + dy * dy + dz * dz;
-                        if (__ballot(!(q < kFar2)) != 0ull && !(q < kFar2)) lds_write<v4f>(at, far);
-                        const v2h xy = __builtin_amdgcn_cvt_pkrtz(dx, dy),
-                                  z1 = __builtin_amdgcn_cvt_pkrtz(dz, 1.0f),
-                                  q1 = __builtin_amdgcn_cvt_pkrtz(q, 1.0f);
-                        const v2h lo = half ? q1 : xy, hi = half ? v2h{0, 0} : z1;
-                        const v16f d = __builtin_amdgcn_mfma_f32_32x32x8f16(
-                            v4h{static_cast<_Float16>(lo.x), static_cast<_Float16>(lo.y),
-                                static_cast<_Float16>(hi.x), static_cast<_Float16>(hi.y)},
-                            col, v16f{}, 0, 0, 0);
+                    for (int k = 0; k < 2; ++k) {
+                        const v16f d =
+                            __builtin_amdgcn_mfma_f32_32x32x8f16(rows8, cols[k], base, 0, 0, 0);
 #pragma unroll
                         for (int r = 0; r < 16; ++r)
                             bits = __builtin_amdgcn_alignbit(bits, __float_as_uint(d[r]), 31);

@@ -189,7 +189,7 @@ __global__ __launch_bounds__(kBlock) void k_xorder(const uint32_t* __restrict__ 
 // Candidates in a wave's tile: a group of a resting fluid (spacing h/2, 1M
 // particles) lists about 400, the dense cells of a collapse 600 and more.  A
 // smaller tile means more waves in flight and more parts per list.  Force at
-// 1M / 30 scenes of 4096..16384: 256 slots 223 / 98 us, 192 slots 226-239 /
+// 1M / 24 scenes of 4096..98304: 256 slots 223 / 98 us, 192 slots 226-239 /
 // 94-99 us, 320 slots (half the waves) 252 / 112 us; density 320 slots 144 / 67,
 // 256 slots 149 / 66, 384 slots 152 / 68 us.
 constexpr uint32_t kDensityCap = 320, kForceCap = 256;
@@ -320,13 +320,14 @@ __device__ __forceinline__ float both_halves(float v) { return v + __shfl_xor(v,
 // with the state as (x, A) and (v, B), which the force pass copies to LDS as
 // they lie.  Bound by VALU issue.
 // Against one lane per target with a block-staged tile per grid row (us, before
-// -> now): 4096 particles 29 -> 18, 30 scenes of 4096..16384 72 -> 67, one
-// million 138 -> 144.
+// -> now): 4096 particles 29 -> 17, 24 scenes of 4096..98304 72 -> 65, one
+// million 138 -> 140.  Five waves per SIMD (95 VGPRs), as many as the tiles
+// allow: with four (110 VGPRs, two filter products in flight) 72 and 149.
 // Batched scenes (kBatched): a group's constants come from scenes[id]; runs
 // never leave a scene because each scene's cells occupy their own range of the
 // global cell array.
 template <bool kKahan, bool kFinalize, bool kBatched>
-__global__ __launch_bounds__(512) void k_density(
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(5))) void k_density(
     const float4* __restrict__ ipos, const float4* __restrict__ ivel,
     const uint32_t* __restrict__ skeys, const uint32_t* __restrict__ cs,
     const uint32_t* __restrict__ ce, StepParams p_in, GridView g_in,
@@ -484,8 +485,8 @@ __device__ __forceinline__ void force_finish(const PairSums<kTension>& S, const 
 // Bound by VALU issue.  A queue of hits per lane, filled by distance tests on a
 // block-staged tile, spent most of its time on lanes waiting for the slowest
 // and on block barriers; two lanes per target with the matrix filter's masks
-// take (us, before -> now): 4096 particles 50 -> 21, 30 scenes of 4096..16384
-// 116 -> 98, one million 320 -> 223.
+// take (us, before -> now): 4096 particles 50 -> 21, 24 scenes of 4096..98304
+// 116 -> 95, one million 320 -> 219.
 template <bool kTension, bool kIntegrate, bool kBatched>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_force(
     const float4* __restrict__ ipos, const float4* __restrict__ ivel,
