@@ -2,11 +2,12 @@
 // with the matrix cores as the range filter.
 //
 // A wave owns a group of 32 targets, two lanes each (lane l and l + 32 share
-// target l & 31 and take its even and its odd candidates).  The
-// group's candidates -- the particles of every grid row that the group's
-// x-window reaches -- are staged once, back to back, in the wave's own LDS
-// tile, so there are no block barriers and no per-row phases.  For each 64
-// staged candidates two V_MFMA_F32_32X32X8_F16 products form
+// target l & 31 and take its even and its odd candidates).  The group's
+// candidates are the particles of every grid row that the group's x-window
+// reaches.  They pass through a ring of four words of 60 in the wave's own LDS
+// tile, so there are no block barriers and no per-row phases, and a lane may be
+// up to three words ahead of another.  For each word two
+// V_MFMA_F32_32X32X16_F16 products form
 //   |x_j - o|^2 - 2 (x_i - o).(x_j - o) + |x_i - o|^2 - h^2 - margin
 // (o: a point among the targets) for all 32 targets in FP16, whose sign bits are
 // the lanes' hit masks: one VALU instruction per 64 pairs instead of the seven
@@ -15,6 +16,14 @@
 // its set bits in order and evaluates each pair from the staged global
 // coordinates with the exact test, so the pairs summed and their values are
 // those of a direct scan.
+//
+// A word holds fours of candidates from all over the group's list, so that each
+// word has its share of every target's neighbours and the lanes stay even, and a
+// four is 64 bytes of memory (single candidates touched 60 cache lines a word:
+// the force pass spent half its time on them).  Takes per lane, modelled at 8 / 24 particles per h^3, where a lane has
+// 16 / 49 neighbours: 24 / 60 with the ring, 30 / 71 with the list in parts of
+// 320 that all lanes finish before the next, and three words or eight instead of
+// four make it 25 / 61 and 24 / 59.
 //
 // The index of a candidate in the group's list decides the lane that takes it
 // and its place in the order, so a target's sums depend on its group alone: not
@@ -30,9 +39,10 @@ namespace sph {
 constexpr uint32_t kGroupTargets = 32;
 typedef float v2f __attribute__((ext_vector_type(2)));
 typedef float v4f __attribute__((ext_vector_type(4)));
+typedef uint32_t v2u __attribute__((ext_vector_type(2)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef __fp16 v2h __attribute__((ext_vector_type(2)));
-typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
 // LDS by byte address.  16-byte elements are read whole (keep4): the 12-byte
 // form that the compiler narrows an unused component to is markedly slower.
@@ -218,36 +228,33 @@ __device__ __forceinline__ float group_margin(float q) { return (7.0f * q + 5.0f
 // Waits for the wave's loads into LDS.
 __device__ __forceinline__ void wait_vmem() { __builtin_amdgcn_s_waitcnt(0x0f70); }
 
-// Lanes below `lanes` each copy 16 bytes from src[step * lane] to LDS at
-// `to` + 16 lane (`to` wave-uniform), without passing through registers.
-__device__ __forceinline__ void lds_copy16(const float4* src, uint32_t step, uint32_t to,
-                                           uint32_t lanes) {
-    const uint32_t lane = threadIdx.x & 63u;
-    if (lane < lanes)
-        __builtin_amdgcn_global_load_lds(
-            reinterpret_cast<const __attribute__((address_space(1))) void*>(
-                reinterpret_cast<uintptr_t>(src + step * lane)),
-            reinterpret_cast<__attribute__((address_space(3))) void*>(to), 16, 0, 0);
+// Waits for the wave's LDS reads.
+__device__ __forceinline__ void wait_lds() { __builtin_amdgcn_s_waitcnt(0xc07f); }
+
+// Active lanes each copy 16 bytes from `src` to LDS at `to` + 16 lane (`to`
+// wave-uniform), without passing through registers.
+__device__ __forceinline__ void lds_copy16(const float4* src, uint32_t to) {
+    __builtin_amdgcn_global_load_lds(
+        reinterpret_cast<const __attribute__((address_space(1))) void*>(
+            reinterpret_cast<uintptr_t>(src)),
+        reinterpret_cast<__attribute__((address_space(3))) void*>(to), 16, 0, 0);
 }
 
-// t / d for a quotient below 2^20 (d > 0; inv_d ~ 1 / d).
-__device__ __forceinline__ uint32_t small_quotient(uint32_t t, uint32_t d, float inv_d) {
-    uint32_t q = static_cast<uint32_t>(static_cast<float>(t) * inv_d);
-    q -= q * d > t ? 1u : 0u;
-    q += t - q * d >= d ? 1u : 0u;
-    return q;
-}
-
-// A wave's tile of kCap candidates (a multiple of 64): their (x, .) as float4,
-// with kVelocity their (v, .) too, and the 64 lanes' mask words of every 64
-// candidates.  The two slots and the mask words past the last ones in use are
-// where a lane that has finished points (it reads one word ahead).
-template <uint32_t kCap, bool kVelocity>
+// A wave's tile: the hit masks of the ring's words (64 lanes each; the first
+// once more past the last, so that the word after any is 256 bytes on), the
+// list's rows, and the words' candidates, kArrays float4 each: (x, .), (v, .) and
+// one more.  A word's slots from 60 on are beyond any target's range for good: a
+// lane that has nothing to take points there.
+constexpr uint32_t kRing = 4, kWordSlots = 60;
+template <uint32_t kArrays>
 struct PairTile {
-    static constexpr uint32_t kSlots = 16u * (kCap + 2u);
-    static constexpr uint32_t kMask = kVelocity ? 2u * kSlots : kSlots;
-    static constexpr uint32_t kBytes = kMask + 4u * (kCap + 128u);
+    static constexpr uint32_t kRows = 256u * (kRing + 1u);
+    static constexpr uint32_t kSlots = 2048u;           // kRows + 8 * 65 rounded up
+    static constexpr uint32_t kArray = 1024u * kRing;   // from one array to the next
+    static constexpr uint32_t kBytes = kSlots + kArrays * kArray;
+    static_assert(kRows + 8u * 65u <= kSlots, "64 rows and the end");
 };
+constexpr uint32_t kTileAlign = 256u * kRing;  // of a tile's LDS address
 
 // Row r of a subgroup's ny x nz rows.
 __device__ __forceinline__ void row_of(const Subgroup& s, uint32_t r, int& y, int& z) {
@@ -270,51 +277,50 @@ __device__ __forceinline__ float4 target_position(const GroupTargets& t) {
     return q < kFar2 ? t.x : make_float4(-kFar, -kFar, -kFar, t.x.w);
 }
 
-// Walks the candidates of a group: their (x, .) in `xs` and, with kVelocity,
-// (v, .) in `vs`, in the internal x-order.  pair(xv...) evaluates this lane's
-// target with one candidate: pair(x) or pair(x, v); every8() is called after at
-// most nine of them, and at the end.
-// tile: LDS address of the wave's PairTile; a longer list is taken kCap
-// candidates at a time.
-template <uint32_t kCap, bool kVelocity, class F, class G>
+// Walks the candidates of a group in the internal x-order: their arrays a0 (x, .),
+// a1 and a2 (kArrays of them).  pair(q0, ..) evaluates this lane's target with one
+// candidate; every8() is called after at most nine of them, and at the end.
+// tile: LDS address of the wave's PairTile.
+template <uint32_t kArrays, class F, class G>
 __device__ __forceinline__ void walk_group(const GridView& g, const GroupTargets& t, float inv_h,
                                            const uint32_t* __restrict__ cs,
                                            const uint32_t* __restrict__ ce,
                                            const uint4* __restrict__ bins, uint32_t n,
-                                           const float4* __restrict__ xs,
-                                           const float4* __restrict__ vs, uint32_t tile, F&& pair,
+                                           const float4* __restrict__ a0,
+                                           const float4* __restrict__ a1,
+                                           const float4* __restrict__ a2, uint32_t tile, F&& pair,
                                            G&& every8) {
-    typedef PairTile<kCap, kVelocity> T;
+    typedef PairTile<kArrays> T;
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t half = lane >> 5;
     // A lane half converts 32 of 64 candidates; the first product takes the lower
     // half's (the upper half's target operand is 0), the second the upper's.
     // Row m of a product reads slot 2 r + q of its 32, where (q, r) are the lane
-    // half and accumulator that receive row m: a lane's 32 mask bits
-    // are the even (half 0) or odd slots of 64, so a target's hits, which lie
-    // together along a row, fall evenly on its two lanes.
+    // half and accumulator that receive row m: a lane's 32 mask bits are the even
+    // (half 0) or odd slots of 64, so a target's hits, which lie together along a
+    // row, fall evenly on its two lanes.  The rows of slots 60 to 63 read others;
+    // their bits are dropped.
     const uint32_t m = lane & 31u;
-    const uint32_t slot_of_row = 2u * (4u * (m >> 3) + (m & 3u)) + ((m >> 2) & 1u);
+    const uint32_t slot_of_row = 2u * (4u * (m >> 3) + (m & 3u)) + ((m >> 2) & 1u) + 32u * half;
+    const uint32_t row_slot =
+        tile + T::kSlots + 16u * (slot_of_row < kWordSlots ? slot_of_row : slot_of_row - 4u);
+    const uint32_t mask0 = tile + 4u * lane;
+    // The slots nobody is near.
+    if (lane < 4u * kRing) {
+        const uint32_t at = tile + T::kSlots + 1024u * (lane >> 2) + 16u * (kWordSlots + (lane & 3u));
+        lds_write<v4f>(at, v4f{kFar, kFar, kFar, 0.0f});
+#pragma unroll
+        for (uint32_t k = 1; k < kArrays; ++k)
+            lds_write<v4f>(at + k * T::kArray, v4f{0.0f, 0.0f, 0.0f, 0.0f});
+    }
+    uint32_t turn = 0u;
     uint32_t rem = static_cast<uint32_t>(__ballot(t.active));
     while (rem) {
         const Subgroup s = next_subgroup(g, t, rem);
-        // Fills a tile to whole words: out of the members' range, yet finite in
-        // FP16 (an infinity would make the products NaN, and its sign a hit).
+        // Fills the words: out of the members' range, yet finite in FP16 (an
+        // infinity would make the products NaN, and its sign a hit).
         const v4f far = {s.ox + 100.0f * __builtin_amdgcn_rcpf(inv_h), s.oy, s.oz, 0.0f};
-        // Target operands of the filter, in units of h: columns (-2 x, -2 y, -2 z, 1)
-        // against rows (x, y, z, |x|^2), added to the column's |x|^2 - 1 - margin.
-        const float sx = -s.ox * inv_h, sy = -s.oy * inv_h, sz = -s.oz * inv_h;
-        const float ix = __builtin_fmaf(t.x.x, inv_h, sx), iy = __builtin_fmaf(t.x.y, inv_h, sy),
-                    iz = __builtin_fmaf(t.x.z, inv_h, sz);
-        const float qi = ix * ix + iy * iy + iz * iz;
-        const float ci = s.member && qi < 1e4f ? qi - 1.0f - group_margin(qi) : 1e30f;
-        const v4h none = {0, 0, 0, 0},
-                  col = {static_cast<_Float16>(-2.0f * ix), static_cast<_Float16>(-2.0f * iy),
-                         static_cast<_Float16>(-2.0f * iz), 1},
-                  cols[2] = {half ? none : col, half ? col : none};
-        v16f base;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) base[r] = ci;
+        const uint64_t members = __ballot(s.member);
         const uint32_t rows = static_cast<uint32_t>(s.ny) * static_cast<uint32_t>(s.nz);
         for (uint32_t row0 = 0; row0 < rows; row0 += 64u) {
             uint32_t rb = 0u, re = 0u;
@@ -323,125 +329,177 @@ __device__ __forceinline__ void walk_group(const GridView& g, const GroupTargets
                 row_of(s, row0 + lane, y, z);
                 subgroup_row(g, s, cs, ce, bins, n, y, z, rb, re);
             }
+            // The list: the rows that are not empty, as (its end in the list,
+            // first particle less its start), and an end that is never reached.
             const uint32_t len = re - rb;
             const uint32_t end = wave_scan_add(len);
             const uint32_t total = lane_u32(end, 63);
-            const int live_rows = static_cast<int>(min(64u, rows - row0));
-            // A list longer than the tile is taken in `parts`, part p holding
-            // every parts-th candidate from p on: each part then has its share
-            // of every target's neighbours, and the lanes stay even.  (Modelled
-            // takes per lane at 24 particles per h^3, 50 of them neighbours, with
-            // 256 candidates at a time: 106 one stretch after the other, 77 so.)
-            const uint32_t parts = (total + kCap - 1u) / kCap;
-            const float inv_parts = __builtin_amdgcn_rcpf(static_cast<float>(parts));
-            for (uint32_t part = 0; part < parts; ++part) {
-                const uint32_t cnt = (total - part + parts - 1u) / parts;
-                // Slots [first, past) of this lane's row.
-                const uint32_t past = small_quotient(end - part + parts - 1u, parts, inv_parts);
-                const uint32_t first = small_quotient(end - len - part + parts - 1u, parts, inv_parts);
-                for (int r = 0; r < live_rows; ++r) {
-                    const uint32_t s0 = lane_u32(first, r), s1 = lane_u32(past, r);
-                    // Particle of slot k: its row's first one plus its place.
-                    const uint32_t from = lane_u32(rb + len - end, r) + part;
-                    for (uint32_t k = s0; k < s1; k += 64u) {
-                        lds_copy16(xs + (from + parts * k), parts, tile + 16u * k, s1 - k);
-                        if (kVelocity)
-                            lds_copy16(vs + (from + parts * k), parts, tile + T::kSlots + 16u * k,
-                                       s1 - k);
-                    }
+            if (total == 0u) continue;
+            uint64_t live = __ballot(len != 0u);
+            const uint32_t place = __builtin_amdgcn_mbcnt_hi(
+                static_cast<uint32_t>(live >> 32),
+                __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(live), 0u));
+            if (len != 0u) lds_write<v2u>(tile + T::kRows + 8u * place, v2u{end, rb + len - end});
+            if (lane == 0u)
+                lds_write<v2u>(tile + T::kRows + 8u * static_cast<uint32_t>(__builtin_popcountll(live)),
+                               v2u{0xFFFFFFFFu, 0u});
+            // Target operands of the filter, in units of h: columns
+            // (-2 x, -2 y, -2 z, 1, c, c') against rows (x, y, z, |x|^2, 1, 1), with
+            // c + c' = |x|^2 - 1 - margin.
+            const float sx = -s.ox * inv_h, sy = -s.oy * inv_h, sz = -s.oz * inv_h;
+            const float ix = __builtin_fmaf(t.x.x, inv_h, sx), iy = __builtin_fmaf(t.x.y, inv_h, sy),
+                        iz = __builtin_fmaf(t.x.z, inv_h, sz);
+            const float qi = ix * ix + iy * iy + iz * iz;
+            float ci = s.member && qi < 1e4f ? qi - 1.0f - group_margin(qi) : 6e4f;
+            asm volatile("" : "+v"(ci));  // here, not before the rows: registers
+            const _Float16 c_hi = static_cast<_Float16>(ci);
+            const v8h none = {0, 0, 0, 0, 0, 0, 0, 0},
+                      col = {static_cast<_Float16>(-2.0f * ix), static_cast<_Float16>(-2.0f * iy),
+                             static_cast<_Float16>(-2.0f * iz), 1, c_hi,
+                             static_cast<_Float16>(ci - static_cast<float>(c_hi)), 0, 0},
+                      cols[2] = {half ? none : col, half ? col : none};
+            // Word w holds, of every 4 words candidates, four from 4 w on.  This
+            // lane copies its slot's ones, one word after the other: `at` in the
+            // list, in a row that ends at entry.x, whose table entry is at row.
+            const uint32_t words = (total + kWordSlots - 1u) / kWordSlots;
+            uint32_t at = 4u * words * (lane >> 2) + (lane & 3u), row = tile + T::kRows;
+            for (; live; live &= live - 1u)
+                row += at >= lane_u32(end, static_cast<int>(__builtin_ctzll(live))) ? 8u : 0u;
+            wave_sync();
+            v2u entry = lds_read<v2u>(row);
+            auto stage = [&](uint32_t w) {
+                const uint32_t to = tile + T::kSlots + 1024u * (w % kRing);
+                while (__ballot(at >= entry.x) != 0ull) {  // rows of less than four
+                    row += at >= entry.x ? 8u : 0u;
+                    entry = lds_read<v2u>(row);
                 }
-                const uint32_t words = (cnt + 63u) >> 6;
-                // Far candidates up to the end of the last 64, and two beyond
-                // for the finished lanes: those are any target's, so out of
-                // everyone's range wherever it is.
-                for (uint32_t k = cnt + lane; k < 64u * words + 2u; k += 64u) {
-                    lds_write<v4f>(tile + 16u * k,
-                                   k < 64u * words ? far : v4f{kFar, kFar, kFar, 0.0f});
-                    if (kVelocity)
-                        lds_write<v4f>(tile + T::kSlots + 16u * k, v4f{0.0f, 0.0f, 0.0f, 0.0f});
-                }
-                const uint32_t mask0 = tile + T::kMask + 4u * lane;
-                const uint32_t end_mask = mask0 + 256u * words;
-                lds_write<uint32_t>(end_mask, 0x80000000u);
-                lds_write<uint32_t>(end_mask + 256u, 0x80000000u);
-                wait_vmem();
-                wave_sync();
-                for (uint32_t w = 0; w < words; ++w) {
-                    const uint32_t at = tile + 16u * (64u * w + 32u * half + slot_of_row);
-                    const v4f x = lds_read<v4f>(at);
-                    keep4(x);
-                    float dx = __builtin_fmaf(x.x, inv_h, sx), dy = __builtin_fmaf(x.y, inv_h, sy),
-                          dz = __builtin_fmaf(x.z, inv_h, sz);
-                    float q = dx * dx + dy * dy + dz * dz;
-                    if (__ballot(!(q < kFar2)) != 0ull && !(q < kFar2)) {
-                        lds_write<v4f>(at, far);
-                        dx = 100.0f;
-                        dy = dz = 0.0f;
-                        q = 1e4f;
-                    }
-                    const v2h xy = __builtin_amdgcn_cvt_pkrtz(dx, dy),
-                              zq = __builtin_amdgcn_cvt_pkrtz(dz, q);
-                    const v4h rows8 = {static_cast<_Float16>(xy.x), static_cast<_Float16>(xy.y),
-                                       static_cast<_Float16>(zq.x), static_cast<_Float16>(zq.y)};
-                    uint32_t bits = 0u;
+                if (lane < kWordSlots) {
+                    if (at < total) {
+                        const uint32_t j = at + entry.y;
+                        lds_copy16(a0 + j, to);
+                        if (kArrays > 1) lds_copy16(a1 + j, to + T::kArray);
+                        if (kArrays > 2) lds_copy16(a2 + j, to + 2u * T::kArray);
+                    } else {
+                        lds_write<v4f>(to + 16u * lane, far);
 #pragma unroll
-                    for (int k = 0; k < 2; ++k) {
-                        const v16f d =
-                            __builtin_amdgcn_mfma_f32_32x32x8f16(rows8, cols[k], base, 0, 0, 0);
-#pragma unroll
-                        for (int r = 0; r < 16; ++r)
-                            bits = __builtin_amdgcn_alignbit(bits, __float_as_uint(d[r]), 31);
+                        for (uint32_t k = 1; k < kArrays; ++k)
+                            lds_write<v4f>(to + k * T::kArray + 16u * lane,
+                                           v4f{0.0f, 0.0f, 0.0f, 0.0f});
                     }
-                    // No word is empty: the last slot stands in for none, and
-                    // the exact test of pair() turns it down.
-                    lds_write<uint32_t>(mask0 + 256u * w, max(bits, 1u));
                 }
+                at += 4u;
+                row += at >= entry.x ? 8u : 0u;
+                entry = lds_read<v2u>(row);
+            };
+            auto set_mask = [&](uint32_t w, uint32_t bits) {
+                lds_write<uint32_t>(mask0 + 256u * (w % kRing), bits);
+                if (w % kRing == 0u) lds_write<uint32_t>(mask0 + 256u * kRing, bits);
+            };
+            // Each member's lane takes the set bits of its words in order.  The
+            // word after the last one filtered has the mask 1, a bit that stays
+            // set: a lane there, or one that is no member, takes a slot that
+            // nobody is near.  word: where the lane's current word is, whose
+            // first slot is at 4 word + to_slots; one candidate is on its way
+            // while another is evaluated.
+            const uint32_t to_slots = tile + T::kSlots + 16u * half - 4u * mask0;
+            uint32_t word = mask0, cur = 1u, nxt = 1u, wrap = 256u * kRing - 1u;
+            asm("" : "+v"(wrap));  // one and-or, which takes one scalar operand
+            auto next_word = [&](uint32_t w) { return ((w + 256u) & wrap) | tile; };
+            auto filter = [&](uint32_t w) {
+                const uint32_t from = row_slot + 1024u * (w % kRing);
+                const v4f x = lds_read<v4f>(from);
+                keep4(x);
+                float dx = __builtin_fmaf(x.x, inv_h, sx), dy = __builtin_fmaf(x.y, inv_h, sy),
+                      dz = __builtin_fmaf(x.z, inv_h, sz);
+                float q = dx * dx + dy * dy + dz * dz;
+                if (__ballot(!(q < kFar2)) != 0ull && !(q < kFar2)) {
+                    lds_write<v4f>(from, far);
+                    dx = 100.0f;
+                    dy = dz = 0.0f;
+                    q = 1e4f;
+                }
+                const v2h xy = __builtin_amdgcn_cvt_pkrtz(dx, dy),
+                          zq = __builtin_amdgcn_cvt_pkrtz(dz, q);
+                const v8h rows8 = {static_cast<_Float16>(xy.x), static_cast<_Float16>(xy.y),
+                                   static_cast<_Float16>(zq.x), static_cast<_Float16>(zq.y),
+                                   1, 1, 0, 0};
+                uint32_t bits = 0u;
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    const v16f d =
+                        __builtin_amdgcn_mfma_f32_32x32x16_f16(rows8, cols[k], v16f{}, 0, 0, 0);
+#pragma unroll
+                    for (int r = 0; r < 16 - 2 * k; ++r)
+                        bits = __builtin_amdgcn_alignbit(bits, __float_as_uint(d[r]), 31);
+                    __builtin_amdgcn_sched_barrier(0);  // one product's registers at a time
+                }
+                // No word is empty: slot 60 or 61 stands in for none.
+                bits = max(bits << 2, 2u);
+                set_mask(w, bits);
+                set_mask(w + 1u, 1u);
                 wave_sync();
-                // Each member's lane takes the set bits of its words in order;
-                // a lane that has finished (or is no member) keeps taking the
-                // far candidate past the end.  word: where the lane's current
-                // word is, whose first slot is at 4 word + to_slots.  One
-                // candidate is on its way while another is evaluated.
-                const uint32_t to_slots = tile + 16u * half - 4u * mask0;
-                uint32_t word = s.member ? mask0 : end_mask;
-                uint32_t cur = lds_read<uint32_t>(word), nxt = lds_read<uint32_t>(word + 256u);
-                auto take = [&](v4f& x, v4f& v) {
-                    const uint32_t z = __builtin_clz(cur);
-                    uint32_t first = 4u * word + to_slots;
-                    asm("" : "+v"(first));  // two shift-and-adds, not three instructions
-                    const uint32_t p = 32u * z + first;
-                    x = lds_read<v4f>(p);
-                    if (kVelocity) v = lds_read<v4f>(p + T::kSlots);
-                    cur &= ~(0x80000000u >> z);
-                    const bool over = cur == 0u;
-                    cur = over ? nxt : cur;
-                    word = over ? min(word + 256u, end_mask) : word;
-                    nxt = lds_read<uint32_t>(word + 256u);
-                };
-                auto eval = [&](const v4f& x, const v4f& v) {
-                    keep4(x);
-                    if constexpr (kVelocity)
-                        pair(x, v);
-                    else
-                        pair(x);
-                };
-                v4f xa, va, xb, vb;
-                take(xa, va);
-                uint32_t turn = 0u;
-                do {
-                    take(xb, vb);
-                    eval(xa, va);
-                    take(xa, va);
-                    eval(xb, vb);
-                    if ((++turn & 3u) == 0u) {
-                        asm volatile("");  // a branch, not selects on every turn
-                        every8();
+                // Lanes that waited for this word or read ahead to it.
+                cur = s.member && word == mask0 + 256u * (w % kRing) ? bits : cur;
+                nxt = lds_read<uint32_t>(word + 256u);
+            };
+            auto take = [&](v4f* q) {
+                const uint32_t z = __builtin_clz(cur);
+                uint32_t first = 4u * word + to_slots;
+                asm("" : "+v"(first));  // two shift-and-adds, not three instructions
+                const uint32_t p = 32u * z + first;
+#pragma unroll
+                for (uint32_t k = 0; k < kArrays; ++k) q[k] = lds_read<v4f>(p + k * T::kArray);
+                cur &= ~(0x80000000u >> z) | 1u;
+                const bool over = cur == 0u;
+                cur = over ? nxt : cur;
+                word = over ? next_word(word) : word;
+                nxt = lds_read<uint32_t>(word + 256u);
+            };
+            auto eval = [&](const v4f* q) {
+#pragma unroll
+                for (uint32_t k = 0; k < kArrays; ++k) keep4(q[k]);
+                if constexpr (kArrays == 1)
+                    pair(q[0]);
+                else if constexpr (kArrays == 2)
+                    pair(q[0], q[1]);
+                else
+                    pair(q[0], q[1], q[2]);
+            };
+            uint32_t staged = 0u, filtered = 0u, oldest = 0u, oldest_word = mask0;
+            do stage(staged);
+            while (++staged < min(words, kRing));
+            wait_vmem();
+            wave_sync();
+            do filter(filtered);
+            while (++filtered < min(words, kRing - 1u));
+            v4f qa[kArrays], qb[kArrays];
+            take(qa);
+            for (;;) {
+                take(qb);
+                eval(qa);
+                take(qa);
+                eval(qb);
+                if ((++turn & 3u) == 0u) {
+                    asm volatile("");  // a branch, not selects on every turn
+                    every8();
+                }
+                // Someone is still in the oldest word.
+                if ((__ballot(word == oldest_word) & members) != 0ull) continue;
+                if (++oldest == words) break;
+                oldest_word = next_word(oldest_word);
+                if (filtered < words) {
+                    wait_vmem();
+                    filter(filtered++);
+                    if (staged < words) {
+                        wait_lds();  // of the word that goes
+                        stage(staged++);
                     }
-                } while (__ballot(word != end_mask) != 0ull);
-                eval(xa, va);
-                every8();
-                wave_sync();
+                }
             }
+            eval(qa);
+            every8();
+            wait_lds();
+            wave_sync();
         }
     }
 }

@@ -186,15 +186,8 @@ __global__ __launch_bounds__(kBlock) void k_xorder(const uint32_t* __restrict__ 
 //   bits 20-21 density, bits 22-23 force: groups taken by a wave one after the
 //              other, 1 (0) or 2 (1), with the default block (single scenes)
 //
-// Candidates in a wave's tile: a group of a resting fluid (spacing h/2, 1M
-// particles) lists about 400, the dense cells of a collapse 600 and more.  A
-// smaller tile means more waves in flight and more parts per list.  Force at
-// 1M / 24 scenes of 4096..98304: 256 slots 223 / 98 us, 192 slots 226-239 /
-// 94-99 us, 320 slots (half the waves) 252 / 112 us; density 320 slots 144 / 67,
-// 256 slots 149 / 66, 384 slots 152 / 68 us.
-constexpr uint32_t kDensityCap = 320, kForceCap = 256;
-typedef PairTile<kDensityCap, false> DensityTile;
-typedef PairTile<kForceCap, true> ForceTile;
+typedef PairTile<1> DensityTile;
+typedef PairTile<2> ForceTile;
 // Waves share nothing but the launch: 2 and 4 waves are within 3% of each other
 // on every size, the rest is left to the tuner.
 constexpr uint32_t kTileWaves[] = {4, 1, 2, 3, 5, 6, 4, 4, 4, 4};
@@ -320,9 +313,11 @@ __device__ __forceinline__ float both_halves(float v) { return v + __shfl_xor(v,
 // with the state as (x, A) and (v, B), which the force pass copies to LDS as
 // they lie.  Bound by VALU issue.
 // Against one lane per target with a block-staged tile per grid row (us, before
-// -> now): 4096 particles 29 -> 17, 24 scenes of 4096..98304 72 -> 65, one
-// million 138 -> 140.  Five waves per SIMD (95 VGPRs), as many as the tiles
-// allow: with four (110 VGPRs, two filter products in flight) 72 and 149.
+// -> now): 4096 particles 29 -> 18, 24 scenes of 4096..98304 72 -> 63, one
+// million 138 -> 134, one million at rest 95 -> 80.  At one million 23 of them go
+// to finding the rows, 22 to the filter products and their masks, and most of the
+// rest is takes and staging.  Five waves per SIMD (96 VGPRs): with four 63 and
+// 143, with six (spills) 67 and 144 us.
 // Batched scenes (kBatched): a group's constants come from scenes[id]; runs
 // never leave a scene because each scene's cells occupy their own range of the
 // global cell array.
@@ -334,7 +329,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(5))) void k
     const uint32_t* __restrict__ n_dev, float* __restrict__ rho, float2* __restrict__ aux,
     float4* __restrict__ ixa, float4* __restrict__ ivb, const SceneParams* __restrict__ scenes,
     const uint4* __restrict__ groups, uint32_t n_groups, XOrder xo, LaunchShape sh) {
-    extern __shared__ __align__(16) unsigned char lds[];
+    extern __shared__ __align__(kTileAlign) unsigned char lds[];
     const uint32_t wave = uniform_u32(threadIdx.x >> 6), waves = blockDim.x >> 6;
     const uint32_t tile = lds_address(lds) + wave * DensityTile::kBytes;
     const uint32_t n = *n_dev;
@@ -349,13 +344,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(5))) void k
             const GroupTargets t = load_targets(g, gr, ipos, skeys, s);
             const float4 xi = target_position(t);
             const float inv_h2 = p.inv_h2;
-            // What the end needs, loaded before the walk.
-            const uint32_t o = xo.i2r[t.active ? s : gr.start];
-            const float4 v = kFinalize ? ivel[t.active ? s : gr.start] : t.x;
             double sum64 = 0.0;
             float sum32 = 0.0f;
-            walk_group<kDensityCap, false>(
-                g, t, p.inv_h, cs, ce, xo.bins, n, ipos, nullptr, tile, [&](const v4f& x) {
+            walk_group<1>(
+                g, t, p.inv_h, cs, ce, xo.bins, n, ipos, nullptr, nullptr, tile, [&](const v4f& x) {
 #pragma clang fp contract(off)
                     const float a = poly6_unit(xi, x, inv_h2);
                     sum32 = __builtin_fmaf(a * a, a, sum32);
@@ -369,8 +361,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(5))) void k
             const float r = p.c6m_h6 * (kKahan ? static_cast<float>(both_halves(sum64))
                                                : both_halves(sum32));
             if (t.active && (threadIdx.x & 32u) == 0u) {
+                const uint32_t o = xo.i2r[s];
                 rho[o] = r;
                 if (kFinalize) {
+                    const float4 v = ivel[s];
                     const float inv = __builtin_amdgcn_rcpf(r);
                     const float A = p.stiffness * (r - p.rest_density) * inv * inv;
                     ixa[s] = make_float4(t.x.x, t.x.y, t.x.z, A);
@@ -485,8 +479,8 @@ __device__ __forceinline__ void force_finish(const PairSums<kTension>& S, const 
 // Bound by VALU issue.  A queue of hits per lane, filled by distance tests on a
 // block-staged tile, spent most of its time on lanes waiting for the slowest
 // and on block barriers; two lanes per target with the matrix filter's masks
-// take (us, before -> now): 4096 particles 50 -> 21, 24 scenes of 4096..98304
-// 116 -> 95, one million 320 -> 219.
+// take (us, before -> now): 4096 particles 50 -> 20, 24 scenes of 4096..98304
+// 116 -> 90, one million 320 -> 200, one million at rest 150 -> 110.
 template <bool kTension, bool kIntegrate, bool kBatched>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_force(
     const float4* __restrict__ ipos, const float4* __restrict__ ivel,
@@ -496,7 +490,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
     const uint32_t* __restrict__ n_dev, float dt, float4* __restrict__ pos,
     float4* __restrict__ vel, float4* __restrict__ accel, const SceneParams* __restrict__ scenes,
     const uint4* __restrict__ groups, uint32_t n_groups, XOrder xo, LaunchShape sh) {
-    extern __shared__ __align__(16) unsigned char lds[];
+    extern __shared__ __align__(kTileAlign) unsigned char lds[];
     const uint32_t wave = uniform_u32(threadIdx.x >> 6), waves = blockDim.x >> 6;
     const uint32_t tile = lds_address(lds) + wave * ForceTile::kBytes;
     const uint32_t n = *n_dev;
@@ -510,15 +504,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
             uint32_t s;
             const GroupTargets t = load_targets(g, gr, ixa, skeys, s);
             const float4 xi = target_position(t);
-            // What the end needs, loaded before the walk; the id and tag words
-            // come with the unpacked state.
-            const uint32_t at = t.active ? s : gr.start;
-            const float4 vi = ivb[at];
-            const uint32_t o = xo.i2r[at];
-            const float id = kIntegrate ? ipos[at].w : 0.0f, tag = kIntegrate ? ivel[at].w : 0.0f;
+            const float4 vi = ivb[t.active ? s : gr.start];
             PairSums<kTension> S;
-            walk_group<kForceCap, true>(
-                g, t, p.inv_h, cs, ce, xo.bins, n, ixa, ivb, tile,
+            walk_group<2>(
+                g, t, p.inv_h, cs, ce, xo.bins, n, ixa, ivb, nullptr, tile,
                 [&](const v4f& x, const v4f& v) { S.add(xi, vi, t.x.w, p.h, p.h2, x, v); }, [] {});
             S.Px = both_halves(S.Px);
             S.Py = both_halves(S.Py);
@@ -533,10 +522,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
             }
             if (t.active && (threadIdx.x & 32u) == 0u) {
                 float4 x = t.x, v = vi;
-                x.w = id;
-                v.w = tag;
-                force_finish<kTension, kIntegrate>(S, p, x, v, make_float2(t.x.w, vi.w), o, xo.bacc,
-                                                   dt, pos, vel, accel, xo.err);
+                if (kIntegrate) {  // the id and tag words come with the unpacked state
+                    x.w = ipos[s].w;
+                    v.w = ivel[s].w;
+                }
+                force_finish<kTension, kIntegrate>(S, p, x, v, make_float2(t.x.w, vi.w), xo.i2r[s],
+                                                   xo.bacc, dt, pos, vel, accel, xo.err);
             }
         }
     }

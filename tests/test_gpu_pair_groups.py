@@ -1,8 +1,7 @@
 """The neighbour walk of groups of 32 particles, where it can go wrong.
 
 Group remainders (1 to 65 particles), a batch whose scenes end inside a group,
-candidate lists around the wave's tile (256 and 320 candidates) and around its
-64-candidate words, grid cells smaller and larger than h, a group that spans
+candidate lists from a few to several rings of four 60-candidate words, grid cells smaller and larger than h, a group that spans
 rows or lies at both
 ends of long ones, and particles outside the grid.  Each against the FP64 oracle with the
 suite's bars: density 1e-5 relative, acceleration 1e-5 of max |a*|, for these
@@ -56,8 +55,14 @@ def test_group_remainders(n):
     _check("remainder", _config(), *_state(n, n, 1.2 * H, 3.1 * H))
 
 
+@pytest.mark.parametrize("n", [3, 4, 5, 59, 60, 61, 119, 120, 121, 180, 181, 239, 241, 300])
+def test_lists_around_the_words(n):
+    # One cell again: a word holds 60 candidates, the ring four of them.
+    _check("words", _config(), *_state(n, 1000 + n, 2.01 * H, 2.99 * H))
+
+
 @pytest.mark.parametrize("n", [255, 256, 257, 319, 320, 321, 383, 511, 513, 640, 641, 769])
-def test_lists_around_the_tile(n):
+def test_lists_longer_than_the_ring(n):
     # All in one cell: every group's list holds all n.
     _check("one cell", _config(), *_state(n, n, 2.01 * H, 2.99 * H))
 
