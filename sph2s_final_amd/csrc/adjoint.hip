@@ -34,19 +34,20 @@
 //
 // Memory: the state is checkpointed every K steps; the backward sweep
 // recomputes each K-step segment from its checkpoint, keeping every step's
-// x-ordered state, accelerations, densities, A/B factors, permutations, cell
-// ranges and x-bin tables (68 B per particle + 24 B per cell per step), then
-// runs the adjoint passes over the segment in reverse.  The forward writes the last segment's records
-// itself, so that segment is never recomputed.  Parameter gradients accumulate per slot in
-// FP64 (a slot always belongs to the same scene) and are reduced per scene in
-// a fixed order, so the result is deterministic.
+// x-ordered state packed with the A/B factors, accelerations, densities,
+// permutations, cell ranges and x-bin tables (60 B per particle + 40 B per cell
+// per step), then runs the adjoint passes over the segment in reverse.  The
+// forward writes the last segment's records itself, so that segment is never
+// recomputed.  Parameter gradients accumulate in FP64 per group of 32 slots
+// (a group always belongs to the same scene) and are reduced per scene in a
+// fixed order, so the result is deterministic.
 #include <algorithm>
 #include <cmath>
 #include <new>
 #include <vector>
 
 #include "batch.hpp"
-#include "pairwalk.hpp"
+#include "pairtile.hpp"
 
 using namespace sph;
 
@@ -110,27 +111,27 @@ __global__ void k_unpack3(const float4* __restrict__ src, uint32_t n, float* __r
     dst[3 * i + 2] = v.z;
 }
 
-__device__ __forceinline__ const SceneParams& scene_for(const SceneParams* __restrict__ scenes,
-                                                        const float4& v) {
-    return scenes[__float_as_uint(v.w)];
-}
-
 // Clamp and symplectic Euler.  The pre-clamp position is recomputed with the
 // forward kernel's expressions from the stored sorted state and acceleration.
+// Half a wave per group of the batch's table, which holds the scene.
 __global__ __launch_bounds__(kBlock) void k_adj_integrate(
-    const float4* __restrict__ ipos, const float4* __restrict__ ivel,
+    const float4* __restrict__ ixa, const float4* __restrict__ ivb,
     const float4* __restrict__ accel, const uint32_t* __restrict__ i2r,
     const float4* __restrict__ gx, const float4* __restrict__ gv,
-    const SceneParams* __restrict__ scenes, const uint32_t* __restrict__ n_dev, float dt,
-    float4* __restrict__ abar, float4* __restrict__ gxd, float4* __restrict__ gvd) {
+    const SceneParams* __restrict__ scenes, const uint4* __restrict__ groups, uint32_t n_groups,
+    const uint32_t* __restrict__ n_dev, float dt, float4* __restrict__ abar,
+    float4* __restrict__ gxd, float4* __restrict__ gvd) {
     const uint32_t n = *n_dev;
-    const uint32_t s = xcd_local_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
-    if (s >= n) return;
+    const uint32_t group = (xcd_local_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x) / kGroupTargets;
+    if (group >= n_groups) return;
+    const uint4 gr = groups[group];
+    const uint32_t s = gr.x + threadIdx.x % kGroupTargets;
+    if (s >= min(gr.y, n)) return;
     // s: internal slot; the step's outputs (and their adjoints) sit at its
     // sorted slot i2r[s].
     const uint32_t o = min(i2r[s], n - 1);
-    const float4 xi = ipos[s], vi = ivel[s], ai = accel[o], gxi = gx[o], gvi = gv[o];
-    const StepParams& p = scene_for(scenes, vi).p;
+    const float4 xi = ixa[s], vi = ivb[s], ai = accel[o], gxi = gx[o], gvi = gv[o];
+    const StepParams& p = scenes[gr.z].p;
     const bool clamp = (p.flags & SPH_FLAG_WALL_CLAMP) != 0u;
     const float e = p.restitution;
     auto axis = [&](float x, float v, float a, float gxo, float gvo, float lo, float hi, float& ga,
@@ -157,149 +158,128 @@ __global__ __launch_bounds__(kBlock) void k_adj_integrate(
     gvd[s] = V;
 }
 
-#ifndef SPH_ADJ_FORCE_TILE
-#define SPH_ADJ_FORCE_TILE 512
-#endif
-#ifndef SPH_ADJ_DENSITY_TILE
-#define SPH_ADJ_DENSITY_TILE 1024
-#endif
-constexpr int kAdjForceTile = SPH_ADJ_FORCE_TILE;
-constexpr int kAdjDensityTile = SPH_ADJ_DENSITY_TILE;
-constexpr int kWaves = kBlock / 64;
-constexpr int kAdjGroup = 8;   // candidates loaded together before any test
-constexpr int kAdjQueue = 16;  // per-lane queue of in-range candidates (force adjoint)
+typedef PairTile<3> AdjForceTile;
+typedef PairTile<1> AdjDensityTile;
+// One wave per block: the force adjoint's tile, 14 KB, then has 11 waves on a
+// CU, where blocks of four leave room for 8 (197 against 235 us at one million).
+constexpr uint32_t kAdjForceWaves = 1, kAdjDensityWaves = 4;
+constexpr uint32_t kAdjChunkGroups = 128;  // groups in a row that one XCD takes
 
-// 0 < r2 < h2 as one unsigned compare (r2 >= +0; non-negative floats order
-// like their bit patterns).
-__device__ __forceinline__ bool pair_in_range(float r2, uint32_t h2_bits_m1) {
-    return __float_as_uint(r2) - 1u < h2_bits_m1;
+// The wave's group and its targets; the cells come from the positions, as the
+// step's sort took them.
+template <uint32_t kWavesPerBlock>
+__device__ __forceinline__ GroupRange adjoint_group(uint32_t n, const uint4* __restrict__ groups,
+                                                    uint32_t n_groups) {
+    const uint32_t block = xcd_local_block(blockIdx.x, gridDim.x, kAdjChunkGroups / kWavesPerBlock);
+    return group_range<true>(block * kWavesPerBlock + uniform_u32(threadIdx.x >> 6), n, groups,
+                             n_groups);
 }
 
-// Force-pair adjoint; see the file comment for the terms.  Candidates are
-// staged in LDS as (x, A), (v, B) and abar.  A lane first queues the tile
-// indices of its in-range candidates (whole groups of candidates are loaded
-// before any test) and evaluates the queued pair terms, in queue order, when
-// some lane's queue is nearly full and at the end of each staged run.
-__global__ __launch_bounds__(kBlock) void k_adj_force(
-    const float4* __restrict__ tpos, const float4* __restrict__ tvel,
+__device__ __forceinline__ GroupTargets adjoint_targets(const GridView& g, const GroupRange& r,
+                                                        const float4* __restrict__ xs, uint32_t& s) {
+    GroupTargets t;
+    s = r.start + (threadIdx.x & 31u);
+    t.active = s < r.end;
+    t.x = xs[t.active ? s : r.start];
+    t.key = cell_hash(t.x.x, t.x.y, t.x.z, g.ox, g.oy, g.oz, g.spacing, g.dx, g.dy, g.dz);
+    return t;
+}
+
+// Force-pair adjoint; see the file comment for the terms.  The group walk
+// (pairtile.hpp) with (x, A), (v, B) and abar per candidate; a pair out of range
+// or coincident adds 0.  Writes (x, dL/drho) packed for the density adjoint, and
+// adds each group's parameter terms, in FP64, to the group's own accumulators.
+// Bound by VALU issue.  Against a queue of hits per lane on a block-staged tile
+// (us, one million in 16 scenes): 233 -> 197.
+__global__ __launch_bounds__(64 * kAdjForceWaves) __attribute__((amdgpu_waves_per_eu(3)))
+void k_adj_force(
     const float4* __restrict__ ixa, const float4* __restrict__ ivb, const float* __restrict__ rho,
     const uint32_t* __restrict__ i2r, const float4* __restrict__ abar,
     const uint32_t* __restrict__ cs, const uint32_t* __restrict__ ce,
     const uint4* __restrict__ bins, const SceneParams* __restrict__ scenes,
-    const uint32_t* __restrict__ n_dev, float* __restrict__ grho, float4* __restrict__ gxd,
-    float4* __restrict__ gvd, double* __restrict__ kacc, double* __restrict__ macc) {
-    __shared__ float4 tx[kAdjForceTile + kAdjGroup];  // padded for whole-group loads
-    __shared__ float4 tv[kAdjForceTile];
-    __shared__ float4 ta[kAdjForceTile];
-    __shared__ uint16_t queue[kAdjQueue][kBlock];
-    __shared__ uint32_t red[2 * kWaves];
+    const uint4* __restrict__ groups, uint32_t n_groups, const uint32_t* __restrict__ n_dev,
+    float4* __restrict__ xg, float4* __restrict__ gxd, float4* __restrict__ gvd,
+    double* __restrict__ kacc, double* __restrict__ macc) {
+    __shared__ __align__(kTileAlign) unsigned char lds[kAdjForceWaves * AdjForceTile::kBytes];
+    const uint32_t wave = uniform_u32(threadIdx.x >> 6);
     const uint32_t n = *n_dev;
-    const uint32_t block0 = xcd_local_block(blockIdx.x, gridDim.x) * kBlock;
-    if (block0 >= n) return;  // block-uniform: the grid covers the capacity
-    const uint32_t s = block0 + threadIdx.x;
-    const bool active = s < n;
-    const float4 vi = active ? tvel[s] : make_float4(0.f, 0.f, 0.f, 0.f);
-    const SceneParams& sp = scenes[active ? __float_as_uint(vi.w) : 0u];
-    const GridView g = sp.g;
-    const float h = sp.p.h, h2 = sp.p.h2;
-    const float4 xi = active ? tpos[s] : make_float4(0.f, 0.f, 0.f, 0.f);
-    const float4 bi = active ? abar[s] : make_float4(0.f, 0.f, 0.f, 0.f);
-    const float2 ABi = active ? make_float2(ixa[s].w, ivb[s].w) : make_float2(0.f, 1.f);
-    const Probe pr = make_probe(g, xi.x, xi.y, xi.z);
-    const uint32_t h2_bits_m1 = __float_as_uint(h2) - 1u;
-    float sumA = 0.f, S1 = 0.f, S2 = 0.f;
+    const GroupRange gr = adjoint_group<kAdjForceWaves>(n, groups, n_groups);
+    if (gr.start >= gr.end) return;
+    const StepParams& p = scenes[gr.scene].p;
+    const GridView& g = scenes[gr.scene].g;
+    uint32_t s;
+    const GroupTargets t = adjoint_targets(g, gr, ixa, s);
+    const float4 xi = target_position(t);
+    const uint32_t own = t.active ? s : gr.start;
+    const float4 vi = ivb[own], bi = abar[own];
+    const float h = p.h;
+    // 0 < r2 < h2 as one unsigned compare (r2 >= +0; non-negative floats order
+    // like their bit patterns).
+    const uint32_t h2_bits_m1 = __float_as_uint(p.h2) - 1u;
+    float sumA = 0.f, S1 = 0.f, Sd = 0.f;  // Sd: sum (h - r) B_j dv.dA
     float gPx = 0.f, gPy = 0.f, gPz = 0.f;   // sum (A_i + A_j)[F dA + F'/r (x.dA) x]
     float gVx = 0.f, gVy = 0.f, gVz = 0.f;   // sum B_j (dv.dA) x / r
     float gWx = 0.f, gWy = 0.f, gWz = 0.f;   // sum (h - r) B_j dA
-
-    // xa = (x_j, A_j), vb = (v_j, B_j), bj = abar_j; requires 0 < r < h.
-    auto pair = [&](float dx, float dy, float dz, float r2, const float4& xa, const float4& vb,
-                    const float4& bj) {
-        const float inv_r = __builtin_amdgcn_rsqf(r2);
-        const float r = r2 * inv_r;
-        const float hr = h - r;
-        const float F = hr * hr * inv_r;
-        const float Fr = -hr * (h + r) * inv_r * inv_r * inv_r;
-        const float ax = bi.x - bj.x, ay = bi.y - bj.y, az = bi.z - bj.z;
-        const float ux = vb.x - vi.x, uy = vb.y - vi.y, uz = vb.z - vi.z;
-        const float xdA = dx * ax + dy * ay + dz * az;
-        const float udA = ux * ax + uy * ay + uz * az;
-        sumA += F * xdA;
-        const float wB = hr * vb.w;
-        S1 += wB * (ux * bi.x + uy * bi.y + uz * bi.z);
-        S2 += wB * (ux * bj.x + uy * bj.y + uz * bj.z);
-        const float pa = ABi.x + xa.w;
-        const float cP = pa * Fr * xdA, pF = pa * F;
-        gPx += pF * ax + cP * dx;
-        gPy += pF * ay + cP * dy;
-        gPz += pF * az + cP * dz;
-        const float cV = vb.w * udA * inv_r;
-        gVx += cV * dx;
-        gVy += cV * dy;
-        gVz += cV * dz;
-        gWx += wB * ax;
-        gWy += wB * ay;
-        gWz += wB * az;
-    };
-    // The scan loads whole groups of kAdjGroup slots: tx must hold them past
-    // a full tile (the loads past a run are masked out by the range test).
-    static_assert(sizeof(tx) / sizeof(tx[0]) >= kAdjForceTile + kAdjGroup,
-                  "the force-adjoint tile must be padded by one group");
-    walk_stencil_staged<kBlock, kAdjForceTile, true>(
-        g, pr, cs, ce, n, active, red,
-        [&](uint32_t k, uint32_t j) {
-            tx[k] = ixa[j];
-            tv[k] = ivb[j];
-            ta[k] = abar[j];
+    walk_group<3>(
+        g, t, p.inv_h, cs, ce, bins, n, ixa, ivb, abar,
+        lds_address(lds) + wave * AdjForceTile::kBytes,
+        [&](const v4f& xa, const v4f& vb, const v4f& bj) {
+            const float dx = xi.x - xa.x, dy = xi.y - xa.y, dz = xi.z - xa.z;
+            const float r2 = dx * dx + dy * dy + dz * dz;
+            const float rs = __builtin_amdgcn_rsqf(r2);
+            const float hr = __builtin_amdgcn_fmed3f(h - r2 * rs, 0.0f, h);
+            const float inv_r = __float_as_uint(r2) - 1u < h2_bits_m1 ? rs : 0.0f;
+            const float hi = hr * inv_r, F = hr * hi;
+            const float Fr = -hi * (h + r2 * inv_r) * inv_r * inv_r;
+            const float ax = bi.x - bj.x, ay = bi.y - bj.y, az = bi.z - bj.z;
+            const float ux = vb.x - vi.x, uy = vb.y - vi.y, uz = vb.z - vi.z;
+            const float xdA = dx * ax + dy * ay + dz * az;
+            const float udA = ux * ax + uy * ay + uz * az;
+            sumA += F * xdA;
+            const float wB = hr * vb.w;
+            S1 += wB * (ux * bi.x + uy * bi.y + uz * bi.z);
+            Sd += wB * udA;
+            const float pa = t.x.w + xa.w;
+            const float cP = pa * Fr * xdA, pF = pa * F;
+            gPx += pF * ax + cP * dx;
+            gPy += pF * ay + cP * dy;
+            gPz += pF * az + cP * dz;
+            const float cV = vb.w * udA * inv_r;
+            gVx += cV * dx;
+            gVy += cV * dy;
+            gVz += cV * dz;
+            gWx += wB * ax;
+            gWy += wB * ay;
+            gWz += wB * az;
         },
-        [&](uint32_t t0, uint32_t t1, uint32_t) {
-            uint32_t cnt = 0;
-            auto flush = [&]() {
-                for (uint32_t k = 0; k < cnt; ++k) {
-                    const uint32_t t = queue[k][threadIdx.x];
-                    const float4 xa = tx[t], va = tv[t], ba = ta[t];
-                    keep_lds_quad(va);
-                    keep_lds_quad(ba);
-                    const float dx = xi.x - xa.x, dy = xi.y - xa.y, dz = xi.z - xa.z;
-                    const float r2 = dx * dx + dy * dy + dz * dz;
-                    pair(dx, dy, dz, r2, xa, va, ba);
-                }
-                cnt = 0;
-            };
-            for (uint32_t t = t0; t < t1; t += kAdjGroup) {
-                float4 q[kAdjGroup];
+        [] {});
+    sumA = both_halves(sumA);
+    S1 = both_halves(S1);
+    Sd = both_halves(Sd);
+    gPx = both_halves(gPx);
+    gPy = both_halves(gPy);
+    gPz = both_halves(gPz);
+    gVx = both_halves(gVx);
+    gVy = both_halves(gVy);
+    gVz = both_halves(gVz);
+    gWx = both_halves(gWx);
+    gWy = both_halves(gWy);
+    gWz = both_halves(gWz);
+    const float Bi = vi.w, ri = rho[min(i2r[own], n - 1)];
+    const float gA = p.c45m * sumA, gB = p.visc * Sd;
+    // The lower lane half sums the group's stiffness terms, the upper one its
+    // viscosity terms, in a fixed order.
+    const bool upper = (threadIdx.x & 32u) != 0u;
+    double acc = !t.active ? 0.0
+                           : static_cast<double>(upper ? p.c45m * Bi * S1
+                                                       : gA * (ri - p.rest_density) * Bi * Bi);
 #pragma unroll
-                for (int u = 0; u < kAdjGroup; ++u) q[u] = tx[t + u];
-#pragma unroll
-                for (int u = 0; u < kAdjGroup; ++u) {
-                    keep_lds_quad(q[u]);
-                    const float dx = xi.x - q[u].x, dy = xi.y - q[u].y, dz = xi.z - q[u].z;
-                    const float r2 = dx * dx + dy * dy + dz * dz;
-                    const bool hit = (t + u < t1) & pair_in_range(r2, h2_bits_m1);
-                    queue[cnt][threadIdx.x] = static_cast<uint16_t>(t + u);
-                    cnt += hit ? 1u : 0u;
-                }
-                if (__ballot(cnt > kAdjQueue - kAdjGroup) != 0ull) flush();
-            }
-            flush();
-        },
-        [&](uint32_t b, uint32_t e) {
-            for (uint32_t j = b; j < e; ++j) {
-                const float4 xj = tpos[j];
-                const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
-                const float r2 = dx * dx + dy * dy + dz * dz;
-                if (!pair_in_range(r2, h2_bits_m1)) continue;
-                pair(dx, dy, dz, r2, ixa[j], ivb[j], abar[j]);
-            }
-        },
-        bins);
-    if (!active) return;
-    const StepParams& p = sp.p;
-    const float Bi = ABi.y, ri = rho[min(i2r[s], n - 1)];
-    const float gA = p.c45m * sumA, gB = p.visc * (S1 - S2);
-    grho[s] = gA * p.stiffness * (2.0f * p.rest_density - ri) * Bi * Bi * Bi - gB * Bi * Bi;
-    kacc[s] += static_cast<double>(gA * (ri - p.rest_density) * Bi * Bi);
-    macc[s] += static_cast<double>(p.c45m * Bi * S1);
+    for (int d = 16; d > 0; d >>= 1) acc += __shfl_xor(acc, d);
+    const uint32_t group = gr.index;
+    if ((threadIdx.x & 31u) == 0u) (upper ? macc : kacc)[group] += acc;
+    if (!t.active || upper) return;
+    xg[s] = make_float4(t.x.x, t.x.y, t.x.z,
+                        gA * p.stiffness * (2.0f * p.rest_density - ri) * Bi * Bi * Bi - gB * Bi * Bi);
     const float vb = p.visc * Bi;
     float4 X = gxd[s], V = gvd[s];
     X.x += p.c45m * gPx - vb * gVx;
@@ -312,94 +292,85 @@ __global__ __launch_bounds__(kBlock) void k_adj_force(
     gvd[s] = V;
 }
 
-// Density-pair adjoint, then the scatter to the step's input order.
-// Candidates are staged in LDS as (x, dL/drho).  Five waves per SIMD fit in
-// 93 VGPRs (the compiler's own choice, 106, allowed four).
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) void k_adj_density(
-    const float4* __restrict__ tpos, const float4* __restrict__ tvel,
-    const float* __restrict__ grho, const uint32_t* __restrict__ cs,
+// Density-pair adjoint, then the scatter to the step's input order.  The group
+// walk with (x, dL/drho) per candidate.
+// Bound by VALU issue; one lane per target with block-staged rows took (us, one
+// million in 16 scenes) 121, this 84 to 92.
+__global__ __launch_bounds__(64 * kAdjDensityWaves) __attribute__((amdgpu_waves_per_eu(5)))
+void k_adj_density(
+    const float4* __restrict__ xg, const uint32_t* __restrict__ cs,
     const uint32_t* __restrict__ ce, const uint4* __restrict__ bins,
     const uint32_t* __restrict__ i2r, const uint32_t* __restrict__ perm,
-    const SceneParams* __restrict__ scenes, const uint32_t* __restrict__ n_dev,
-    const float4* __restrict__ gxd, const float4* __restrict__ gvd, float4* __restrict__ gx,
-    float4* __restrict__ gv) {
-    __shared__ float4 tile[kAdjDensityTile + kAdjGroup];  // padded for whole-group loads
-    __shared__ uint32_t red[2 * kWaves];
+    const SceneParams* __restrict__ scenes, const uint4* __restrict__ groups, uint32_t n_groups,
+    const uint32_t* __restrict__ n_dev, const float4* __restrict__ gxd,
+    const float4* __restrict__ gvd, float4* __restrict__ gx, float4* __restrict__ gv) {
+    __shared__ __align__(kTileAlign) unsigned char lds[kAdjDensityWaves * AdjDensityTile::kBytes];
+    const uint32_t wave = uniform_u32(threadIdx.x >> 6);
     const uint32_t n = *n_dev;
-    const uint32_t block0 = xcd_local_block(blockIdx.x, gridDim.x) * kBlock;
-    if (block0 >= n) return;  // block-uniform: the grid covers the capacity
-    const uint32_t s = block0 + threadIdx.x;
-    const bool active = s < n;
-    const SceneParams& sp = scenes[active ? __float_as_uint(tvel[s].w) : 0u];
-    const GridView g = sp.g;
-    const float h2 = sp.p.h2, inv_h2 = 1.0f / h2;
-    const float4 xi = active ? tpos[s] : make_float4(0.f, 0.f, 0.f, 0.f);
-    const float gi = active ? grho[s] : 0.0f;
-    const Probe pr = make_probe(g, xi.x, xi.y, xi.z);
+    const GroupRange gr = adjoint_group<kAdjDensityWaves>(n, groups, n_groups);
+    if (gr.start >= gr.end) return;
+    const StepParams& p = scenes[gr.scene].p;
+    const GridView& g = scenes[gr.scene].g;
+    uint32_t s;
+    const GroupTargets t = adjoint_targets(g, gr, xg, s);
+    const float4 xi = target_position(t);
+    const float inv_h2 = p.inv_h2;
     // Sums of a^2 (g_i + g_j) x_ij with a = 1 - r^2 / h^2 clamped to [0, 1]
     // (one clamped fused multiply-add): the pair's (h^2 - r^2)^2 is h^4 a^2,
     // and a = 0 out of range.  A coincident pair (x_ij = 0) adds zero.
     float sx = 0.f, sy = 0.f, sz = 0.f;
-    auto pair = [&](float dx, float dy, float dz, float gj, bool live) {
-        const float r2 = dx * dx + dy * dy + dz * dz;
-        const float a = live ? __builtin_amdgcn_fmed3f(__builtin_fmaf(-r2, inv_h2, 1.0f), 0.0f, 1.0f)
-                             : 0.0f;
-        const float c = a * a * (gi + gj);
-        sx += c * dx;
-        sy += c * dy;
-        sz += c * dz;
-    };
-    // Padded: the scan below loads whole groups and multiplies the loads past
-    // its run by a zero weight, which needs them finite.
-    static_assert(sizeof(tile) / sizeof(tile[0]) >= kAdjDensityTile + kAdjGroup,
-                  "the staged walk fills kTile + kPad slots");
-    walk_stencil_staged<kBlock, kAdjDensityTile, true, kAdjGroup>(
-        g, pr, cs, ce, n, active, red,
-        [&](uint32_t k, uint32_t j) {
-            const float4 x = tpos[j];
-            tile[k] = make_float4(x.x, x.y, x.z, grho[j]);
+    walk_group<1>(
+        g, t, p.inv_h, cs, ce, bins, n, xg, nullptr, nullptr,
+        lds_address(lds) + wave * AdjDensityTile::kBytes,
+        [&](const v4f& q) {
+            const float dx = xi.x - q.x, dy = xi.y - q.y, dz = xi.z - q.z;
+            const float r2 = dx * dx + dy * dy + dz * dz;
+            const float a = __builtin_amdgcn_fmed3f(__builtin_fmaf(-r2, inv_h2, 1.0f), 0.0f, 1.0f);
+            const float c = a * a * (t.x.w + q.w);
+            sx += c * dx;
+            sy += c * dy;
+            sz += c * dz;
         },
-        [&](uint32_t t0, uint32_t t1, uint32_t) {
-            for (uint32_t t = t0; t < t1; t += kAdjGroup) {
-                float4 q[kAdjGroup];
-#pragma unroll
-                for (int u = 0; u < kAdjGroup; ++u) q[u] = tile[t + u];
-#pragma unroll
-                for (int u = 0; u < kAdjGroup; ++u) {
-                    keep_lds_quad(q[u]);
-                    // Branch-free: a candidate past the run (a finite pad
-                    // or staged copy) adds zero.
-                    pair(xi.x - q[u].x, xi.y - q[u].y, xi.z - q[u].z, q[u].w, t + u < t1);
-                }
-            }
-        },
-        [&](uint32_t b, uint32_t e) {
-            for (uint32_t j = b; j < e; ++j) {
-                const float4 xj = tpos[j];
-                pair(xi.x - xj.x, xi.y - xj.y, xi.z - xj.z, grho[j], true);
-            }
-        },
-        bins);
-    if (!active) return;
-    const float k6 = -6.0f * sp.p.c6m * (h2 * h2);
+        [] {});
+    sx = both_halves(sx);
+    sy = both_halves(sy);
+    sz = both_halves(sz);
+    if (!t.active) return;
+    const uint32_t q = min(perm[min(i2r[s], n - 1)], n - 1);
+    if ((threadIdx.x & 32u) != 0u) {
+        gv[q] = gvd[s];
+        return;
+    }
+    const float k6 = -6.0f * p.c6m * (p.h2 * p.h2);
     float4 X = gxd[s];
     X.x += k6 * sx;
     X.y += k6 * sy;
     X.z += k6 * sz;
-    const uint32_t q = min(perm[min(i2r[s], n - 1)], n - 1);
     gx[q] = X;
-    gv[q] = gvd[s];
 }
 
-// Per-scene sums of the per-slot FP64 accumulators in a fixed order: one
-// block per scene, strided partial sums, then a tree in LDS.
+// Per-scene sums of the groups' FP64 accumulators in a fixed order: one block
+// per scene, strided partial sums, then a tree in LDS.  (One million particles
+// in 16 scenes, one sum per group instead of one per particle: 71 -> 11 us.)
 __global__ __launch_bounds__(kBlock) void k_scene_reduce(const double* __restrict__ kacc,
                                                          const double* __restrict__ macc,
-                                                         const uint32_t* __restrict__ off,
+                                                         const uint4* __restrict__ groups,
+                                                         uint32_t n_groups,
                                                          double* __restrict__ out) {
     __shared__ double sk[kBlock], sm[kBlock];
     const uint32_t sc = blockIdx.x;
-    const uint32_t b = off[sc], e = off[sc + 1];
+    auto first_of = [&](uint32_t scene) {  // the first group of a scene or a later one
+        uint32_t lo = 0, hi = n_groups;
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (groups[mid].z < scene)
+                lo = mid + 1;
+            else
+                hi = mid;
+        }
+        return lo;
+    };
+    const uint32_t b = first_of(sc), e = first_of(sc + 1);
     double a = 0.0, m = 0.0;
     for (uint32_t i = b + threadIdx.x; i < e; i += kBlock) {
         a += kacc[i];
@@ -427,9 +398,9 @@ size_t al(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
 
 // One recomputed step's record inside a segment.
 struct RolloutSlot {
-    float4 *ipos, *ivel, *accel;  // internal x-order state; accelerations at sorted slots
-    float* rho;                   // sorted slots
-    float4 *ixa, *ivb;            // (x, A), (v, B), internal order
+    float4 *ixa, *ivb;  // (x, A), (v, B), internal order
+    float4* accel;      // sorted slots
+    float* rho;         // sorted slots
     uint32_t *perm, *i2r, *cell_start, *cell_end;
     uint4* xbins;
     hipGraphExec_t graph = nullptr;
@@ -444,7 +415,7 @@ struct sph_rollout {
     float4 *ckpt_pos = nullptr, *ckpt_vel = nullptr;
     std::vector<RolloutSlot> slot;
     float4 *gx, *gv, *abar, *gxd, *gvd;
-    float* grho;
+    float4* xg;  // (x, dL/drho), internal order
     double *kacc, *macc, *red;
     hipEvent_t ev_in = nullptr, ev_out = nullptr;
     // With more than one segment the backward keeps two sets of K records:
@@ -474,8 +445,6 @@ int leave(sph_rollout* r, void* stream) {
 
 StepBuffers slot_buffers(const sph_rollout* r, const RolloutSlot& s) {
     StepBuffers sb = r->b->buf;
-    sb.ipos = s.ipos;
-    sb.ivel = s.ivel;
     sb.ixa = s.ixa;
     sb.ivb = s.ivb;
     sb.i2r = s.i2r;
@@ -511,17 +480,20 @@ int slot_graph(sph_rollout* r, RolloutSlot& s) {
 
 int adjoint_step(sph_rollout* r, const RolloutSlot& s) {
     sph_batch* b = r->b;
-    const uint32_t n = b->n;
     hipStream_t st = b->stream;
-    hipLaunchKernelGGL(k_adj_integrate, blocks_for(n), dim3(kBlock), 0, st, s.ipos, s.ivel,
-                       s.accel, s.i2r, r->gx, r->gv, b->scenes, b->buf.n_dev, r->dt, r->abar,
-                       r->gxd, r->gvd);
-    hipLaunchKernelGGL(k_adj_force, blocks_for(n), dim3(kBlock), 0, st, s.ipos, s.ivel, s.ixa, s.ivb,
-                       s.rho, s.i2r, r->abar, s.cell_start, s.cell_end, s.xbins, b->scenes,
-                       b->buf.n_dev, r->grho, r->gxd, r->gvd, r->kacc, r->macc);
-    hipLaunchKernelGGL(k_adj_density, blocks_for(n), dim3(kBlock), 0, st, s.ipos, s.ivel, r->grho,
-                       s.cell_start, s.cell_end, s.xbins, s.i2r, s.perm, b->scenes, b->buf.n_dev,
-                       r->gxd, r->gvd, r->gx, r->gv);
+    const uint4* const groups = b->buf.groups;
+    const uint32_t ng = b->buf.n_groups;
+    hipLaunchKernelGGL(k_adj_integrate, blocks_for(ng * kGroupTargets), dim3(kBlock), 0, st, s.ixa,
+                       s.ivb, s.accel, s.i2r, r->gx, r->gv, b->scenes, groups, ng, b->buf.n_dev,
+                       r->dt, r->abar, r->gxd, r->gvd);
+    hipLaunchKernelGGL(k_adj_force, dim3((ng + kAdjForceWaves - 1) / kAdjForceWaves),
+                       dim3(64 * kAdjForceWaves), 0, st, s.ixa, s.ivb, s.rho, s.i2r, r->abar,
+                       s.cell_start, s.cell_end, s.xbins, b->scenes, groups, ng, b->buf.n_dev,
+                       r->xg, r->gxd, r->gvd, r->kacc, r->macc);
+    hipLaunchKernelGGL(k_adj_density, dim3((ng + kAdjDensityWaves - 1) / kAdjDensityWaves),
+                       dim3(64 * kAdjDensityWaves), 0, st, r->xg, s.cell_start, s.cell_end, s.xbins,
+                       s.i2r, s.perm, b->scenes, groups, ng, b->buf.n_dev, r->gxd, r->gvd, r->gx,
+                       r->gv);
     SPH_HIP(hipGetLastError());
     return SPH_OK;
 }
@@ -570,16 +542,16 @@ int sph_rollout_create(const sph_config* cfgs, uint32_t n_scenes, const uint32_t
     r->n_steps = n_steps;
     r->every = std::min(checkpoint_every, std::max(n_steps, 1u));
     r->n_ckpt = (n_steps + r->every - 1) / r->every;
-    const size_t N = r->b->n, C = r->b->total_cells, S = r->b->n_scenes;
+    const size_t N = r->b->n, C = r->b->total_cells, S = r->b->n_scenes,
+                 G = r->b->buf.n_groups;
     const uint32_t K = n_steps ? r->every : 0u;
     const size_t n_stored = r->n_ckpt ? r->n_ckpt - 1 : 0;  // the last segment keeps records
     r->n_sets = (r->n_ckpt > 1) ? 2u : 1u;
     std::vector<size_t> sizes = {al(16 * N * n_stored), al(16 * N * n_stored)};
     for (uint32_t k = 0; k < K * r->n_sets; ++k)
-        for (size_t v : {16 * N, 16 * N, 16 * N, 4 * N, 16 * N, 16 * N, 4 * N, 4 * N, 4 * C, 4 * C,
-                         kXBinBytes * C})
+        for (size_t v : {16 * N, 4 * N, 16 * N, 16 * N, 4 * N, 4 * N, 4 * C, 4 * C, kXBinBytes * C})
             sizes.push_back(al(v));
-    for (size_t v : {16 * N, 16 * N, 16 * N, 16 * N, 16 * N, 4 * N, 8 * N, 8 * N, 16 * S})
+    for (size_t v : {16 * N, 16 * N, 16 * N, 16 * N, 16 * N, 16 * N, 8 * G, 8 * G, 16 * S})
         sizes.push_back(al(v));
     size_t total = 0;
     for (size_t v : sizes) total += v;
@@ -610,8 +582,6 @@ int sph_rollout_create(const sph_config* cfgs, uint32_t n_scenes, const uint32_t
     r->ckpt_vel = static_cast<float4*>(take());
     r->slot.resize(static_cast<size_t>(K) * r->n_sets);
     for (auto& s : r->slot) {
-        s.ipos = static_cast<float4*>(take());
-        s.ivel = static_cast<float4*>(take());
         s.accel = static_cast<float4*>(take());
         s.rho = static_cast<float*>(take());
         s.ixa = static_cast<float4*>(take());
@@ -627,7 +597,7 @@ int sph_rollout_create(const sph_config* cfgs, uint32_t n_scenes, const uint32_t
     r->abar = static_cast<float4*>(take());
     r->gxd = static_cast<float4*>(take());
     r->gvd = static_cast<float4*>(take());
-    r->grho = static_cast<float*>(take());
+    r->xg = static_cast<float4*>(take());
     r->kacc = static_cast<double*>(take());
     r->macc = static_cast<double*>(take());
     r->red = static_cast<double*>(take());
@@ -700,8 +670,8 @@ int sph_rollout_backward(sph_rollout* r, const float* grad_final, float* grad_po
     hipLaunchKernelGGL(k_seed, blocks_for(n), dim3(kBlock), 0, b->stream, b->buf.pos, grad_final,
                        n, r->gx, r->gv);
     SPH_HIP(hipGetLastError());
-    SPH_HIP(hipMemsetAsync(r->kacc, 0, 8 * size_t(n), b->stream));
-    SPH_HIP(hipMemsetAsync(r->macc, 0, 8 * size_t(n), b->stream));
+    SPH_HIP(hipMemsetAsync(r->kacc, 0, 8 * size_t(b->buf.n_groups), b->stream));
+    SPH_HIP(hipMemsetAsync(r->macc, 0, 8 * size_t(b->buf.n_groups), b->stream));
     // Segment c's records live in set (last - c) % 2 (the forward wrote the
     // last segment's into set 0).  Segment c - 1 is recomputed on rs while
     // the batch's stream runs the adjoint of segment c; a set is refilled only
@@ -758,7 +728,7 @@ int sph_rollout_backward(sph_rollout* r, const float* grad_final, float* grad_po
         hipLaunchKernelGGL(k_unpack3, blocks_for(n), dim3(kBlock), 0, b->stream, r->gv, n,
                            grad_vel0);
     hipLaunchKernelGGL(k_scene_reduce, dim3(b->n_scenes), dim3(kBlock), 0, b->stream, r->kacc,
-                       r->macc, b->part_offset_dev, r->red);
+                       r->macc, b->buf.groups, b->buf.n_groups, r->red);
     SPH_HIP(hipGetLastError());
     if (grad_stiffness || grad_viscosity) {
         std::vector<double> h(2 * size_t(b->n_scenes));

@@ -100,6 +100,37 @@ struct GroupTargets {
     bool active;
 };
 
+// One group of targets: slots [start, end) of the internal order, all of one
+// scene.  Single scenes are cut every 32 slots; a batch
+// starts anew at each scene (its table of groups), so a scene's groups, and
+// with them its sums, are those of the scene alone.
+struct GroupRange {
+    uint32_t start, end, scene, index;
+};
+
+template <bool kBatched>
+__device__ __forceinline__ GroupRange group_range(uint32_t group, uint32_t n,
+                                                  const uint4* __restrict__ groups,
+                                                  uint32_t n_groups) {
+    GroupRange r{0u, 0u, 0u, group};
+    if (kBatched) {
+        if (group < n_groups) {
+            const uint4 v = groups[group];
+            r.start = uniform_u32(v.x);
+            r.end = min(uniform_u32(v.y), n);
+            r.scene = uniform_u32(v.z);
+        }
+    } else if (group < n_groups) {
+        r.start = group * kGroupTargets;
+        r.end = min(r.start + kGroupTargets, n);
+    }
+    return r;
+}
+
+// The sum of both lane halves' partial sums of a target.
+__device__ __forceinline__ double both_halves(double v) { return v + __shfl_xor(v, 32); }
+__device__ __forceinline__ float both_halves(float v) { return v + __shfl_xor(v, 32); }
+
 // A subgroup: the targets of a group that share a grid row and span at most
 // g.span cells along it.
 struct Subgroup {

@@ -258,33 +258,6 @@ __device__ __forceinline__ float poly6_unit(const float4& xi, const v4f& xj, flo
     return __builtin_amdgcn_fmed3f(__builtin_fmaf(-r2, inv_h2, 1.0f), 0.0f, 1.0f);
 }
 
-// One group of targets: slots [start, end) of the internal order, all of one
-// scene.  Single scenes are cut every 32 slots; a batch
-// starts anew at each scene (its table of groups), so a scene's groups, and
-// with them its sums, are those of the scene alone.
-struct GroupRange {
-    uint32_t start, end, scene;
-};
-
-template <bool kBatched>
-__device__ __forceinline__ GroupRange group_range(uint32_t group, uint32_t n,
-                                                  const uint4* __restrict__ groups,
-                                                  uint32_t n_groups) {
-    GroupRange r{0u, 0u, 0u};
-    if (kBatched) {
-        if (group < n_groups) {
-            const uint4 v = groups[group];
-            r.start = uniform_u32(v.x);
-            r.end = min(uniform_u32(v.y), n);
-            r.scene = uniform_u32(v.z);
-        }
-    } else if (group < n_groups) {
-        r.start = group * kGroupTargets;
-        r.end = min(r.start + kGroupTargets, n);
-    }
-    return r;
-}
-
 // The group's targets: positions, and cells from the sorted keys (a cell's
 // slots are the same in the sorted and the internal order).
 __device__ __forceinline__ GroupTargets load_targets(const GridView& g, const GroupRange& r,
@@ -299,10 +272,6 @@ __device__ __forceinline__ GroupTargets load_targets(const GridView& g, const Gr
     t.key = skeys[at] - g.cell_offset;
     return t;
 }
-
-// The sum of both lane halves' partial sums of a target.
-__device__ __forceinline__ double both_halves(double v) { return v + __shfl_xor(v, 32); }
-__device__ __forceinline__ float both_halves(float v) { return v + __shfl_xor(v, 32); }
 
 // computeDensitiesPressuresD + computeDensityCell (Solver.cu:198-229,536-599):
 // rho_i = m c6 sum_{r_ij < h} (h^2 - r_ij^2)^3, self included, evaluated as

@@ -1,14 +1,15 @@
 """The neighbour walk of groups of 32 particles, where it can go wrong.
 
 Group remainders (1 to 65 particles), a batch whose scenes end inside a group,
-candidate lists from a few to several rings of four 60-candidate words, grid cells smaller and larger than h, a group that spans
-rows or lies at both
-ends of long ones, and particles outside the grid.  Each against the FP64 oracle with the
-suite's bars: density 1e-5 relative, acceleration 1e-5 of max |a*|, for these
+candidate lists from a few to several rings of four 60-candidate words, grid
+cells smaller and larger than h, a group that spans rows or lies at both ends of
+long ones, and particles outside the grid.  Each against the FP64 oracle with
+the suite's bars: density 1e-5 relative, acceleration 1e-5 of max |a*|, for these
 sums of at most a few hundred FP32 terms (FP64 partial sums in the density).
 """
 import numpy as np
 import pytest
+import torch
 
 import oracle as O
 from sph2s_final_amd import (FIELD_ACCEL, FIELD_DENSITY, SPH_DEBUG_ACCEL, BatchSolver,
@@ -111,3 +112,40 @@ def test_batch_groups_restart_at_each_scene(counts):
         at += n
         assert np.max(np.abs(r - ref["rho"]) / ref["rho"]) <= TOL
         assert np.max(np.abs(a - ref["acc"])) <= TOL * np.max(np.abs(ref["acc"]))
+
+
+def test_adjoint_of_uneven_scenes():
+    # The adjoint's groups: remainders, lists of several rings and rows of all
+    # lengths, two steps, against the FP64 adjoint with its suite's bar of 1e-3
+    # (the parameters' against the largest of the batch: a scene's own can
+    # cancel to nothing).
+    from sph2s_final_amd.autograd import Rollout
+    cfg = _config()
+    states = [_state(33, 3, 1.1 * H, 2.4 * H), _state(1, 4, H, 2.0 * H),
+              _state(700, 5, 0.3 * H, 4.2 * H), _state(31, 6, 1.1 * H, 2.4 * H),
+              _state(321, 8, 2.01 * H, 2.99 * H)]
+    refs, seeds = [], []
+    for p, v in states:
+        target = np.roll(p, 1, axis=0).astype(np.float64)
+        refs.append(O.rollout_loss_grad(O.params_from_config(cfg), p, v, scenes.DT, 2, target))
+        seeds.append(2.0 * (refs[-1]["x_final"] - target) / (3.0 * len(p)))
+
+    def dev(parts):
+        return torch.from_numpy(np.ascontiguousarray(np.concatenate(parts), np.float32)).cuda()
+
+    with Rollout([cfg] * len(states), [len(p) for p, _ in states], scenes.DT, 2, 1) as r:
+        r.forward(dev([p for p, _ in states]), dev([v for _, v in states]))
+        gp, gv, gk, gm = r.backward(dev(seeds))
+        torch.cuda.synchronize()
+        assert r.device_errors() == 0
+        gp, gv = gp.cpu().numpy(), gv.cpu().numpy()
+    at = 0
+    for (p, _), ref in zip(states, refs):
+        print(f"case adjoint of {len(p)}", flush=True)
+        for got, want in ((gp, ref["g_pos0"]), (gv, ref["g_vel0"])):
+            err = np.max(np.abs(got[at:at + len(p)] - want))
+            assert err <= 1e-3 * np.max(np.abs(want))
+        at += len(p)
+    for got, name in ((gk, "g_stiffness"), (gm, "g_viscosity")):
+        want = np.array([ref[name] for ref in refs])
+        assert np.max(np.abs(got - want)) <= 1e-3 * np.max(np.abs(want))
