@@ -13,6 +13,8 @@
 // number of candidates tested drops.
 #pragma once
 
+#include <type_traits>
+
 #include "internal.hpp"
 
 namespace sph {
@@ -149,6 +151,32 @@ __device__ __forceinline__ void for_each_run(const GridView& g, const uint32_t* 
 }  // namespace sph
 
 namespace sph {
+
+// Wave helpers: a value made uniform, one lane's value, a prefix sum.
+__device__ __forceinline__ uint32_t uniform_u32(uint32_t v) {
+    return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v)));
+}
+__device__ __forceinline__ uint32_t lane_u32(uint32_t v, int lane) {
+    return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), lane));
+}
+__device__ __forceinline__ float lane_f32(float v, int lane) {
+    return __uint_as_float(lane_u32(__float_as_uint(v), lane));
+}
+
+// Inclusive prefix sum over the wave's 64 lanes (every lane active).
+__device__ __forceinline__ uint32_t wave_scan_add(uint32_t v) {
+    auto step = [&](auto ctrl, auto rows) {
+        v += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(
+            0, static_cast<int>(v), decltype(ctrl)::value, decltype(rows)::value, 0xf, false));
+    };
+    step(std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xf>{});  // row_shr:1
+    step(std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xf>{});  // row_shr:2
+    step(std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xf>{});  // row_shr:4
+    step(std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xf>{});  // row_shr:8
+    step(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});  // row_bcast:15
+    step(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});  // row_bcast:31
+    return v;
+}
 
 // Per-scene constants of a batch: the scene's step parameters and grid, whose
 // cells start at g.cell_offset in the batch's global cell array.

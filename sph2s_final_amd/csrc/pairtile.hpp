@@ -30,8 +30,6 @@
 // on the block size or the grid.
 #pragma once
 
-#include <type_traits>
-
 #include "neighbors.hpp"
 
 namespace sph {
@@ -66,31 +64,6 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-__device__ __forceinline__ uint32_t uniform_u32(uint32_t v) {
-    return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v)));
-}
-__device__ __forceinline__ uint32_t lane_u32(uint32_t v, int lane) {
-    return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), lane));
-}
-__device__ __forceinline__ float lane_f32(float v, int lane) {
-    return __uint_as_float(lane_u32(__float_as_uint(v), lane));
-}
-
-// Inclusive prefix sum over the wave's 64 lanes (every lane active).
-__device__ __forceinline__ uint32_t wave_scan_add(uint32_t v) {
-    auto step = [&](auto ctrl, auto rows) {
-        v += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(
-            0, static_cast<int>(v), decltype(ctrl)::value, decltype(rows)::value, 0xf, false));
-    };
-    step(std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xf>{});  // row_shr:1
-    step(std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xf>{});  // row_shr:2
-    step(std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xf>{});  // row_shr:4
-    step(std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xf>{});  // row_shr:8
-    step(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});  // row_bcast:15
-    step(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});  // row_bcast:31
-    return v;
 }
 
 // Targets of one group: lane l holds target l & 31 (both halves the same).

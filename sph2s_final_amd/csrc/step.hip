@@ -5,11 +5,10 @@
 //                  histograms, plus the empty-cell reset of the ranges
 //                  (computeHashs :401-424 and the two cudaMemsets :1118-1127)
 //   radix passes   stable (hash, slot) sort          (thrust, :1110-1115)
-//   k_reorder      cell start/end, and the gather of x, v into sorted slots
-//                  when a pass needs the sorted copies
-//                  (reorderAndComputeCellStartEndD :478-534)
-//   k_xorder       internal x-order of each cell (reads the state through
-//                  the sort's permutation) and its x-bin table
+//   k_order        cell start/end (reorderAndComputeCellStartEndD :478-534),
+//                  internal x-order of each cell (reads the state through the
+//                  sort's permutation) and its x-bin table, and the state in
+//                  sorted slots when a pass needs it
 //   k_density      Poly6 density                    (:536-599, :198-229)
 //   k_force        spiky pressure + viscosity Laplacian (+ tension) fused with
 //                  symplectic Euler and the wall clamp (:601-711, :713-755)
@@ -29,46 +28,6 @@ namespace {
 
 constexpr int kBlock = 256;
 
-// Boundary detection compares each sorted key with its predecessor read
-// straight from global memory (no block barrier, so no divergent
-// __syncthreads as in the reference at Solver.cu:494-518).  With kCopy the
-// state is also gathered into the sorted copies tpos / tvel; without it only
-// the cell ranges are written (the internal x-order then reads the state
-// through perm itself).
-template <bool kCopy>
-__global__ __launch_bounds__(kBlock) void k_reorder(const uint32_t* __restrict__ skeys,
-                                                    const uint32_t* __restrict__ perm,
-                                                    const float4* __restrict__ pos,
-                                                    const float4* __restrict__ vel,
-                                                    float4* __restrict__ tpos,
-                                                    float4* __restrict__ tvel,
-                                                    uint32_t* __restrict__ cell_start,
-                                                    uint32_t* __restrict__ cell_end,
-                                                    const uint32_t* __restrict__ n_dev,
-                                                    uint32_t num_cells) {
-    const uint32_t n = *n_dev;
-    const uint32_t s = xcd_local_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
-    if (s >= n) return;
-    // Keys are clamped cell hashes (< num_cells) and perm is a permutation of
-    // [0, n); the min() guards keep every access in bounds regardless.
-    const uint32_t k = min(skeys[s], num_cells - 1);
-    if (s == 0) {
-        cell_start[k] = 0;
-    } else {
-        const uint32_t kp = min(skeys[s - 1], num_cells - 1);
-        if (k != kp) {
-            cell_start[k] = s;
-            cell_end[kp] = s;
-        }
-    }
-    if (s == n - 1) cell_end[k] = n;
-    if (kCopy) {
-        const uint32_t j = min(perm[s], n - 1);
-        tpos[s] = pos[j];
-        tvel[s] = vel[j];
-    }
-}
-
 // Internal x-order: slot s of the sorted order (cell c, run [b, e)) moves to
 // b + rank, its rank by (x, sorted slot) among the cell's particles, so each
 // cell's particles are sorted by x (deterministically: ties keep the sorted
@@ -76,67 +35,177 @@ __global__ __launch_bounds__(kBlock) void k_reorder(const uint32_t* __restrict__
 // a direct count over the cell.  The block stages
 // the x of every particle in its cells' runs in LDS (lanes of one cell then
 // read the same LDS word each step); runs beyond the staged range are read
-// from global memory.  The state of sorted slot j is tpos[j] / tvel[j], or,
-// with kPerm, pos[perm[j]] / vel[perm[j]] of the previous order (tpos / tvel
-// then name pos / vel).
+// from global memory.  The state of sorted slot j is pos[perm[j]], vel[perm[j]]
+// of the previous order; with kCopy it is also written to tpos[j], tvel[j].
+//
+// A run's bounds are where neighbouring sorted keys differ: inside the block
+// from ballots, beyond it from the 64 keys on either side, and only for a cell
+// of more particles by a search of the sorted keys.  The first and last slot of
+// a run write the cell's range.  Bound by latency (two rounds of loads) and, at
+// one million, by its 76 MB (15 us at the card's copy rate).  Before, the ranges
+// were a kernel of their own and the ranks compared floats and slots apart: us
+// at 4096 particles / one million 4.6 + 5.8 / 4.8 + 23, now 4.5 / 19.
 constexpr int kXorderTile = 2048;
 
-template <bool kBatched, bool kPerm = false>
-__global__ __launch_bounds__(kBlock) void k_xorder(const uint32_t* __restrict__ skeys,
-                                                   const float4* __restrict__ tpos,
-                                                   const float4* __restrict__ tvel,
-                                                   const uint32_t* __restrict__ cell_start,
-                                                   const uint32_t* __restrict__ cell_end,
-                                                   const uint32_t* __restrict__ n_dev,
-                                                   StepParams p,
-                                                   const SceneParams* __restrict__ scenes,
-                                                   float4* __restrict__ ipos,
-                                                   float4* __restrict__ ivel,
-                                                   uint32_t* __restrict__ i2r,
-                                                   uint4* __restrict__ bins,
-                                                   const uint32_t* __restrict__ perm = nullptr) {
-    __shared__ float xs_tile[kXorderTile];
-    __shared__ uint32_t red[2 * (kBlock / 64)];
+// Bits that order as unsigned like the floats do (-0 as 0; NaNs beyond the
+// infinities), and back.
+__device__ __forceinline__ uint32_t ordered_bits(float x) {
+    const uint32_t u = __float_as_uint(x + 0.0f);
+    return u ^ (static_cast<uint32_t>(static_cast<int32_t>(u) >> 31) | 0x80000000u);
+}
+__device__ __forceinline__ float from_ordered(uint32_t u) {
+    return __uint_as_float(u ^ ((u >> 31) ? 0x80000000u : 0xFFFFFFFFu));
+}
+
+// The first index in [lo, hi) of the sorted keys that holds `key` or more
+// (kAfter: more than `key`), or hi.  All lanes of a wave call it; 64 probes a
+// round.
+template <bool kAfter>
+__device__ __forceinline__ uint32_t search_keys(const uint32_t* __restrict__ skeys, uint32_t lo,
+                                                uint32_t hi, uint32_t key, uint32_t num_cells) {
+    const uint32_t lane = threadIdx.x & 63u;
+    while (lo < hi) {
+        const uint32_t step = (hi - lo + 63u) / 64u;
+        const uint32_t at = lo + lane * step;
+        const uint32_t k = at < hi ? min(skeys[at], num_cells - 1) : 0xFFFFFFFFu;
+        const uint64_t found = __ballot(kAfter ? k > key : k >= key);  // lanes past hi among them
+        const uint32_t f = found ? static_cast<uint32_t>(__builtin_ctzll(found)) : 64u;
+        if (f > 0u) lo += (f - 1u) * step + 1u;
+        if (f > 0u && f < 64u) hi = min(hi, lo + step - 1u);
+        if (f == 0u) hi = lo;
+    }
+    return lo;
+}
+
+template <bool kBatched, bool kCopy>
+__global__ __launch_bounds__(kBlock) void k_order(const uint32_t* __restrict__ skeys,
+                                                  const uint32_t* __restrict__ perm,
+                                                  const float4* __restrict__ pos,
+                                                  const float4* __restrict__ vel,
+                                                  float4* __restrict__ tpos,
+                                                  float4* __restrict__ tvel,
+                                                  uint32_t* __restrict__ cell_start,
+                                                  uint32_t* __restrict__ cell_end,
+                                                  const uint32_t* __restrict__ n_dev, StepParams p,
+                                                  const SceneParams* __restrict__ scenes,
+                                                  float4* __restrict__ ipos,
+                                                  float4* __restrict__ ivel,
+                                                  uint32_t* __restrict__ i2r,
+                                                  uint4* __restrict__ bins) {
+    __shared__ uint32_t xs_tile[kXorderTile];
+    __shared__ uint64_t heads[kBlock / 64];
+    __shared__ uint32_t edge[2];  // where the block's first run starts, its last run ends
     const uint32_t n = *n_dev;
-    auto slot = [&](uint32_t j) { return kPerm ? min(perm[j], n - 1) : j; };
     const uint32_t block0 = blockIdx.x * kBlock;
     if (block0 >= n) return;  // block-uniform
-    const uint32_t s = block0 + threadIdx.x;
+    const uint32_t wave = uniform_u32(threadIdx.x >> 6), lane = threadIdx.x & 63u;
+    const uint32_t s = block0 + threadIdx.x, end = min(block0 + kBlock, n);
     const bool active = s < n;
-    uint32_t key = 0, b = kEmptyCell, e = 0u;
-    if (active) {
-        key = min(skeys[s], p.num_cells - 1);
-        // s lies in its cell's run, so the run is non-empty and b <= s < e <= n.
-        b = min(cell_start[key], s);
-        e = max(min(cell_end[key], n), s + 1);
+    // Keys are clamped cell hashes (< num_cells) and perm is a permutation of
+    // [0, n); the min() guards keep every access in bounds regardless.
+    auto key_at = [&](uint32_t j) { return min(skeys[j], p.num_cells - 1); };
+    auto source = [&](uint32_t j) { return min(perm[j], n - 1); };
+    // Two rounds of loads: the keys and the sources of the block's slots and of
+    // 64 slots on either side (waves 0 and 1 look at the keys there, 2 and 3
+    // take the x), then the states.
+    const uint32_t own = active ? s : end - 1u;
+    const uint32_t src = source(own);
+    const uint32_t key = key_at(own);
+    const uint32_t before = key_at(max(own, 1u) - 1u);
+    const bool low = (wave & 1u) == 0u;  // the slots below the block, nearest first, or above it
+    const bool in = low ? lane < block0 : end + lane < n;
+    const uint32_t at = in ? (low ? block0 - 1u - lane : end + lane) : own;
+    const uint32_t key_last = key_at(end - 1u);
+    const uint32_t* const list = wave < 2u ? skeys : perm;
+    const uint32_t beside = min(list[at], (wave < 2u ? p.num_cells : n) - 1u);
+    // As vectors: a struct copy of which the x is used here goes through an array
+    // in LDS, whose index reads the dispatch packet in host memory (10 us).
+    const v4f xs = *reinterpret_cast<const v4f*>(pos + src);
+    const v4f vs = *reinterpret_cast<const v4f*>(vel + src);
+    if (wave >= 2u && in) xs_tile[low ? 63u - lane : 64u + (end - block0) + lane] = ordered_bits(pos[beside].x);
+    if (active) xs_tile[64u + threadIdx.x] = ordered_bits(xs.x);
+    const bool head = active && (s == 0u || before != key);
+    const uint64_t wave_heads = __ballot(head);
+    if (lane == 0u) heads[wave] = wave_heads;
+    if (wave == 0u) {
+        const uint32_t k0 = uniform_u32(key);  // block0's
+        const uint64_t other = ~__ballot(in && beside == k0);
+        uint32_t b = block0;
+        if ((wave_heads & 1u) == 0u)
+            b = other ? block0 - static_cast<uint32_t>(__builtin_ctzll(other))
+                      : search_keys<false>(skeys, 0u, block0 - 64u, k0, p.num_cells);
+        if (lane == 0u) edge[0] = b;
+    } else if (wave == 1u) {
+        const uint32_t k1 = uniform_u32(key_last);
+        const uint64_t other = ~__ballot(in && beside == k1);
+        const uint32_t e = other ? end + static_cast<uint32_t>(__builtin_ctzll(other))
+                                 : search_keys<true>(skeys, min(end + 64u, n), n, k1, p.num_cells);
+        if (lane == 0u) edge[1] = e;
     }
-    uint32_t ub, ue;
-    block_run_union<kBlock>(b, e, red, ub, ue);
-    const uint32_t seg_n = (ue > ub) ? min(ue - ub, static_cast<uint32_t>(kXorderTile)) : 0u;
-    for (uint32_t k = threadIdx.x; k < seg_n; k += kBlock) xs_tile[k] = tpos[slot(ub + k)].x;
     __syncthreads();
+    // This slot's run [b, e): heads of its own wave, or of the nearest wave that
+    // has one (wave-uniform), or the block's edge.
+    uint32_t b = edge[0], e = edge[1];
+    for (uint32_t w = 0; w < wave; ++w)
+        if (const uint64_t m = heads[w])
+            b = block0 + 64u * w + 63u - static_cast<uint32_t>(__builtin_clzll(m));
+    for (uint32_t w = kBlock / 64; --w > wave;)
+        if (const uint64_t m = heads[w]) e = block0 + 64u * w + static_cast<uint32_t>(__builtin_ctzll(m));
+    const uint64_t upto_lane = ~0ull >> (63u - lane);
+    if (const uint64_t m = wave_heads & upto_lane)
+        b = block0 + 64u * wave + 63u - static_cast<uint32_t>(__builtin_clzll(m));
+    if (const uint64_t m = wave_heads & ~upto_lane)
+        e = block0 + 64u * wave + static_cast<uint32_t>(__builtin_ctzll(m));
+    // The x of slots [from, upto) are staged, from `tile` on.
+    uint32_t from = block0 - min(block0, 64u), upto = min(end + 64u, n);
+    const uint32_t* tile = xs_tile + 64u - (block0 - from);
+    if (edge[0] < from || edge[1] > upto) {  // block-uniform: a run that reaches further
+        from = edge[0];
+        upto = min(edge[1], from + kXorderTile);
+        tile = xs_tile;
+        __syncthreads();
+        for (uint32_t k = threadIdx.x; k < upto - from; k += kBlock)
+            xs_tile[k] = ordered_bits(pos[source(from + k)].x);
+        __syncthreads();
+    }
     if (!active) return;
-    const uint32_t src = slot(s);
-    const float4 xs = tpos[src];
-    const float4 vs = tvel[src];
-    const bool staged = e <= ub + seg_n;
+    if (head) cell_start[key] = s;
+    if (e == s + 1u) cell_end[key] = e;
+    if (kCopy) {
+        *reinterpret_cast<v4f*>(tpos + s) = xs;
+        *reinterpret_cast<v4f*>(tvel + s) = vs;
+    }
+    const bool staged = b >= from && e <= upto;
     // rank: particles before s in (x, sorted slot) order; xg: the smallest x
-    // after it, which is the x of the next particle in the cell's x-order.
-    uint32_t rank = 0;
-    float xg = __builtin_inff();
-    auto count = [&](uint32_t j, float xj) {
-        const bool before = (xj < xs.x) | ((xj == xs.x) & (j < s));
-        rank += before ? 1u : 0u;
-        xg = (!before & (j != s)) ? fminf(xg, xj) : xg;
+    // after it, which is the x of the next particle in the cell's x-order.  One
+    // 64-bit compare a candidate, which counts s itself too.
+    uint32_t upto_s = 0, next = 0xFFFFFFFFu;
+    const uint64_t mine = static_cast<uint64_t>(ordered_bits(xs.x)) << 32 | s;
+    auto count = [&](uint32_t j, uint32_t u) {
+        const bool after = (static_cast<uint64_t>(u) << 32 | j) > mine;
+        upto_s += after ? 0u : 1u;
+        next = after ? min(next, u) : next;
     };
     if (staged) {
-        for (uint32_t j = b; j < e; ++j) count(j, xs_tile[j - ub]);
+        const uint32_t* const xr = tile + (b - from);
+        const uint32_t m = e - b;
+        uint32_t k = 0;
+        for (; k + 4u <= m; k += 4u) {
+            const uint32_t u0 = xr[k], u1 = xr[k + 1], u2 = xr[k + 2], u3 = xr[k + 3];
+            count(b + k, u0);
+            count(b + k + 1, u1);
+            count(b + k + 2, u2);
+            count(b + k + 3, u3);
+        }
+        for (; k < m; ++k) count(b + k, xr[k]);
     } else {
-        for (uint32_t j = b; j < e; ++j) count(j, tpos[slot(j)].x);
+        for (uint32_t j = b; j < e; ++j) count(j, ordered_bits(pos[source(j)].x));
     }
+    const uint32_t rank = upto_s - 1u;
+    const float xg = from_ordered(next);
     const uint32_t q = b + rank;
-    ipos[q] = xs;
-    ivel[q] = vs;
+    *reinterpret_cast<v4f*>(ipos + q) = xs;
+    *reinterpret_cast<v4f*>(ivel + q) = vs;
     i2r[q] = s;
 
     // The cell's x-bin table: cumulative counts of its kXBins x-bins (one
@@ -153,16 +222,16 @@ __global__ __launch_bounds__(kBlock) void k_xorder(const uint32_t* __restrict__ 
             for (int k = 0; k < kXBins; ++k) t[k] = static_cast<uint8_t>(kXBinUnbinned);
         return;
     }
-    float ox = p.ox, inv = 1.0f / p.spacing;
-    uint32_t local = key, dx = static_cast<uint32_t>(p.dx);
+    float ox = p.ox, spacing = p.spacing, inv = 1.0f / p.spacing;
+    int dx = p.dx;
     if (kBatched) {
         const GridView& g = scenes[__float_as_uint(vs.w)].g;
         ox = g.ox;
+        spacing = g.spacing;
         inv = g.inv_spacing;
-        dx = static_cast<uint32_t>(g.dx);
-        local = key - g.cell_offset;
+        dx = g.dx;
     }
-    const float cx = static_cast<float>(local % dx);
+    const float cx = static_cast<float>(cell_coord(xs.x, ox, spacing, dx));
     const int kq = xbin_of((xs.x - ox) * inv - cx);
     const int kn = (rank + 1 < cnt) ? max(kq, xbin_of((xg - ox) * inv - cx)) : kXBins;
     if (rank == 0)
@@ -823,30 +892,15 @@ int launch_pass(int pass, const StepParams& p, const StepBuffers& b, float dt,
             break;
         }
         case kPassReorder: {
+            if (!b.ipos) return set_error(SPH_ERR_INVALID_ARGUMENT, "step buffers lack the x-order");
             // The sorted copies tpos / tvel are read by the colour, wall and
-            // XSPH passes and by a step without the x-order; otherwise the
-            // x-order reads the state through perm and no copy is made.
-            const bool copy = !b.ipos || b.color || (b.walls && b.bacc) ||
-                              (p.flags & SPH_FLAG_XSPH) || b.keep_sorted;
-            if (copy)
-                hipLaunchKernelGGL(k_reorder<true>, blocks_for(p.n), dim3(kBlock), 0, stream,
-                                   b.skeys, b.perm, b.pos, b.vel, b.tpos, b.tvel, b.cell_start,
-                                   b.cell_end, b.n_dev, p.num_cells);
-            else
-                hipLaunchKernelGGL(k_reorder<false>, blocks_for(p.n), dim3(kBlock), 0, stream,
-                                   b.skeys, b.perm, b.pos, b.vel, b.tpos, b.tvel, b.cell_start,
-                                   b.cell_end, b.n_dev, p.num_cells);
-            if (b.ipos) {
-                if (copy)
-                    hipLaunchKernelGGL(k_xorder<false>, blocks_for(p.n), dim3(kBlock), 0, stream,
-                                       b.skeys, b.tpos, b.tvel, b.cell_start, b.cell_end, b.n_dev,
-                                       p, kNoScenes, b.ipos, b.ivel, b.i2r, b.xbins, nullptr);
-                else
-                    hipLaunchKernelGGL((k_xorder<false, true>), blocks_for(p.n), dim3(kBlock), 0,
-                                       stream, b.skeys, b.pos, b.vel, b.cell_start, b.cell_end,
-                                       b.n_dev, p, kNoScenes, b.ipos, b.ivel, b.i2r, b.xbins,
-                                       b.perm);
-            }
+            // XSPH passes and by the two-scale step.
+            const bool copy = b.color || (b.walls && b.bacc) || (p.flags & SPH_FLAG_XSPH) ||
+                              b.keep_sorted;
+            hipLaunchKernelGGL((copy ? k_order<false, true> : k_order<false, false>),
+                               blocks_for(p.n), dim3(kBlock), 0, stream, b.skeys, b.perm, b.pos,
+                               b.vel, b.tpos, b.tvel, b.cell_start, b.cell_end, b.n_dev, p,
+                               kNoScenes, b.ipos, b.ivel, b.i2r, b.xbins);
             break;
         }
         case kPassDensity:
@@ -1090,12 +1144,9 @@ int launch_batch_pass(int pass, const StepParams& cap, const StepBuffers& b,
             // Cell ranges only, then the x-order reads the state through perm
             // (no pass of a batched step reads the sorted copies).
             if (!b.ipos) return set_error(SPH_ERR_INVALID_ARGUMENT, "step buffers lack the x-order");
-            hipLaunchKernelGGL(k_reorder<false>, blocks_for(cap.n), dim3(kBlock), 0, stream, b.skeys,
-                               b.perm, b.pos, b.vel, b.tpos, b.tvel, b.cell_start, b.cell_end,
-                               b.n_dev, cap.num_cells);
-            hipLaunchKernelGGL((k_xorder<true, true>), blocks_for(cap.n), dim3(kBlock), 0, stream,
-                               b.skeys, b.pos, b.vel, b.cell_start, b.cell_end, b.n_dev, cap,
-                               scenes, b.ipos, b.ivel, b.i2r, b.xbins, b.perm);
+            hipLaunchKernelGGL((k_order<true, false>), blocks_for(cap.n), dim3(kBlock), 0, stream,
+                               b.skeys, b.perm, b.pos, b.vel, b.tpos, b.tvel, b.cell_start,
+                               b.cell_end, b.n_dev, cap, scenes, b.ipos, b.ivel, b.i2r, b.xbins);
             break;
         }
         case kPassDensity:
