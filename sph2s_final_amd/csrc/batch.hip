@@ -120,6 +120,11 @@ int batch_alloc(const sph_config* cfgs, uint32_t n_scenes, const uint32_t* count
         for (uint32_t i = b->part_offset[s]; i < b->part_offset[s + 1]; i += kGroupTargets)
             groups.push_back(make_uint4(i, std::min(i + kGroupTargets, b->part_offset[s + 1]), s, 0u));
     b->buf.n_groups = static_cast<uint32_t>(groups.size());
+    uint32_t largest = 0, cells_of_one = 0;
+    for (uint32_t s = 0; s < n_scenes; ++s) {
+        largest = std::max(largest, counts[s]);
+        cells_of_one = std::max(cells_of_one, b->cell_offset[s + 1] - b->cell_offset[s]);
+    }
 
     const size_t N = b->n, C = b->total_cells;
     const size_t sort_temp = radix_sort_temp_bytes(b->n);
@@ -175,6 +180,8 @@ int batch_alloc(const sph_config* cfgs, uint32_t n_scenes, const uint32_t* count
     b->buf.xbins = static_cast<uint4*>(take());
     uint4* const groups_dev = static_cast<uint4*>(take());
     b->buf.groups = groups_dev;
+    b->buf.segments =
+        SceneSegments{b->part_offset_dev, n_scenes, largest, key_bits_for_cells(cells_of_one)};
 
     e = hipMemsetAsync(b->arena, 0, total, b->stream);
     if (e == hipSuccess)

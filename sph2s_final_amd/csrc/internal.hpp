@@ -122,11 +122,24 @@ int hash_hist_cells(const StepParams& p, const uint32_t* n_dev, const float4* po
                     uint32_t key_bits, void* temp, size_t temp_bytes, uint32_t* cell_start,
                     uint32_t* cell_end, hipStream_t stream);
 // The digit passes: (keys, slot) -> (skeys, perm).
+// Hash, sort and reset of the cell ranges in one launch, where the largest
+// segment (a scene, or all of a single scene's slots) fits a block's sort.
+bool block_sort_fits(uint32_t largest);
+int sort_cells_block(const StepParams& p, const uint32_t* n_dev, const float4* pos, uint32_t* skeys,
+                     uint32_t* perm, uint32_t key_bits, uint32_t* cell_start, uint32_t* cell_end,
+                     hipStream_t stream);
 int sort_cells(const StepParams& p, const uint32_t* keys, uint32_t* skeys, uint32_t* perm,
                uint32_t key_bits, void* temp, hipStream_t stream);
 
 // ---- single-scale step kernels (step.hip) ----
 struct Walls;  // boundary-particle walls (walls.hpp)
+
+// Batched scenes: first slot of each (and the end), their number, the largest
+// count and the key bits of the largest grid.
+struct SceneSegments {
+    const uint32_t* off;
+    uint32_t count, largest, key_bits;
+};
 
 struct StepBuffers {
     float4* pos;        // state, sorted order of the previous step (w = id bits)
@@ -168,6 +181,7 @@ struct StepBuffers {
     // as (first slot, end, scene, 0); n_groups of them.
     const uint4* groups;
     uint32_t n_groups;
+    SceneSegments segments;
 };
 
 // Passes of one step, in launch order.

@@ -192,6 +192,9 @@ int hash_hist_cells_batched(const StepParams& cap, const uint32_t* n_dev, const 
                             const float4* vel, const SceneParams* scenes, uint32_t* keys,
                             uint32_t key_bits, void* temp, size_t temp_bytes,
                             uint32_t* cell_start, uint32_t* cell_end, hipStream_t stream);
+int sort_cells_block_batched(const StepParams& cap, const SceneSegments& seg, const float4* pos,
+                             const SceneParams* scenes, uint32_t* skeys, uint32_t* perm,
+                             uint32_t* cell_start, uint32_t* cell_end, hipStream_t stream);
 int launch_batch_pass(int pass, const StepParams& cap, const StepBuffers& b,
                       const SceneParams* scenes, bool kahan, bool tension, float dt,
                       uint32_t key_bits, bool write_accel, hipStream_t stream);

@@ -2,8 +2,9 @@
 // for gfx950.  Replaces thrust::sort_by_key(hash, ids)
 // (SPH2S_FINAL_SINGLE_SCALE/Solver.cu:1110-1115).
 //
-// Single-sweep scheme, 10-bit digits (fewer bits in the last pass; 19-bit
-// cell hashes take two passes), one thread per digit in the pass kernel:
+// Up to kBlockSortMax pairs (of a scene, in a batch): k_sort_block, one block.
+// Beyond, a single-sweep scheme, digits of up to 10 bits (19-bit cell hashes take
+// two passes), one thread per digit in the pass kernel:
 //   k_prepare   zeroes the digit histograms, tile tickets and look-back
 //               status words (and, for the solver, resets the cell ranges)
 //   k_hist      one read of the keys -> LDS digit histograms of every pass
@@ -165,7 +166,7 @@ struct BatchHashKeys {
 // is counted.
 template <class Src>
 __global__ __launch_bounds__(kBlock) void k_hist(Src src, const uint32_t* __restrict__ n_dev,
-                                                 int passes, uint32_t key_bits,
+                                                 int passes, int width, uint32_t key_bits,
                                                  uint32_t* __restrict__ ghist) {
     constexpr int kHistItems = Src::kHistItems;
     constexpr uint32_t kHistTile = kBlock * kHistItems;
@@ -190,8 +191,8 @@ __global__ __launch_bounds__(kBlock) void k_hist(Src src, const uint32_t* __rest
         const bool valid = static_cast<uint32_t>(lane) < nvalid;
         const uint32_t prev = static_cast<uint32_t>(__shfl_up(static_cast<int>(key[r]), 1));
         for (int p = 0; p < passes; ++p) {
-            const int shift = kDigitBits * p;
-            const int bits = min(kDigitBits, static_cast<int>(key_bits) - shift);
+            const int shift = width * p;
+            const int bits = min(width, static_cast<int>(key_bits) - shift);
             const uint32_t m = (1u << bits) - 1u;
             const uint32_t d = (key[r] >> shift) & m;
             const bool start = valid && (lane == 0 || ((prev >> shift) & m) != d);
@@ -206,7 +207,7 @@ __global__ __launch_bounds__(kBlock) void k_hist(Src src, const uint32_t* __rest
     }
     __syncthreads();
     for (int p = 0; p < passes; ++p) {
-        const int bits = min(kDigitBits, static_cast<int>(key_bits) - kDigitBits * p);
+        const int bits = min(width, static_cast<int>(key_bits) - width * p);
         for (int d = threadIdx.x; d < (1 << bits); d += kBlock)
             if (cnt[p][d]) atomicAdd(&ghist[p * kRadix + d], cnt[p][d]);
     }
@@ -344,6 +345,189 @@ __global__ __launch_bounds__(kPassBlock) void k_pass(
     }
 }
 
+// Digit passes of a key, and their width: the bits divided evenly, so that 11-bit
+// keys take digits of 6 and 5 bits and not of 10 and 1.
+inline int passes_for(uint32_t key_bits) { return static_cast<int>((key_bits + kDigitBits - 1) / kDigitBits); }
+inline int width_for(uint32_t key_bits) {
+    const int passes = passes_for(key_bits);
+    return (static_cast<int>(key_bits) + passes - 1) / passes;
+}
+
+// ---- few keys: one block sorts them all --------------------------------------
+// At a few thousand keys the four launches of the general sort are latency.  Here
+// one block keeps a segment of up to 1024 kSegItems pairs in registers and LDS
+// through every digit pass, and further blocks clear the cell ranges.  A batch has
+// a block per scene: the scenes' slots and key ranges do not mix.  A sort of
+// (keys, bits) took, general -> block, us: (2000, 12) 21 -> 7.6, (4096, 19) 29 ->
+// 12.3, (8000, 17) 29 -> 18.4, (12000, 17) 27 -> 29.7, where the line lies: one
+// block's ranking rounds then cost what the launches did.
+constexpr uint32_t kBlockSortMax = 10u * 1024u;
+
+// What a block sorts: slots [off[b], off[b + 1]) (off null: [0, live count)).
+struct SortSegments {
+    const uint32_t* off;
+    const uint32_t* n_dev;  // off null: the live count, or n if null too
+    uint32_t n, blocks;
+};
+
+// Keys of a segment less its base (the first key of a scene's range): an array's;
+// cell hashes of positions; the same with the scene's grid.  at(b): segment b's.
+struct SegmentArray {
+    const uint32_t* keys;
+    static constexpr uint32_t base = 0u;
+    __device__ uint32_t operator()(uint32_t i) const { return keys[i]; }
+    __device__ SegmentArray at(uint32_t) const { return *this; }
+};
+struct SegmentHash {
+    const float4* pos;
+    float ox, oy, oz, spacing;
+    int dx, dy, dz;
+    uint32_t base;
+    __device__ uint32_t operator()(uint32_t i) const {
+        const float4 x = pos[i];
+        return cell_hash(x.x, x.y, x.z, ox, oy, oz, spacing, dx, dy, dz);
+    }
+    __device__ SegmentHash at(uint32_t) const { return *this; }
+};
+struct SegmentScenes {
+    const float4* pos;
+    const SceneParams* scenes;
+    __device__ SegmentHash at(uint32_t b) const {
+        const GridView& g = scenes[b].g;
+        return SegmentHash{pos, g.ox, g.oy, g.oz, g.spacing, g.dx, g.dy, g.dz, g.cell_offset};
+    }
+};
+
+template <class Src, int kSegItems>
+__global__ __launch_bounds__(1024) void k_sort_block(Src src, SortSegments seg,
+                                                     const uint32_t* __restrict__ vals_in,
+                                                     uint32_t* __restrict__ keys_out,
+                                                     uint32_t* __restrict__ vals_out, int passes,
+                                                     int width, int key_bits,
+                                                     uint32_t* __restrict__ fill_a,
+                                                     uint32_t* __restrict__ fill_b,
+                                                     uint32_t fill_words) {
+    constexpr int kSegWaves = 16;
+    __shared__ uint32_t lkey[1024 * kSegItems];
+    __shared__ uint16_t lsrc[1024 * kSegItems];
+    __shared__ __align__(16) uint16_t wcnt[kSegWaves * kRadix];
+    __shared__ uint32_t dbase[kRadix], wsum[kSegWaves];
+    const int t = threadIdx.x;
+    if (blockIdx.x >= seg.blocks) {
+        const uint32_t stride = (gridDim.x - seg.blocks) * 1024u;
+        for (uint32_t i = (blockIdx.x - seg.blocks) * 1024u + t; i < fill_words; i += stride) {
+            fill_a[i] = kEmptyCell;
+            fill_b[i] = kEmptyCell;
+        }
+        return;
+    }
+    const uint32_t first = seg.off ? seg.off[blockIdx.x] : 0u;
+    const uint32_t live = seg.off ? seg.off[blockIdx.x + 1] - first : seg.n_dev ? *seg.n_dev : seg.n;
+    const uint32_t n = min(live, 1024u * kSegItems);
+    if (n == 0u) return;  // block-uniform
+    const int wave = t >> 6, lane = t & 63;
+    const uint64_t lt = lanemask_lt(lane);
+    const auto key_of = src.at(blockIdx.x);
+    const uint32_t base = wave * (64 * kSegItems);
+    // Of each pair its key and, in 16 bits each, its slot in the segment and its
+    // rank among the wave's equal digits.
+    uint32_t key[kSegItems], from[kSegItems];
+#pragma unroll
+    for (int r = 0; r < kSegItems; ++r) {
+        from[r] = base + r * 64 + lane;
+        key[r] = key_of(first + min(from[r], n - 1u));  // no branch: the loads go out together
+    }
+    for (int p = 0; p < passes; ++p) {
+        const int shift = p * width, bits = min(width, key_bits - shift), radix = 1 << bits;
+        const uint32_t mask = static_cast<uint32_t>(radix - 1);
+        for (int i = t; i < kSegWaves * radix / 2; i += 1024) reinterpret_cast<uint32_t*>(wcnt)[i] = 0u;
+        __syncthreads();
+        uint16_t* const mine = wcnt + wave * radix;
+#pragma unroll
+        for (int r = 0; r < kSegItems; ++r) {
+            const bool valid = base + r * 64 + lane < n;
+            const uint32_t d = (key[r] >> shift) & mask;
+            const uint64_t peers = match_digit(d, valid, bits);
+            const uint32_t before = mine[d];
+            from[r] |= (before + static_cast<uint32_t>(__popcll(peers & lt))) << 16;
+            // One wave instruction reads the count before the leader's write, and
+            // the written value depends on the read, so all lanes see the old count.
+            if (valid && lane == __builtin_ctzll(peers))
+                mine[d] = static_cast<uint16_t>(before + static_cast<uint32_t>(__popcll(peers)));
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_sched_barrier(0);  // one round's masks at a time
+        }
+        __syncthreads();
+        uint32_t run = 0;
+        if (t < radix) {
+            for (int w = 0; w < kSegWaves; ++w) {
+                const uint32_t c = wcnt[w * radix + t];
+                wcnt[w * radix + t] = static_cast<uint16_t>(run);
+                run += c;
+            }
+        }
+        const uint32_t upto = wave_scan_add(run);
+        if (lane == 63) wsum[wave] = upto;
+        __syncthreads();
+        uint32_t excl = upto - run;
+        for (int w = 0; w < wave; ++w) excl += wsum[w];
+        if (t < radix) dbase[t] = excl;
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kSegItems; ++r) {
+            if (base + r * 64 + lane < n) {
+                asm volatile("" : "+v"(key[r]));  // the digit again: no register held for it
+                const uint32_t d = (key[r] >> shift) & mask;
+                const uint32_t dst = min(dbase[d] + mine[d] + (from[r] >> 16), 1024u * kSegItems - 1u);
+                lkey[dst] = key[r];
+                lsrc[dst] = static_cast<uint16_t>(from[r]);
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kSegItems; ++r) {
+            const uint32_t i = base + r * 64 + lane;
+            if (i < n) {
+                key[r] = lkey[i];
+                from[r] = lsrc[i];
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < kSegItems; ++r) {
+        const uint32_t i = base + r * 64 + lane;
+        if (i < n) {
+            keys_out[first + i] = key[r] + key_of.base;
+            vals_out[first + i] = vals_in ? vals_in[first + from[r]] : first + from[r];
+        }
+    }
+}
+
+template <class Src>
+int sort_segments(Src src, const SortSegments& seg, uint32_t largest, const uint32_t* vals_in,
+                  uint32_t* keys_out, uint32_t* vals_out, uint32_t key_bits, uint32_t* fill_a,
+                  uint32_t* fill_b, uint32_t fill_words, hipStream_t stream) {
+    const uint32_t fill_blocks = std::min((fill_words + 8191u) / 8192u, 256u);
+    const int passes = passes_for(key_bits), width = width_for(key_bits);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(seg.blocks + fill_blocks), dim3(1024), 0, stream, src, seg,
+                           vals_in, keys_out, vals_out, passes, width, static_cast<int>(key_bits),
+                           fill_a, fill_b, fill_words);
+    };
+    if (largest <= 2048u)
+        launch(k_sort_block<Src, 2>);
+    else if (largest <= 4096u)
+        launch(k_sort_block<Src, 4>);
+    else if (largest <= 6144u)
+        launch(k_sort_block<Src, 6>);
+    else if (largest <= 8192u)
+        launch(k_sort_block<Src, 8>);
+    else
+        launch(k_sort_block<Src, 10>);
+    SPH_HIP(hipGetLastError());
+    return SPH_OK;
+}
+
 constexpr uint32_t tiles_for(uint32_t n) { return (n + kTile - 1) / kTile; }
 constexpr size_t align_up(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
 
@@ -404,7 +588,7 @@ int prepare_hist(Src src, uint32_t cap, const uint32_t* n_src, uint32_t n_host, 
                  hipStream_t stream) {
     const uint32_t tiles = tiles_for(cap);
     const TempLayout L = layout(temp, cap);
-    const int passes = static_cast<int>((key_bits + kDigitBits - 1) / kDigitBits);
+    const int passes = passes_for(key_bits);
     const uint32_t zero_words =
         static_cast<uint32_t>(L.status - L.header) + static_cast<uint32_t>(passes) * tiles * kRadix;
     const uint32_t prep_words = zero_words > fill_words ? zero_words : fill_words;
@@ -414,7 +598,7 @@ int prepare_hist(Src src, uint32_t cap, const uint32_t* n_src, uint32_t n_host, 
     constexpr uint32_t kHistTile = kBlock * Src::kHistItems;
     const uint32_t hist_blocks = std::max(1u, (cap + kHistTile - 1) / kHistTile);
     hipLaunchKernelGGL(k_hist<Src>, dim3(hist_blocks), dim3(kBlock), 0, stream, src,
-                       L.header + kNWord, passes, key_bits, L.header);
+                       L.header + kNWord, passes, width_for(key_bits), key_bits, L.header);
     SPH_HIP(hipGetLastError());
     return SPH_OK;
 }
@@ -425,12 +609,12 @@ int run_passes(const uint32_t* keys_in, const uint32_t* vals_in, uint32_t* keys_
                hipStream_t stream) {
     const uint32_t tiles = tiles_for(cap);
     const TempLayout L = layout(temp, cap);
-    const int passes = static_cast<int>((key_bits + kDigitBits - 1) / kDigitBits);
+    const int passes = passes_for(key_bits), width = width_for(key_bits);
     const uint32_t* kin = keys_in;
     const uint32_t* vin = vals_in;
     for (int p = 0; p < passes; ++p) {
-        const int shift = kDigitBits * p;
-        const int bits = std::min(kDigitBits, static_cast<int>(key_bits) - shift);
+        const int shift = width * p;
+        const int bits = std::min(width, static_cast<int>(key_bits) - shift);
         const bool to_out = ((passes - 1 - p) % 2) == 0;
         uint32_t* kout = to_out ? keys_out : L.ktmp;
         uint32_t* vout = to_out ? vals_out : L.vtmp;
@@ -459,6 +643,9 @@ int radix_sort_pairs(const uint32_t* keys_in, const uint32_t* vals_in, uint32_t*
     int rc = check_sort_args(keys_in, vals_in, keys_out, vals_out, n, key_bits, temp, temp_bytes);
     if (rc != SPH_OK || n == 0) return rc;
     if (!keys_in) return set_error(SPH_ERR_INVALID_ARGUMENT, "radix sort: null keys");
+    if (n <= kBlockSortMax)
+        return sort_segments(SegmentArray{keys_in}, SortSegments{nullptr, nullptr, n, 1u}, n, vals_in,
+                             keys_out, vals_out, key_bits, nullptr, nullptr, 0u, stream);
     rc = prepare_hist(ArrayKeys{keys_in}, n, nullptr, n, key_bits, temp, nullptr, nullptr, 0u,
                       stream);
     if (rc != SPH_OK) return rc;
@@ -484,6 +671,26 @@ int hash_hist_cells_batched(const StepParams& cap, const uint32_t* n_dev, const 
     BatchHashKeys src{pos, vel, scenes, keys};
     return prepare_hist(src, cap.n, n_dev, cap.n, key_bits, temp, cell_start, cell_end,
                         cap.num_cells, stream);
+}
+
+// The block sort's hash and sort (and the reset of the cell ranges) in one
+// launch, for segments of at most kBlockSortMax slots.
+bool block_sort_fits(uint32_t largest) { return largest <= kBlockSortMax; }
+
+int sort_cells_block(const StepParams& p, const uint32_t* n_dev, const float4* pos, uint32_t* skeys,
+                     uint32_t* perm, uint32_t key_bits, uint32_t* cell_start, uint32_t* cell_end,
+                     hipStream_t stream) {
+    const SegmentHash src{pos, p.ox, p.oy, p.oz, p.spacing, p.dx, p.dy, p.dz, 0u};
+    return sort_segments(src, SortSegments{nullptr, n_dev, p.n, 1u}, p.n, nullptr, skeys, perm,
+                         key_bits, cell_start, cell_end, p.num_cells, stream);
+}
+
+int sort_cells_block_batched(const StepParams& cap, const SceneSegments& seg, const float4* pos,
+                             const SceneParams* scenes, uint32_t* skeys, uint32_t* perm,
+                             uint32_t* cell_start, uint32_t* cell_end, hipStream_t stream) {
+    return sort_segments(SegmentScenes{pos, scenes}, SortSegments{seg.off, nullptr, 0u, seg.count},
+                         seg.largest, nullptr, skeys, perm, seg.key_bits, cell_start, cell_end,
+                         cap.num_cells, stream);
 }
 
 int sort_cells(const StepParams& p, const uint32_t* keys, uint32_t* skeys, uint32_t* perm,

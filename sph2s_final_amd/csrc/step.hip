@@ -881,13 +881,18 @@ int launch_pass(int pass, const StepParams& p, const StepBuffers& b, float dt,
     const GridView g = make_grid_view(p.ox, p.oy, p.oz, p.spacing, p.dx, p.dy, p.dz, p.h);
     switch (pass) {
         case kPassHash: {
+            if (block_sort_fits(p.n)) break;  // with the sort
             const int rc = hash_hist_cells(p, b.n_dev, b.pos, b.keys, key_bits, b.sort_temp,
                                            b.sort_temp_bytes, b.cell_start, b.cell_end, stream);
             if (rc != SPH_OK) return rc;
             break;
         }
         case kPassSort: {
-            const int rc = sort_cells(p, b.keys, b.skeys, b.perm, key_bits, b.sort_temp, stream);
+            const int rc =
+                block_sort_fits(p.n)
+                    ? sort_cells_block(p, b.n_dev, b.pos, b.skeys, b.perm, key_bits, b.cell_start,
+                                       b.cell_end, stream)
+                    : sort_cells(p, b.keys, b.skeys, b.perm, key_bits, b.sort_temp, stream);
             if (rc != SPH_OK) return rc;
             break;
         }
@@ -1132,14 +1137,22 @@ int launch_batch_pass(int pass, const StepParams& cap, const StepBuffers& b,
                                        cap.h);
     switch (pass) {
         case kPassHash: {
+            if (block_sort_fits(b.segments.largest)) break;  // with the sort
             const int rc = hash_hist_cells_batched(cap, b.n_dev, b.pos, b.vel, scenes, b.keys,
                                                    key_bits, b.sort_temp, b.sort_temp_bytes,
                                                    b.cell_start, b.cell_end, stream);
             if (rc != SPH_OK) return rc;
             break;
         }
-        case kPassSort:
-            return launch_pass(pass, cap, b, dt, key_bits, write_accel, stream);
+        case kPassSort: {
+            const int rc =
+                block_sort_fits(b.segments.largest)
+                    ? sort_cells_block_batched(cap, b.segments, b.pos, scenes, b.skeys, b.perm,
+                                               b.cell_start, b.cell_end, stream)
+                    : sort_cells(cap, b.keys, b.skeys, b.perm, key_bits, b.sort_temp, stream);
+            if (rc != SPH_OK) return rc;
+            break;
+        }
         case kPassReorder: {
             // Cell ranges only, then the x-order reads the state through perm
             // (no pass of a batched step reads the sorted copies).

@@ -44,3 +44,34 @@ def test_runs_at_block_edges(sizes):
     assert np.array_equal(got[FIELD_CELL_START], ref["cell_start"])
     assert np.array_equal(got[FIELD_CELL_END], ref["cell_end"])
     assert np.max(np.abs(rho - ref["rho"]) / ref["rho"]) <= 1e-5
+
+
+@pytest.mark.parametrize("n", [1, 63, 1023, 1025, 2047, 2048, 2049, 4096, 4097, 6144, 6145, 8193,
+                               10239, 10240, 10241])
+@pytest.mark.parametrize("bits", [1, 11, 20, 32])
+def test_sorts_of_few_pairs(n, bits):
+    # Around each block-sort size and the line to the general sort: a stable
+    # sort, against numpy's.
+    import ctypes
+
+    import torch
+
+    import sph2s_final_amd as sph
+    rng = np.random.default_rng(n + bits)
+    keys = rng.integers(0, 1 << bits, n, dtype=np.uint64).astype(np.uint32)
+    keys[n // 2:] = keys[n // 2:] & np.uint32((1 << max(bits // 2, 1)) - 1)
+    vals = rng.integers(0, 1 << 32, n, dtype=np.uint64).astype(np.uint32)
+    dev = [torch.from_numpy(a.view(np.int32)).cuda() for a in (keys, vals)]
+    out = [torch.empty_like(d) for d in dev]
+    size = int(sph.lib().sph_radix_sort_temp_bytes(n))
+    temp = torch.empty(size, dtype=torch.uint8, device="cuda")
+    print(f"case sort {n} pairs of {bits} bits", flush=True)
+    rc = sph.lib().sph_radix_sort_pairs(
+        *[ctypes.c_void_p(d.data_ptr()) for d in dev + out], ctypes.c_uint32(n),
+        ctypes.c_uint32(bits), ctypes.c_void_p(temp.data_ptr()), size,
+        ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0
+    torch.cuda.synchronize()
+    order = np.argsort(keys, kind="stable")
+    assert np.array_equal(out[0].cpu().numpy().view(np.uint32), keys[order])
+    assert np.array_equal(out[1].cpu().numpy().view(np.uint32), vals[order])
