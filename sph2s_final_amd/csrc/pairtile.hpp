@@ -104,6 +104,21 @@ __device__ __forceinline__ GroupRange group_range(uint32_t group, uint32_t n,
 __device__ __forceinline__ double both_halves(double v) { return v + __shfl_xor(v, 32); }
 __device__ __forceinline__ float both_halves(float v) { return v + __shfl_xor(v, 32); }
 
+// The group's targets: positions, and cells from the sorted keys (a cell's
+// slots are the same in the sorted and the internal order).
+__device__ __forceinline__ GroupTargets load_targets(const GridView& g, const GroupRange& r,
+                                                     const float4* __restrict__ tpos,
+                                                     const uint32_t* __restrict__ skeys,
+                                                     uint32_t& s) {
+    GroupTargets t;
+    s = r.start + (threadIdx.x & 31u);
+    t.active = s < r.end;
+    const uint32_t at = t.active ? s : r.start;
+    t.x = tpos[at];
+    t.key = skeys[at] - g.cell_offset;
+    return t;
+}
+
 // A subgroup: the targets of a group that share a grid row and span at most
 // g.span cells along it.
 struct Subgroup {

@@ -327,21 +327,6 @@ __device__ __forceinline__ float poly6_unit(const float4& xi, const v4f& xj, flo
     return __builtin_amdgcn_fmed3f(__builtin_fmaf(-r2, inv_h2, 1.0f), 0.0f, 1.0f);
 }
 
-// The group's targets: positions, and cells from the sorted keys (a cell's
-// slots are the same in the sorted and the internal order).
-__device__ __forceinline__ GroupTargets load_targets(const GridView& g, const GroupRange& r,
-                                                     const float4* __restrict__ tpos,
-                                                     const uint32_t* __restrict__ skeys,
-                                                     uint32_t& s) {
-    GroupTargets t;
-    s = r.start + (threadIdx.x & 31u);
-    t.active = s < r.end;
-    const uint32_t at = t.active ? s : r.start;
-    t.x = tpos[at];
-    t.key = skeys[at] - g.cell_offset;
-    return t;
-}
-
 // computeDensitiesPressuresD + computeDensityCell (Solver.cu:198-229,536-599):
 // rho_i = m c6 sum_{r_ij < h} (h^2 - r_ij^2)^3, self included, evaluated as
 // (m c6 h^6) sum a^3 with a = 1 - r_ij^2 / h^2 (poly6_unit).  Terms are added in
@@ -1025,22 +1010,6 @@ int launch_gather_aux(const StepParams& p, const StepBuffers& b, hipStream_t str
     if (p.n == 0) return SPH_OK;
     hipLaunchKernelGGL(k_gather_aux, blocks_for(p.n), dim3(kBlock), 0, stream, b.aux, b.i2r,
                        b.n_dev, b.ipos, b.ivel, b.ixa, b.ivb);
-    SPH_HIP(hipGetLastError());
-    return SPH_OK;
-}
-
-__global__ __launch_bounds__(kBlock) void k_gather_x(const float2* __restrict__ src,
-                                                     const uint32_t* __restrict__ i2r,
-                                                     const uint32_t* __restrict__ n_dev,
-                                                     float2* __restrict__ dst) {
-    const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
-    if (s < *n_dev) dst[s] = src[i2r[s]];
-}
-
-int launch_gather_x(const float2* src, const uint32_t* i2r, const uint32_t* n_dev, uint32_t cap,
-                    float2* dst, hipStream_t stream) {
-    if (cap == 0) return SPH_OK;
-    hipLaunchKernelGGL(k_gather_x, blocks_for(cap), dim3(kBlock), 0, stream, src, i2r, n_dev, dst);
     SPH_HIP(hipGetLastError());
     return SPH_OK;
 }

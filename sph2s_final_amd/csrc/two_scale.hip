@@ -42,7 +42,7 @@
 
 #include "diagnostics.hpp"
 #include "neighbors.hpp"
-#include "pairwalk.hpp"
+#include "pairtile.hpp"
 #include "walls.hpp"
 
 namespace sph {
@@ -649,59 +649,87 @@ __global__ __launch_bounds__(kBlock) void k_cross_integrate(
 // ---------------------------------------------------------------------------
 // Blended coupling (TWO_SCALE/Solver.cu:215-499, 732-1083, 1163-1289): every
 // neighbour term carries the neighbour's blend weight lambda_j.  Each set's
-// own sums walk its own grid in the internal x-order with the block-staged
-// stencil walk (the kernels below); the complementary sums are the fixed
+// own sums walk its own grid in the internal x-order (the kernels below); the complementary sums are the fixed
 // coupling's walks (one lane group per listed particle) with lambda weights.  Blend
 // state words: float2 (lambda, state bits).
 
-constexpr int kBlendDensityTile = 1024;
-constexpr int kBlendForceTile = 512;
+// One wave per block for the force's 14 KB tile, four for the density's.
+constexpr uint32_t kBlendDensityWaves = 4, kBlendForceWaves = 1;
+constexpr uint32_t kBlendChunkGroups = 128;  // groups in a row that one XCD takes
+
+template <uint32_t kWavesPerBlock>
+__device__ __forceinline__ GroupRange blend_group(uint32_t n) {
+    const uint32_t block = xcd_local_block(blockIdx.x, gridDim.x, kBlendChunkGroups / kWavesPerBlock);
+    return group_range<false>(block * kWavesPerBlock + uniform_u32(threadIdx.x >> 6), n, nullptr,
+                              (n + kGroupTargets - 1u) / kGroupTargets);
+}
+template <uint32_t kWavesPerBlock>
+dim3 blend_blocks(uint32_t cap) {
+    return dim3((cap + kGroupTargets * kWavesPerBlock - 1u) / (kGroupTargets * kWavesPerBlock));
+}
+
+// The walks' candidates.  Density: (x, lambda), and the blend words themselves,
+// in the internal order; force: (x, A), (v, B) and lambda, the last in place of
+// the unpacked velocities.
+__global__ __launch_bounds__(kBlock) void k_pack_blend(
+    const float2* __restrict__ tblend, const uint32_t* __restrict__ i2r,
+    const uint32_t* __restrict__ n_dev, const float4* __restrict__ ipos,
+    float2* __restrict__ iblend, float4* __restrict__ ixl) {
+    const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
+    if (s >= *n_dev) return;
+    const float2 w = tblend[i2r[s]];
+    const float4 x = ipos[s];
+    iblend[s] = w;
+    ixl[s] = make_float4(x.x, x.y, x.z, w.x);
+}
+__global__ __launch_bounds__(kBlock) void k_pack_blend_force(
+    const float2* __restrict__ aux, const float2* __restrict__ iblend,
+    const uint32_t* __restrict__ i2r, const uint32_t* __restrict__ n_dev,
+    const float4* __restrict__ ipos, float4* __restrict__ ivel, float4* __restrict__ ixa,
+    float4* __restrict__ ivb) {
+    const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
+    if (s >= *n_dev) return;
+    const float4 x = ipos[s], v = ivel[s];
+    const float2 a = aux[i2r[s]];
+    ixa[s] = make_float4(x.x, x.y, x.z, a.x);
+    ivb[s] = make_float4(v.x, v.y, v.z, a.y);
+    ivel[s] = make_float4(iblend[s].x, 0.0f, 0.0f, 0.0f);
+}
 
 // The own-set part of rho_i = m_A sum_{A, r < h_A} lambda_j W_hA + m_B
 // sum_{B, r < h0} lambda_j 1/2 (W_h0 + W_h1), and A_i, B_i from it (the
 // complementary walk adds the second sum and recomputes A_i, B_i for the
 // particles it lists).  Targets in the internal order; results at the sorted
 // slot i2r[s].
-__global__ __launch_bounds__(kBlock) void k_blend_density(
-    const float4* __restrict__ ipos_a, const float2* __restrict__ ibl_a,
+// The group walk (pairtile.hpp); one lane per target with block-staged rows took
+// 51 us for 51,200 low and 102,400 high particles side by side, this 22.
+__global__ __launch_bounds__(64 * kBlendDensityWaves) __attribute__((amdgpu_waves_per_eu(5)))
+void k_blend_density(
+    const float4* __restrict__ ixl_a, const uint32_t* __restrict__ skeys_a,
     const uint32_t* __restrict__ cs_a, const uint32_t* __restrict__ ce_a,
     const uint4* __restrict__ bins_a, const uint32_t* __restrict__ i2r_a,
     const uint32_t* __restrict__ n_a, GridView ga, StepParams pa, CrossParams c,
     float* __restrict__ rho_a, float2* __restrict__ aux_a) {
-    __shared__ float4 tile[kBlendDensityTile];
-    __shared__ uint32_t red[2 * (kBlock / 64)];
+    __shared__ __align__(kTileAlign) unsigned char lds[kBlendDensityWaves * PairTile<1>::kBytes];
     const uint32_t na = *n_a;
-    const uint32_t s = xcd_local_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
-    const bool active = s < na;
-    const float4 xi = active ? ipos_a[s] : make_float4(0.f, 0.f, 0.f, 0.f);
-    const Probe pr = make_probe(ga, xi.x, xi.y, xi.z);
+    const GroupRange gr = blend_group<kBlendDensityWaves>(na);
+    if (gr.start >= gr.end) return;
+    uint32_t s;
+    const GroupTargets t = load_targets(ga, gr, ixl_a, skeys_a, s);
+    const float4 xi = target_position(t);
     float own = 0.0f;
-    auto pair = [&](const float4& xj, float lj) {
-        const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
-        const float r2 = dx * dx + dy * dy + dz * dz;
-        if (r2 < pa.h2) {
-            const float a = pa.h2 - r2;
-            own += lj * (a * a * a);
-        }
-    };
-    walk_stencil_staged<kBlock, kBlendDensityTile, true>(
-        ga, pr, cs_a, ce_a, na, active, red,
-        [&](uint32_t k, uint32_t j) {
-            const float4 x = ipos_a[j];
-            tile[k] = make_float4(x.x, x.y, x.z, ibl_a[j].x);
+    walk_group<1>(
+        ga, t, pa.inv_h, cs_a, ce_a, bins_a, na, ixl_a, nullptr, nullptr,
+        lds_address(lds) + uniform_u32(threadIdx.x >> 6) * PairTile<1>::kBytes,
+        [&](const v4f& q) {
+            const float dx = xi.x - q.x, dy = xi.y - q.y, dz = xi.z - q.z;
+            const float r2 = dx * dx + dy * dy + dz * dz;
+            const float a = __builtin_amdgcn_fmed3f(pa.h2 - r2, 0.0f, pa.h2);
+            own += q.w * (a * a * a);
         },
-        [&](uint32_t t0, uint32_t t1, uint32_t) {
-            for (uint32_t t = t0; t < t1; ++t) {
-                const float4 q = tile[t];
-                keep_lds_quad(q);
-                pair(q, q.w);
-            }
-        },
-        [&](uint32_t b, uint32_t e) {
-            for (uint32_t j = b; j < e; ++j) pair(ipos_a[j], ibl_a[j].x);
-        },
-        bins_a);
-    if (!active) return;
+        [] {});
+    own = both_halves(own);
+    if (!t.active || (threadIdx.x & 32u) != 0u) return;
     const float r = pa.c6m * own;
     const uint32_t o = i2r_a[s];
     rho_a[o] = r;
@@ -715,74 +743,76 @@ __global__ __launch_bounds__(kBlock) void k_blend_density(
 // boundary term; then the velocity update with the cap, the position update
 // and the wall clamp, and integrateD's blend update; results at the sorted
 // slot i2r[s].
+// The group walk; block-staged rows took 85 us for 51,200 low and 102,400 high
+// particles side by side, this 38.
 template <bool kTension>
-__global__ __launch_bounds__(kBlock) void k_blend_force_integrate(
-    const float4* __restrict__ ipos_a, const float4* __restrict__ ivel_a,
+__global__ __launch_bounds__(64 * kBlendForceWaves) __attribute__((amdgpu_waves_per_eu(3)))
+void k_blend_force_integrate(
+    const float4* __restrict__ tpos_a, const float4* __restrict__ tvel_a,
     const float4* __restrict__ ixa_a, const float4* __restrict__ ivb_a,
-    const float2* __restrict__ ibl_a,
+    const float4* __restrict__ il_a, const float2* __restrict__ ibl_a,
+    const uint32_t* __restrict__ skeys_a,
     const uint32_t* __restrict__ cs_a, const uint32_t* __restrict__ ce_a,
     const uint4* __restrict__ bins_a, const uint32_t* __restrict__ i2r_a,
     const uint32_t* __restrict__ n_a, GridView ga, StepParams pa, CrossParams c,
     const float4* __restrict__ xacc_a, const float4* __restrict__ bacc, float dt, float inc,
     float4* __restrict__ pos_a, float4* __restrict__ vel_a, float2* __restrict__ nbl_a,
     float4* __restrict__ acc_out) {
-    __shared__ float4 tx[kBlendForceTile];
-    __shared__ float4 tv[kBlendForceTile];
-    __shared__ float tl[kBlendForceTile];
-    __shared__ uint32_t red[2 * (kBlock / 64)];
+    __shared__ __align__(kTileAlign) unsigned char lds[kBlendForceWaves * PairTile<3>::kBytes];
     const uint32_t na = *n_a;
-    const uint32_t s = xcd_local_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
-    const bool active = s < na;
-    const float4 xi = active ? ipos_a[s] : make_float4(0.f, 0.f, 0.f, 0.f);
-    const float4 vi = active ? ivel_a[s] : make_float4(0.f, 0.f, 0.f, 0.f);
-    const float2 ai = active ? make_float2(ixa_a[s].w, ivb_a[s].w) : make_float2(0.f, 1.f);
-    const Probe pr = make_probe(ga, xi.x, xi.y, xi.z);
+    const GroupRange gr = blend_group<kBlendForceWaves>(na);
+    if (gr.start >= gr.end) return;
+    uint32_t s;
+    const GroupTargets t = load_targets(ga, gr, ixa_a, skeys_a, s);
+    const float4 xt = target_position(t);
+    float4 vi = ivb_a[t.active ? s : gr.start];
+    const float2 ai = make_float2(t.x.w, vi.w);
     float Px = 0.f, Py = 0.f, Pz = 0.f, Vx = 0.f, Vy = 0.f, Vz = 0.f, Tx = 0.f, Ty = 0.f,
           Tz = 0.f;
-    const uint32_t h2_bits_m1 = __float_as_uint(pa.h2) - 1u;
-    // xa = (x_j, A_j), vb = (v_j, B_j); 0 < r < h_A.
-    auto pair = [&](const float4& xa, const float4& vb, float lj) {
-        const float dx = xi.x - xa.x, dy = xi.y - xa.y, dz = xi.z - xa.z;
-        const float r2 = dx * dx + dy * dy + dz * dz;
-        if (__float_as_uint(r2) - 1u >= h2_bits_m1) return;
-        const float inv_r = __builtin_amdgcn_rsqf(r2);
-        const float hr = pa.h - r2 * inv_r;
-        const float tpr = lj * (ai.x + xa.w) * hr * hr * inv_r;
-        Px += tpr * dx;
-        Py += tpr * dy;
-        Pz += tpr * dz;
-        const float tvs = lj * hr * vb.w;
-        Vx += tvs * (vb.x - vi.x);
-        Vy += tvs * (vb.y - vi.y);
-        Vz += tvs * (vb.z - vi.z);
-        if (kTension) {
-            const float a = pa.h2 - r2;
-            const float w = lj * (a * a * a);
-            Tx += w * dx;
-            Ty += w * dy;
-            Tz += w * dz;
-        }
-    };
-    walk_stencil_staged<kBlock, kBlendForceTile, true>(
-        ga, pr, cs_a, ce_a, na, active, red,
-        [&](uint32_t k, uint32_t j) {
-            tx[k] = ixa_a[j];
-            tv[k] = ivb_a[j];
-            tl[k] = ibl_a[j].x;
-        },
-        [&](uint32_t t0, uint32_t t1, uint32_t) {
-            for (uint32_t t = t0; t < t1; ++t) {
-                const float4 q = tx[t];
-                keep_lds_quad(q);
-                pair(q, tv[t], tl[t]);
+    // xa = (x_j, A_j), vb = (v_j, B_j), wl = (lambda_j, ..).  Out of range and at
+    // r = 0 (h - r) clamps to 0, with 1 / r held finite, so such a pair adds 0.
+    walk_group<3>(
+        ga, t, pa.inv_h, cs_a, ce_a, bins_a, na, ixa_a, ivb_a, il_a,
+        lds_address(lds) + uniform_u32(threadIdx.x >> 6) * PairTile<3>::kBytes,
+        [&](const v4f& xa, const v4f& vb, const v4f& wl) {
+            const float lj = wl.x;
+            const float dx = xt.x - xa.x, dy = xt.y - xa.y, dz = xt.z - xa.z;
+            const float r2 = dx * dx + dy * dy + dz * dz;
+            const float rs = __builtin_amdgcn_rsqf(r2);
+            const float hr = __builtin_amdgcn_fmed3f(pa.h - r2 * rs, 0.0f, pa.h);
+            const float inv_r = __builtin_amdgcn_fmed3f(rs, 0.0f, 2e19f);
+            const float tpr = lj * (ai.x + xa.w) * hr * hr * inv_r;
+            Px += tpr * dx;
+            Py += tpr * dy;
+            Pz += tpr * dz;
+            const float tvs = lj * hr * vb.w;
+            Vx += tvs * (vb.x - vi.x);
+            Vy += tvs * (vb.y - vi.y);
+            Vz += tvs * (vb.z - vi.z);
+            if (kTension) {
+                const float a = __builtin_amdgcn_fmed3f(pa.h2 - r2, 0.0f, pa.h2);
+                const float w = lj * (a * a * a);
+                Tx += w * dx;
+                Ty += w * dy;
+                Tz += w * dz;
             }
         },
-        [&](uint32_t b, uint32_t e) {
-            for (uint32_t j = b; j < e; ++j) pair(ixa_a[j], ivb_a[j], ibl_a[j].x);
-        },
-        bins_a);
-    if (!active) return;
+        [] {});
+    Px = both_halves(Px);
+    Py = both_halves(Py);
+    Pz = both_halves(Pz);
+    Vx = both_halves(Vx);
+    Vy = both_halves(Vy);
+    Vz = both_halves(Vz);
+    if (kTension) {
+        Tx = both_halves(Tx);
+        Ty = both_halves(Ty);
+        Tz = both_halves(Tz);
+    }
+    if (!t.active || (threadIdx.x & 32u) != 0u) return;
     const uint32_t o = i2r_a[s];  // the target's sorted slot
+    const float4 xi = make_float4(t.x.x, t.x.y, t.x.z, tpos_a[o].w);  // with the id
+    vi.w = tvel_a[o].w;                                               // and the tag
     const float vc = pa.visc * ai.y;
     float ax = pa.c45m * Px + vc * Vx + pa.gx;
     float ay = pa.c45m * Py + vc * Vy + pa.gy;
@@ -1566,8 +1596,8 @@ int launch_blended_passes(sph_two_scale* t, const StepParams* P, const GridView*
         TwoScaleSet& B = t->set[1 - r];
         const hipStream_t s = sst[r];
         const CrossParams c = cross_params(t, r);
-        hipLaunchKernelGGL(k_blend_density, blocks_for(A.cap), dim3(kBlock), 0, s, A.buf.ipos,
-                           A.iblend, A.buf.cell_start, A.buf.cell_end, A.buf.xbins, A.buf.i2r,
+        hipLaunchKernelGGL(k_blend_density, blend_blocks<kBlendDensityWaves>(A.cap),
+                           dim3(64 * kBlendDensityWaves), 0, s, A.buf.ixa, A.buf.skeys, A.buf.cell_start, A.buf.cell_end, A.buf.xbins, A.buf.i2r,
                            A.buf.n_dev, G[r], P[r], c, A.buf.rho, A.buf.aux);
         hipLaunchKernelGGL(k_cross_list, blocks_for(A.cap), dim3(kBlock), 0, s, A.buf.tpos,
                            A.buf.n_dev, B.buf.n_dev, nearby(t, r), X[0], c, A.buf.rho, A.buf.aux,
@@ -1601,20 +1631,17 @@ int launch_blended_passes(sph_two_scale* t, const StepParams* P, const GridView*
         c.vmax = velocity_limit(t, r, dt);
         float4* acc = accel_out ? A.buf.accel : nullptr;
         const float inc = t->opt.blend_increment;
-        rc = launch_gather_aux(P[r], A.buf, s);  // the final A, B in the internal order
-        if (rc != SPH_OK) return rc;
-        if (P[r].tens != 0.0f)
-            hipLaunchKernelGGL(k_blend_force_integrate<true>, blocks_for(A.cap), dim3(kBlock), 0,
-                               s, A.buf.ipos, A.buf.ivel, A.buf.ixa, A.buf.ivb, A.iblend,
-                               A.buf.cell_start, A.buf.cell_end, A.buf.xbins, A.buf.i2r, A.buf.n_dev, G[r], P[r], c,
-                               A.accel, wall_acc(t, r), dt, inc, A.buf.pos, A.buf.vel, A.nblend,
-                               acc);
-        else
-            hipLaunchKernelGGL(k_blend_force_integrate<false>, blocks_for(A.cap), dim3(kBlock), 0,
-                               s, A.buf.ipos, A.buf.ivel, A.buf.ixa, A.buf.ivb, A.iblend,
-                               A.buf.cell_start, A.buf.cell_end, A.buf.xbins, A.buf.i2r, A.buf.n_dev, G[r], P[r], c,
-                               A.accel, wall_acc(t, r), dt, inc, A.buf.pos, A.buf.vel, A.nblend,
-                               acc);
+        // The final A, B in the internal order.
+        hipLaunchKernelGGL(k_pack_blend_force, blocks_for(A.cap), dim3(kBlock), 0, s, A.buf.aux,
+                           A.iblend, A.buf.i2r, A.buf.n_dev, A.buf.ipos, A.buf.ivel, A.buf.ixa,
+                           A.buf.ivb);
+        hipLaunchKernelGGL((P[r].tens != 0.0f ? k_blend_force_integrate<true>
+                                              : k_blend_force_integrate<false>),
+                           blend_blocks<kBlendForceWaves>(A.cap), dim3(64 * kBlendForceWaves), 0, s,
+                           A.buf.tpos, A.buf.tvel, A.buf.ixa, A.buf.ivb, A.buf.ivel, A.iblend,
+                           A.buf.skeys, A.buf.cell_start, A.buf.cell_end, A.buf.xbins, A.buf.i2r,
+                           A.buf.n_dev, G[r], P[r], c, A.accel, wall_acc(t, r), dt, inc, A.buf.pos,
+                           A.buf.vel, A.nblend, acc);
     }
     SPH_HIP(hipGetLastError());
     rc = wait_for(t, 5, sl, st);  // join
@@ -1670,8 +1697,8 @@ int launch_two_scale_step(sph_two_scale* t, float dt, bool accel_out) {
         if (blended(t)) {
             hipLaunchKernelGGL(k_gather_blend, blocks_for(S.cap), dim3(kBlock), 0, s, S.buf.perm,
                                S.buf.n_dev, S.state_blend, S.tblend);
-            rc = launch_gather_x(S.tblend, S.buf.i2r, S.buf.n_dev, S.cap, S.iblend, s);
-            if (rc != SPH_OK) return rc;
+            hipLaunchKernelGGL(k_pack_blend, blocks_for(S.cap), dim3(kBlock), 0, s, S.tblend,
+                               S.buf.i2r, S.buf.n_dev, S.buf.ipos, S.iblend, S.buf.ixa);
         }
         uint32_t* occ = (r == 1) ? t->occ : t->occ + C0;
         hipLaunchKernelGGL(k_mark_occupancy, blocks_for(S.cap), dim3(kBlock), 0, s, S.buf.tpos,
