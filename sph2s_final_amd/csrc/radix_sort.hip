@@ -116,7 +116,9 @@ __global__ __launch_bounds__(kBlock) void k_prepare(uint32_t* __restrict__ zero,
 struct ArrayKeys {
     static constexpr int kHistItems = 8;
     const uint32_t* keys;
-    __device__ uint32_t operator()(uint32_t i) const { return keys[i]; }
+    typedef uint32_t Item;
+    __device__ Item load(uint32_t i) const { return keys[i]; }
+    __device__ uint32_t key(const Item& k, uint32_t) const { return k; }
 };
 
 // Keys computed as cell hashes of float4 positions (computeHashs,
@@ -130,8 +132,9 @@ struct HashKeys {
     uint32_t* keys_out;
     float ox, oy, oz, spacing;
     int dx, dy, dz;
-    __device__ uint32_t operator()(uint32_t i) const {
-        const float4 x = pos[i];
+    typedef float4 Item;
+    __device__ Item load(uint32_t i) const { return pos[i]; }
+    __device__ uint32_t key(const Item& x, uint32_t i) const {
         const uint32_t k = cell_hash(x.x, x.y, x.z, ox, oy, oz, spacing, dx, dy, dz);
         keys_out[i] = k;
         return k;
@@ -141,21 +144,35 @@ struct HashKeys {
 // Batched scenes: the scene id is in vel.w; the key is the scene's first global
 // cell plus the reference hash of the position in the scene's own grid, so a
 // stable sort keeps every scene contiguous and in its own hash order.
-// (kHistItems 8: with 4 the 4.1M-key batch of 64 scenes ran its step 1%
-// slower.)
+// kItems keys per thread: up to 2^21 keys 4 (one million in 24 scenes 12.0 us
+// against 13.6 with 8), beyond 8 (4.1 million in 64: a step of 1100 us against
+// 1130; the blocks' additions to the global histograms then weigh more).
+constexpr uint32_t kBatchHistFew = 1u << 21;
+template <int kItems>
 struct BatchHashKeys {
-    static constexpr int kHistItems = 8;
+    static constexpr int kHistItems = kItems;
     const float4* pos;
     const float4* vel;
     const SceneParams* scenes;
     uint32_t* keys_out;
-    __device__ uint32_t operator()(uint32_t i) const {
-        const float4 x = pos[i];
-        const GridView& g = scenes[__float_as_uint(vel[i].w)].g;
-        const uint32_t k =
-            g.cell_offset + cell_hash(x.x, x.y, x.z, g.ox, g.oy, g.oz, g.spacing, g.dx, g.dy, g.dz);
+    struct Item {
+        float4 x;
+        uint32_t scene;
+    };
+    __device__ Item load(uint32_t i) const { return Item{pos[i], __float_as_uint(vel[i].w)}; }
+    // A wave's slots nearly always belong to one scene, whose grid then comes
+    // through the scalar cache (65k particles 5.8 us, a load a lane and field
+    // and 8 keys per thread before: 9.7).
+    __device__ uint32_t key(const Item& p, uint32_t i) const {
+        const uint32_t first = uniform_u32(p.scene);
+        const uint32_t k = __ballot(p.scene != first) == 0ull ? hash(p.x, scenes[first].g)
+                                                              : hash(p.x, scenes[p.scene].g);
         keys_out[i] = k;
         return k;
+    }
+    __device__ static uint32_t hash(const float4& x, const GridView& g) {
+        return g.cell_offset +
+               cell_hash(x.x, x.y, x.z, g.ox, g.oy, g.oz, g.spacing, g.dx, g.dy, g.dz);
     }
 };
 
@@ -176,11 +193,14 @@ __global__ __launch_bounds__(kBlock) void k_hist(Src src, const uint32_t* __rest
     for (int i = threadIdx.x; i < kMaxPasses * kRadix; i += kBlock) (&cnt[0][0])[i] = 0u;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const uint32_t base = blockIdx.x * kHistTile + wave * (64 * kHistItems);
+    typename Src::Item item[kHistItems];
     uint32_t key[kHistItems];
+#pragma unroll
+    for (int r = 0; r < kHistItems; ++r) item[r] = src.load(min(base + r * 64 + lane, n - 1u));
 #pragma unroll
     for (int r = 0; r < kHistItems; ++r) {
         const uint32_t idx = base + r * 64 + lane;
-        key[r] = (idx < n) ? src(idx) : 0u;
+        key[r] = (idx < n) ? src.key(item[r], idx) : 0u;
     }
     __syncthreads();
 #pragma unroll
@@ -668,8 +688,10 @@ int hash_hist_cells_batched(const StepParams& cap, const uint32_t* n_dev, const 
                             uint32_t* cell_start, uint32_t* cell_end, hipStream_t stream) {
     if (!temp || temp_bytes < radix_sort_temp_bytes(cap.n))
         return set_error(SPH_ERR_INVALID_ARGUMENT, "hash: sort temp buffer too small");
-    BatchHashKeys src{pos, vel, scenes, keys};
-    return prepare_hist(src, cap.n, n_dev, cap.n, key_bits, temp, cell_start, cell_end,
+    if (cap.n > kBatchHistFew)
+        return prepare_hist(BatchHashKeys<8>{pos, vel, scenes, keys}, cap.n, n_dev, cap.n, key_bits,
+                            temp, cell_start, cell_end, cap.num_cells, stream);
+    return prepare_hist(BatchHashKeys<4>{pos, vel, scenes, keys}, cap.n, n_dev, cap.n, key_bits, temp, cell_start, cell_end,
                         cap.num_cells, stream);
 }
 

@@ -75,3 +75,26 @@ def test_sorts_of_few_pairs(n, bits):
     order = np.argsort(keys, kind="stable")
     assert np.array_equal(out[0].cpu().numpy().view(np.uint32), keys[order])
     assert np.array_equal(out[1].cpu().numpy().view(np.uint32), vals[order])
+
+
+def test_batched_hash_across_scene_borders():
+    # Waves of the histogram pass that span scenes: 700 scenes of 1 to 40
+    # particles and one too large for the block sort, against each scene's own
+    # hashes and ranges.
+    from sph2s_final_amd import BatchSolver
+    rng = np.random.default_rng(6)
+    base = scenes.dam_break((8, 8, 8), seed=1).config
+    counts = list(rng.integers(1, 41, 700)) + [10300]
+    states = [rng.uniform(0.0, 0.22, size=(int(n), 3)).astype(np.float32) for n in counts]
+    print(f"case batched hash of {sum(counts)}", flush=True)
+    with BatchSolver([base] * len(counts), states) as b:
+        b.Advance(scenes.DT)
+        b.synchronize()
+        assert b.device_errors() == 0
+        got = b.download(FIELD_SORTED_HASH)
+        cells = b.cell_offsets
+        parts = b.part_offsets
+    p = O.params_from_config(base)
+    for s in list(range(0, 700, 7)) + [700]:
+        keys = np.sort(O.hash_positions(p, states[s]), kind="stable")
+        assert np.array_equal(got[parts[s]:parts[s + 1]] - np.uint32(cells[s]), keys)
