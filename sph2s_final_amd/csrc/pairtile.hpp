@@ -311,19 +311,6 @@ __device__ __forceinline__ void walk_group(const GridView& g, const GroupTargets
                                            G&& every8) {
     typedef PairTile<kArrays> T;
     const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t half = lane >> 5;
-    // A lane half converts 32 of 64 candidates; the first product takes the lower
-    // half's (the upper half's target operand is 0), the second the upper's.
-    // Row m of a product reads slot 2 r + q of its 32, where (q, r) are the lane
-    // half and accumulator that receive row m: a lane's 32 mask bits are the even
-    // (half 0) or odd slots of 64, so a target's hits, which lie together along a
-    // row, fall evenly on its two lanes.  The rows of slots 60 to 63 read others;
-    // their bits are dropped.
-    const uint32_t m = lane & 31u;
-    const uint32_t slot_of_row = 2u * (4u * (m >> 3) + (m & 3u)) + ((m >> 2) & 1u) + 32u * half;
-    const uint32_t row_slot =
-        tile + T::kSlots + 16u * (slot_of_row < kWordSlots ? slot_of_row : slot_of_row - 4u);
-    const uint32_t mask0 = tile + 4u * lane;
     // The slots nobody is near.
     if (lane < 4u * kRing) {
         const uint32_t at = tile + T::kSlots + 1024u * (lane >> 2) + 16u * (kWordSlots + (lane & 3u));
@@ -362,6 +349,24 @@ __device__ __forceinline__ void walk_group(const GridView& g, const GroupTargets
             if (lane == 0u)
                 lds_write<v2u>(tile + T::kRows + 8u * static_cast<uint32_t>(__builtin_popcountll(live)),
                                v2u{0xFFFFFFFFu, 0u});
+            // From here on, not held through the look-up of the rows: with them the
+            // density pass spilled four registers a group (24 scenes of 4096..98304:
+            // force 90 us, now 88.5; a million at rest 113, now 109).
+            uint32_t place_in_wave = lane;
+            asm volatile("" : "+v"(place_in_wave));
+            const uint32_t half = place_in_wave >> 5;
+            // A lane half converts 32 of 64 candidates; the first product takes the lower
+            // half's (the upper half's target operand is 0), the second the upper's.
+            // Row m of a product reads slot 2 r + q of its 32, where (q, r) are the lane
+            // half and accumulator that receive row m: a lane's 32 mask bits are the even
+            // (half 0) or odd slots of 64, so a target's hits, which lie together along a
+            // row, fall evenly on its two lanes.  The rows of slots 60 to 63 read others;
+            // their bits are dropped.
+            const uint32_t m = place_in_wave & 31u;
+            const uint32_t slot_of_row = 2u * (4u * (m >> 3) + (m & 3u)) + ((m >> 2) & 1u) + 32u * half;
+            const uint32_t row_slot =
+                tile + T::kSlots + 16u * (slot_of_row < kWordSlots ? slot_of_row : slot_of_row - 4u);
+            const uint32_t mask0 = tile + 4u * place_in_wave;
             // Target operands of the filter, in units of h: columns
             // (-2 x, -2 y, -2 z, 1, c, c') against rows (x, y, z, |x|^2, 1, 1), with
             // c + c' = |x|^2 - 1 - margin.
