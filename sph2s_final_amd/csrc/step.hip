@@ -564,7 +564,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
 // largest velocity difference, over the RMS velocity, of the same sums in the
 // group walk's order 3e-4 to 1.6e-3, by the initial jitter), so scenes with
 // walls keep this order of additions and with it their trajectories.  The group
-// walk would take the four steps from 826 to 739 us.
+// walk would take the four steps from 826 to 739 us.  (The XSPH and two-scale
+// forms, which integrate in a later kernel, take the group walk with walls too.)
 constexpr int kRowDensityTile = 1280, kRowForceTile = 640, kRowList = 16, kRowScan = 8;
 
 __device__ __forceinline__ v4f as_v4f(const float4& q) { return v4f{q.x, q.y, q.z, q.w}; }
