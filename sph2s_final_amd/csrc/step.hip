@@ -47,10 +47,10 @@ constexpr int kBlock = 256;
 // at 4096 particles / one million 4.6 + 5.8 / 4.8 + 23, now 4.5 / 19.
 constexpr int kXorderTile = 2048;
 
-// Bits that order as unsigned like the floats do (-0 as 0; NaNs beyond the
-// infinities), and back.
+// Bits that order as unsigned like the floats do (-0 as 0; NaNs of either sign
+// beyond the infinities), and back.
 __device__ __forceinline__ uint32_t ordered_bits(float x) {
-    const uint32_t u = __float_as_uint(x + 0.0f);
+    const uint32_t u = x == x ? __float_as_uint(x + 0.0f) : 0x7FC00000u;
     return u ^ (static_cast<uint32_t>(static_cast<int32_t>(u) >> 31) | 0x80000000u);
 }
 __device__ __forceinline__ float from_ordered(uint32_t u) {
@@ -231,9 +231,14 @@ __global__ __launch_bounds__(kBlock) void k_order(const uint32_t* __restrict__ s
         inv = g.inv_spacing;
         dx = g.dx;
     }
+    // A NaN x, last in its cell (which is the row's first), is in the last bin.
     const float cx = static_cast<float>(cell_coord(xs.x, ox, spacing, dx));
-    const int kq = xbin_of((xs.x - ox) * inv - cx);
-    const int kn = (rank + 1 < cnt) ? max(kq, xbin_of((xg - ox) * inv - cx)) : kXBins;
+    auto bin = [&](float x) {
+        const float f = (x - ox) * inv - cx;
+        return f < 1.0f ? xbin_of(f) : kXBins - 1;
+    };
+    const int kq = bin(xs.x);
+    const int kn = (rank + 1 < cnt) ? max(kq, bin(xg)) : kXBins;
     if (rank == 0)
         for (int k = 0; k < kq; ++k) t[k] = 0u;
     const uint8_t c = static_cast<uint8_t>(rank + 1);
