@@ -187,7 +187,7 @@ __device__ __forceinline__ GroupTargets adjoint_targets(const GridView& g, const
 
 // Force-pair adjoint; see the file comment for the terms.  The group walk
 // (pairtile.hpp) with (x, A), (v, B) and abar per candidate; a pair out of range
-// or coincident adds 0.  Writes (x, dL/drho) packed for the density adjoint, and
+// or coincident adds 0 (walk_targets sees to what is not finite).  Writes (x, dL/drho) packed for the density adjoint, and
 // adds each group's parameter terms, in FP64, to the group's own accumulators.
 // Bound by VALU issue.  Against a queue of hits per lane on a block-staged tile
 // (us, one million in 16 scenes): 233 -> 197.
@@ -220,7 +220,7 @@ void k_adj_force(
     float gPx = 0.f, gPy = 0.f, gPz = 0.f;   // sum (A_i + A_j)[F dA + F'/r (x.dA) x]
     float gVx = 0.f, gVy = 0.f, gVz = 0.f;   // sum B_j (dv.dA) x / r
     float gWx = 0.f, gWy = 0.f, gWz = 0.f;   // sum (h - r) B_j dA
-    walk_group<3>(
+    walk_targets<3, false>(
         g, t, p.inv_h, cs, ce, bins, n, ixa, ivb, abar,
         lds_address(lds) + wave * AdjForceTile::kBytes,
         [&](const v4f& xa, const v4f& vb, const v4f& bj) {
@@ -252,7 +252,15 @@ void k_adj_force(
             gWy += wB * ay;
             gWz += wB * az;
         },
-        [] {});
+        [] {},
+        [&] {
+            return __builtin_isfinite(((sumA + S1) + (Sd + gPx)) + ((gPy + gPz) + (gVx + gVy)) +
+                                      ((gVz + gWx) + (gWy + gWz)));
+        },
+        [&] {
+            sumA = S1 = Sd = 0.f;
+            gPx = gPy = gPz = gVx = gVy = gVz = gWx = gWy = gWz = 0.f;
+        });
     sumA = both_halves(sumA);
     S1 = both_halves(S1);
     Sd = both_halves(Sd);
@@ -319,7 +327,7 @@ void k_adj_density(
     // (one clamped fused multiply-add): the pair's (h^2 - r^2)^2 is h^4 a^2,
     // and a = 0 out of range.  A coincident pair (x_ij = 0) adds zero.
     float sx = 0.f, sy = 0.f, sz = 0.f;
-    walk_group<1>(
+    walk_targets<1, false>(
         g, t, p.inv_h, cs, ce, bins, n, xg, nullptr, nullptr,
         lds_address(lds) + wave * AdjDensityTile::kBytes,
         [&](const v4f& q) {
@@ -331,7 +339,7 @@ void k_adj_density(
             sy += c * dy;
             sz += c * dz;
         },
-        [] {});
+        [] {}, [&] { return __builtin_isfinite(sx + sy + sz); }, [&] { sx = sy = sz = 0.f; });
     sx = both_halves(sx);
     sy = both_halves(sy);
     sz = both_halves(sz);

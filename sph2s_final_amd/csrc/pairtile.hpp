@@ -528,4 +528,63 @@ __device__ __forceinline__ void walk_group(const GridView& g, const GroupTargets
     }
 }
 
+// The candidates of the targets in `todo` (a mask of 32) by a direct scan: each
+// lane walks every other row of its target's own stencil and evaluates the
+// candidates in range alone, r = 0 only with kSelf.
+template <uint32_t kArrays, bool kSelf, class F, class G>
+__device__ __forceinline__ void walk_direct(const GridView& g, const GroupTargets& t, uint32_t todo,
+                                            const uint32_t* __restrict__ cs,
+                                            const uint32_t* __restrict__ ce, uint32_t n,
+                                            const float4* __restrict__ a0,
+                                            const float4* __restrict__ a1,
+                                            const float4* __restrict__ a2, F&& pair, G&& every8) {
+    if (((todo >> (threadIdx.x & 31u)) & 1u) == 0u) return;
+    const Probe pr = make_probe(g, t.x.x, t.x.y, t.x.z);
+    const float h2 = g.h * g.h;
+    uint32_t turn = 0u;
+    int ry = pr.sy + ((threadIdx.x & 32u) != 0u ? 1 : 0), rz = pr.sz;
+    for (;; ry += 2) {
+        for (; ry > pr.ey; ry -= pr.ey - pr.sy + 1) ++rz;
+        if (rz > pr.ez) break;
+        uint32_t b, e;
+        probe_row_run(g, pr, cs, ce, n, ry, rz, b, e);
+        for (uint32_t j = b; j < e; ++j) {
+            const v4f q = *reinterpret_cast<const v4f*>(a0 + j);
+            const float dx = t.x.x - q.x, dy = t.x.y - q.y, dz = t.x.z - q.z;
+            const float r2 = dx * dx + dy * dy + dz * dz;
+            if (!(r2 < h2) || !(kSelf || r2 > 0.0f)) continue;  // a NaN too
+            if constexpr (kArrays == 1)
+                pair(q);
+            else if constexpr (kArrays == 2)
+                pair(q, *reinterpret_cast<const v4f*>(a1 + j));
+            else
+                pair(q, *reinterpret_cast<const v4f*>(a1 + j), *reinterpret_cast<const v4f*>(a2 + j));
+            if ((++turn & 7u) == 0u) every8();
+        }
+    }
+    every8();
+}
+
+// The sums of a group's targets: walk_group, which multiplies what a candidate
+// out of range carries (v, A, B, ..) by 0.  That is no 0 if it is infinite or a
+// NaN, so a target whose sums are not finite is taken again by a direct scan,
+// which leaves such candidates out: then they are those of its neighbours.
+// finite(): whether this lane's sums are; reset(): makes them 0.
+template <uint32_t kArrays, bool kSelf, class F, class G, class Ok, class Reset>
+__device__ __forceinline__ void walk_targets(const GridView& g, const GroupTargets& t, float inv_h,
+                                             const uint32_t* __restrict__ cs,
+                                             const uint32_t* __restrict__ ce,
+                                             const uint4* __restrict__ bins, uint32_t n,
+                                             const float4* __restrict__ a0,
+                                             const float4* __restrict__ a1,
+                                             const float4* __restrict__ a2, uint32_t tile,
+                                             F&& pair, G&& every8, Ok&& finite, Reset&& reset) {
+    walk_group<kArrays>(g, t, inv_h, cs, ce, bins, n, a0, a1, a2, tile, pair, every8);
+    const uint64_t bad = __ballot(t.active && !finite());
+    if (bad == 0ull) return;
+    const uint32_t todo = static_cast<uint32_t>(bad) | static_cast<uint32_t>(bad >> 32);
+    if ((todo >> (threadIdx.x & 31u)) & 1u) reset();
+    walk_direct<kArrays, kSelf>(g, t, todo, cs, ce, n, a0, a1, a2, pair, every8);
+}
+
 }  // namespace sph

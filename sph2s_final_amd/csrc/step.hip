@@ -414,7 +414,8 @@ struct PairSums {
 
     // xa = (x_j, A_j), vb = (v_j, B_j), x_j finite.  Branch-free: out of range
     // (h - r) clamps to 0, and at r = 0 it is 0 too (0 * inf is a NaN, which
-    // the clamp takes to 0), with 1 / r held finite, so such a pair adds 0.
+    // the clamp takes to 0), with 1 / r held finite, so such a pair adds 0 if
+    // v, A and B are finite (walk_targets sees to the others).
     __device__ __forceinline__ void add(const float4& xi, const float4& vi, float ai, float h,
                                         float h2, const v4f& xa, const v4f& vb) {
 #pragma clang fp contract(off)
@@ -438,6 +439,10 @@ struct PairSums {
             Ty = __builtin_fmaf(w, dy, Ty);
             Tz = __builtin_fmaf(w, dz, Tz);
         }
+    }
+
+    __device__ __forceinline__ bool finite() const {
+        return __builtin_isfinite(((Px + Py) + (Pz + Vx)) + ((Vy + Vz) + ((Tx + Ty) + Tz)));
     }
 };
 
@@ -534,9 +539,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
             const float4 xi = target_position(t);
             const float4 vi = ivb[t.active ? s : gr.start];
             PairSums<kTension> S;
-            walk_group<2>(
+            walk_targets<2, false>(
                 g, t, p.inv_h, cs, ce, xo.bins, n, ixa, ivb, nullptr, tile,
-                [&](const v4f& x, const v4f& v) { S.add(xi, vi, t.x.w, p.h, p.h2, x, v); }, [] {});
+                [&](const v4f& x, const v4f& v) { S.add(xi, vi, t.x.w, p.h, p.h2, x, v); }, [] {},
+                [&] { return S.finite(); }, [&] { S = PairSums<kTension>{}; });
             S.Px = both_halves(S.Px);
             S.Py = both_halves(S.Py);
             S.Pz = both_halves(S.Pz);

@@ -718,7 +718,7 @@ void k_blend_density(
     const GroupTargets t = load_targets(ga, gr, ixl_a, skeys_a, s);
     const float4 xi = target_position(t);
     float own = 0.0f;
-    walk_group<1>(
+    walk_targets<1, true>(
         ga, t, pa.inv_h, cs_a, ce_a, bins_a, na, ixl_a, nullptr, nullptr,
         lds_address(lds) + uniform_u32(threadIdx.x >> 6) * PairTile<1>::kBytes,
         [&](const v4f& q) {
@@ -727,7 +727,7 @@ void k_blend_density(
             const float a = __builtin_amdgcn_fmed3f(pa.h2 - r2, 0.0f, pa.h2);
             own += q.w * (a * a * a);
         },
-        [] {});
+        [] {}, [&] { return __builtin_isfinite(own); }, [&] { own = 0.0f; });
     own = both_halves(own);
     if (!t.active || (threadIdx.x & 32u) != 0u) return;
     const float r = pa.c6m * own;
@@ -770,8 +770,9 @@ void k_blend_force_integrate(
     float Px = 0.f, Py = 0.f, Pz = 0.f, Vx = 0.f, Vy = 0.f, Vz = 0.f, Tx = 0.f, Ty = 0.f,
           Tz = 0.f;
     // xa = (x_j, A_j), vb = (v_j, B_j), wl = (lambda_j, ..).  Out of range and at
-    // r = 0 (h - r) clamps to 0, with 1 / r held finite, so such a pair adds 0.
-    walk_group<3>(
+    // r = 0 (h - r) clamps to 0, with 1 / r held finite, so such a pair adds 0
+    // (walk_targets sees to what is not finite).
+    walk_targets<3, false>(
         ga, t, pa.inv_h, cs_a, ce_a, bins_a, na, ixa_a, ivb_a, il_a,
         lds_address(lds) + uniform_u32(threadIdx.x >> 6) * PairTile<3>::kBytes,
         [&](const v4f& xa, const v4f& vb, const v4f& wl) {
@@ -797,7 +798,11 @@ void k_blend_force_integrate(
                 Tz += w * dz;
             }
         },
-        [] {});
+        [] {},
+        [&] {
+            return __builtin_isfinite(((Px + Py) + (Pz + Vx)) + ((Vy + Vz) + ((Tx + Ty) + Tz)));
+        },
+        [&] { Px = Py = Pz = Vx = Vy = Vz = Tx = Ty = Tz = 0.f; });
     Px = both_halves(Px);
     Py = both_halves(Py);
     Pz = both_halves(Pz);

@@ -6,9 +6,11 @@ acceleration 1e-5 of max |a|.
 """
 import numpy as np
 import pytest
+import torch
 
 import oracle as O
-from sph2s_final_amd import FIELD_ACCEL, SPH_DEBUG_ACCEL, ParticleData, Solver, scenes
+from sph2s_final_amd import (FIELD_ACCEL, FIELD_DENSITY, FIELD_SORTED_INDEX, SPH2_COUPLING_BLENDED,
+                             SPH_DEBUG_ACCEL, ParticleData, Solver, TwoScaleSolver, scenes)
 
 pytestmark = pytest.mark.gpu
 
@@ -56,3 +58,123 @@ def test_positions_that_are_not_finite(bad):
     print(f"case positions {bad}", flush=True)
     rho, acc, _ = _gpu_step(_config(), pos, vel)
     _assert_close(rho[:n], acc[:n], *_oracle_step(_config(), pos[:n], vel[:n]))
+
+
+def _beyond(pos, bad, reach=1.0):
+    """Particles farther than reach * h from every one of `bad` (indices)."""
+    d2 = ((pos[:, None, :].astype(np.float64) - pos[None, bad, :]) ** 2).sum(2).min(1)
+    return d2 > (reach * H) ** 2
+
+
+def _state_with(value, n, seed):
+    """Random particles, four of them with that velocity, and a lone fifth."""
+    rng = np.random.default_rng(seed)
+    pos = rng.uniform(0.1 * H, 3.9 * H, size=(n, 3)).astype(np.float32)
+    vel = rng.normal(0.0, 0.2, size=(n, 3)).astype(np.float32)
+    bad = np.r_[rng.choice(n - 1, 4, replace=False), n - 1]
+    pos[n - 1] = 5.5 * H
+    wild = vel.copy()
+    wild[bad, rng.integers(0, 3, 5)] = value
+    return pos, vel, wild, bad
+
+
+VALUES = [np.inf, -np.inf, np.nan]
+
+
+@pytest.mark.parametrize("value", VALUES)
+@pytest.mark.parametrize("tension", [0.0, 0.8])
+def test_velocities_that_are_not_finite(value, tension):
+    # No bar for the neighbours; the lone particle keeps gravity's acceleration.
+    cfg = _config()
+    cfg.tension = tension
+    for n, seed in ((40, 1), (700, 2), (2500, 3)):
+        pos, vel, wild, bad = _state_with(value, n, seed)
+        print(f"case velocities {value} n={n} tension={tension}", flush=True)
+        rho, acc, bits = _gpu_step(cfg, pos, wild)
+        assert bits != 0
+        want_rho, want_acc = _oracle_step(cfg, pos, vel)
+        ok = _beyond(pos, bad)
+        assert ok.sum() >= n // 4
+        assert np.max(np.abs(rho - want_rho) / want_rho) <= TOL
+        assert np.max(np.abs(acc[ok] - want_acc[ok])) <= TOL * np.max(np.abs(want_acc))
+        assert np.max(np.abs(acc[-1] - want_acc[-1])) <= TOL * np.max(np.abs(want_acc))
+
+
+@pytest.mark.parametrize("value", VALUES)
+def test_velocities_that_are_not_finite_in_a_batch(value):
+    from sph2s_final_amd import BatchSolver
+    cfg = _config()
+    states = [_state_with(value, n, n) for n in (33, 900, 65)]
+    print(f"case batch velocities {value}", flush=True)
+    with BatchSolver([cfg] * 3, [s[0] for s in states], [s[2] for s in states]) as b:
+        b.set_debug(SPH_DEBUG_ACCEL)
+        b.Advance(scenes.DT)
+        b.device_errors()
+        perm, acc = b.download(FIELD_SORTED_INDEX), b.download(FIELD_ACCEL)
+    by_id = np.empty_like(acc)
+    by_id[perm] = acc
+    at = 0
+    for pos, vel, _, bad in states:
+        got = by_id[at:at + len(pos)]
+        at += len(pos)
+        _, want = _oracle_step(cfg, pos, vel)
+        ok = _beyond(pos, bad)
+        ok[-1] = True
+        assert np.max(np.abs(got[ok] - want[ok])) <= TOL * np.max(np.abs(want))
+
+
+@pytest.mark.parametrize("value", VALUES)
+def test_blended_values_that_are_not_finite(value):
+    # Velocities, then blend weights: particles beyond the low set's h of the
+    # bad ones against the same step without them.
+    cfg = _config()
+    lo = hi = (-1.0, -1.0, -1.0)
+    for field in ("velocity", "lambda"):
+        got = []
+        for use in (False, True):
+            pos, vel, wild, bad = _state_with(value, 1200, 7)
+            with TwoScaleSolver(cfg, lo, hi, pos, wild if use and field == "velocity" else vel) as s:
+                s.set_options(coupling=SPH2_COUPLING_BLENDED, velocity_cap=0.0)
+                s.set_debug(SPH_DEBUG_ACCEL)
+                lam = np.linspace(0.3, 1.0, len(pos)).astype(np.float32)
+                if use and field == "lambda":
+                    lam[bad] = value
+                s.set_blend(0, lam)
+                print(f"case blended {field} {value if use else 'finite'}", flush=True)
+                s.Advance(scenes.DT)
+                s.device_errors()
+                perm = s.download(0, FIELD_SORTED_INDEX)
+                rho, acc = s.download(0, FIELD_DENSITY), s.download(0, FIELD_ACCEL)
+            order = np.argsort(perm)
+            got.append((rho[order], acc[order]))
+        # A density takes the weights in, and an acceleration its neighbours' densities.
+        ok = _beyond(pos, bad, 2.0 if field == "lambda" else 1.0)
+        (rho0, acc0), (rho1, acc1) = got
+        assert ok.sum() >= 200
+        assert np.max(np.abs(rho1[ok] - rho0[ok]) / rho0[ok]) <= TOL
+        assert np.max(np.abs(acc1[ok] - acc0[ok])) <= TOL * np.max(np.abs(acc0[ok]))
+
+
+@pytest.mark.parametrize("value", VALUES)
+def test_adjoint_seeds_that_are_not_finite(value):
+    # One step: a particle farther than 2 h from a bad seed keeps its gradient
+    # (the density adjoint reaches h beyond the force adjoint's h).
+    from sph2s_final_amd.autograd import Rollout
+    pos, vel, _, bad = _state_with(value, 1500, 11)
+    seed = np.random.default_rng(12).normal(size=pos.shape).astype(np.float32)
+    got = []
+    for use in (False, True):
+        if use:
+            seed[bad, 1] = value
+        print(f"case adjoint seed {value if use else 'finite'}", flush=True)
+        with Rollout([_config()], [len(pos)], scenes.DT, 1, 1) as r:
+            r.forward(torch.from_numpy(pos).cuda(), torch.from_numpy(vel).cuda())
+            gp, gv, _, _ = r.backward(torch.from_numpy(seed).cuda())
+            torch.cuda.synchronize()
+            got.append((gp.cpu().numpy(), gv.cpu().numpy()))
+    ok = _beyond(pos, bad, 2.0)
+    assert ok.sum() >= 200
+    for a, b in zip(*got):
+        assert np.max(np.abs(a[ok] - b[ok])) <= TOL * np.max(np.abs(a))
+        # The lone particle's other components see nobody.
+        assert np.array_equal(a[-1, [0, 2]], b[-1, [0, 2]])
