@@ -209,7 +209,7 @@ void k_adj_force(
     const GridView& g = scenes[gr.scene].g;
     uint32_t s;
     const GroupTargets t = adjoint_targets(g, gr, ixa, s);
-    const float4 xi = target_position(t);
+    const float4 xi = t.x;
     const uint32_t own = t.active ? s : gr.start;
     const float4 vi = ivb[own], bi = abar[own];
     const float h = p.h;
@@ -321,7 +321,7 @@ void k_adj_density(
     const GridView& g = scenes[gr.scene].g;
     uint32_t s;
     const GroupTargets t = adjoint_targets(g, gr, xg, s);
-    const float4 xi = target_position(t);
+    const float4 xi = t.x;
     const float inv_h2 = p.inv_h2;
     // Sums of a^2 (g_i + g_j) x_ij with a = 1 - r^2 / h^2 clamped to [0, 1]
     // (one clamped fused multiply-add): the pair's (h^2 - r^2)^2 is h^4 a^2,

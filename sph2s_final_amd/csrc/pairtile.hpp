@@ -286,15 +286,9 @@ __device__ __forceinline__ void row_of(const Subgroup& s, uint32_t r, int& y, in
     y = s.y0 + static_cast<int>(r - q * static_cast<uint32_t>(s.ny));
 }
 
-// A candidate whose position is not finite is replaced by a far one, and a
-// target whose position is not finite is evaluated from -kFar, so neither meets
-// anyone (it keeps its own NaN, and no pair adds one to a sum).
+// A candidate whose position is not finite is replaced by a far one, so it meets
+// no one (targets that far, or not finite, are not walked here: walk_targets).
 constexpr float kFar = 1e15f, kFar2 = 3e30f;
-
-__device__ __forceinline__ float4 target_position(const GroupTargets& t) {
-    const float q = t.x.x * t.x.x + t.x.y * t.x.y + t.x.z * t.x.z;
-    return q < kFar2 ? t.x : make_float4(-kFar, -kFar, -kFar, t.x.w);
-}
 
 // Walks the candidates of a group in the internal x-order: their arrays a0 (x, .),
 // a1 and a2 (kArrays of them).  pair(q0, ..) evaluates this lane's target with one
@@ -565,10 +559,19 @@ __device__ __forceinline__ void walk_direct(const GridView& g, const GroupTarget
     every8();
 }
 
+// Whether the filter's coordinates hold the group: from a million h on (or at a
+// NaN) their origin is off by h / 16 and more, then the words' fill is no longer
+// out of range, and beyond 2^31 h a target would miss itself.
+__device__ __forceinline__ bool filter_holds(const GroupTargets& t, float inv_h) {
+    const float far = fabsf(t.x.x) + fabsf(t.x.y) + fabsf(t.x.z);
+    return __ballot(t.active && !(far * inv_h < 0x1p20f)) == 0ull;
+}
+
 // The sums of a group's targets: walk_group, which multiplies what a candidate
 // out of range carries (v, A, B, ..) by 0.  That is no 0 if it is infinite or a
 // NaN, so a target whose sums are not finite is taken again by a direct scan,
 // which leaves such candidates out: then they are those of its neighbours.
+// Groups that the filter does not hold are scanned directly at once.
 // finite(): whether this lane's sums are; reset(): makes them 0.
 template <uint32_t kArrays, bool kSelf, class F, class G, class Ok, class Reset>
 __device__ __forceinline__ void walk_targets(const GridView& g, const GroupTargets& t, float inv_h,
@@ -579,9 +582,12 @@ __device__ __forceinline__ void walk_targets(const GridView& g, const GroupTarge
                                              const float4* __restrict__ a1,
                                              const float4* __restrict__ a2, uint32_t tile,
                                              F&& pair, G&& every8, Ok&& finite, Reset&& reset) {
-    walk_group<kArrays>(g, t, inv_h, cs, ce, bins, n, a0, a1, a2, tile, pair, every8);
-    const uint64_t bad = __ballot(t.active && !finite());
-    if (bad == 0ull) return;
+    uint64_t bad = __ballot(t.active);
+    if (filter_holds(t, inv_h)) {
+        walk_group<kArrays>(g, t, inv_h, cs, ce, bins, n, a0, a1, a2, tile, pair, every8);
+        bad = __ballot(t.active && !finite());
+        if (bad == 0ull) return;
+    }
     const uint32_t todo = static_cast<uint32_t>(bad) | static_cast<uint32_t>(bad >> 32);
     if ((todo >> (threadIdx.x & 31u)) & 1u) reset();
     walk_direct<kArrays, kSelf>(g, t, todo, cs, ce, n, a0, a1, a2, pair, every8);

@@ -370,11 +370,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(5))) void k
             const GridView& g = kBatched ? scenes[gr.scene].g : g_in;
             uint32_t s;
             const GroupTargets t = load_targets(g, gr, ipos, skeys, s);
-            const float4 xi = target_position(t);
+            const float4 xi = t.x;
             const float inv_h2 = p.inv_h2;
             double sum64 = 0.0;
             float sum32 = 0.0f;
-            walk_group<1>(
+            walk_targets<1, true>(
                 g, t, p.inv_h, cs, ce, xo.bins, n, ipos, nullptr, nullptr, tile, [&](const v4f& x) {
 #pragma clang fp contract(off)
                     const float a = poly6_unit(xi, x, inv_h2);
@@ -385,7 +385,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(5))) void k
                         sum64 += static_cast<double>(sum32);
                         sum32 = 0.0f;
                     }
-                });
+                },
+                [] { return true; }, [] {});
             const float r = p.c6m_h6 * (kKahan ? static_cast<float>(both_halves(sum64))
                                                : both_halves(sum32));
             if (t.active && (threadIdx.x & 32u) == 0u) {
@@ -536,7 +537,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
             const GridView& g = kBatched ? scenes[gr.scene].g : g_in;
             uint32_t s;
             const GroupTargets t = load_targets(g, gr, ixa, skeys, s);
-            const float4 xi = target_position(t);
+            const float4 xi = t.x;
             const float4 vi = ivb[t.active ? s : gr.start];
             PairSums<kTension> S;
             walk_targets<2, false>(

@@ -716,7 +716,7 @@ void k_blend_density(
     if (gr.start >= gr.end) return;
     uint32_t s;
     const GroupTargets t = load_targets(ga, gr, ixl_a, skeys_a, s);
-    const float4 xi = target_position(t);
+    const float4 xi = t.x;
     float own = 0.0f;
     walk_targets<1, true>(
         ga, t, pa.inv_h, cs_a, ce_a, bins_a, na, ixl_a, nullptr, nullptr,
@@ -764,7 +764,7 @@ void k_blend_force_integrate(
     if (gr.start >= gr.end) return;
     uint32_t s;
     const GroupTargets t = load_targets(ga, gr, ixa_a, skeys_a, s);
-    const float4 xt = target_position(t);
+    const float4 xt = t.x;
     float4 vi = ivb_a[t.active ? s : gr.start];
     const float2 ai = make_float2(t.x.w, vi.w);
     float Px = 0.f, Py = 0.f, Pz = 0.f, Vx = 0.f, Vy = 0.f, Vz = 0.f, Tx = 0.f, Ty = 0.f,

@@ -11,6 +11,7 @@ import torch
 import oracle as O
 from sph2s_final_amd import (FIELD_ACCEL, FIELD_DENSITY, FIELD_SORTED_INDEX, SPH2_COUPLING_BLENDED,
                              SPH_DEBUG_ACCEL, ParticleData, Solver, TwoScaleSolver, scenes)
+from sph2s_final_amd._capi import SPH_FLAG_WALL_CLAMP
 
 pytestmark = pytest.mark.gpu
 
@@ -178,3 +179,43 @@ def test_adjoint_seeds_that_are_not_finite(value):
         assert np.max(np.abs(a[ok] - b[ok])) <= TOL * np.max(np.abs(a))
         # The lone particle's other components see nobody.
         assert np.array_equal(a[-1, [0, 2]], b[-1, [0, 2]])
+
+
+@pytest.mark.parametrize("distance", [3e3, 4e4, 1e6, 1e8, 1e10, 1e14, 1e16, 1e18])
+def test_particles_far_outside(distance):
+    # Particles that left an open domain: singles, and pairs at one place, a
+    # few of them beside finite ones in the boundary cells.
+    cfg = _config()
+    cfg.flags &= ~SPH_FLAG_WALL_CLAMP
+    rng = np.random.default_rng(21)
+    n, k = 700, 40
+    pos = rng.uniform(0.1 * H, 3.9 * H, size=(n + k, 3)).astype(np.float32)
+    vel = rng.normal(0.0, 0.2, size=(n + k, 3)).astype(np.float32)
+    axis, sign = rng.integers(0, 3, k), rng.choice([-1.0, 1.0], k)
+    pos[np.arange(n, n + k), axis] = sign * distance * rng.uniform(1.0, 1.9, k)
+    pos[n + 1::4] = pos[n::4]
+    print(f"case far outside {distance}", flush=True)
+    rho, acc, bits = _gpu_step(cfg, pos, vel)
+    want_rho, want_acc = _oracle_step(cfg, pos, vel)
+    assert bits == 0
+    _assert_close(rho, acc, want_rho, want_acc)
+
+
+@pytest.mark.parametrize("distance", [1e6, 1e10, 1e16])
+def test_adjoint_of_particles_far_outside(distance):
+    # One step without a clamp: a particle nobody is near passes its seed on.
+    from sph2s_final_amd.autograd import Rollout
+    cfg = _config()
+    cfg.flags &= ~SPH_FLAG_WALL_CLAMP
+    rng = np.random.default_rng(22)
+    pos = rng.uniform(0.1 * H, 3.9 * H, size=(300, 3)).astype(np.float32)
+    pos[-9:, 0] = distance * np.linspace(1.0, 1.9, 9)
+    seed = rng.normal(size=pos.shape).astype(np.float32)
+    print(f"case adjoint far outside {distance}", flush=True)
+    with Rollout([cfg], [len(pos)], scenes.DT, 1, 1) as r:
+        r.forward(torch.from_numpy(pos).cuda(), torch.zeros(pos.shape).cuda())
+        gp, gv, gk, gm = r.backward(torch.from_numpy(seed).cuda())
+        torch.cuda.synchronize()
+    assert np.isfinite(gp.cpu().numpy()).all() and np.isfinite(gk).all() and np.isfinite(gm).all()
+    assert np.array_equal(gp.cpu().numpy()[-9:], seed[-9:])
+    assert np.max(np.abs(gv.cpu().numpy()[-9:] - scenes.DT * seed[-9:])) <= TOL * scenes.DT * 4.0
