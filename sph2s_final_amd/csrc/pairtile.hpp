@@ -522,9 +522,52 @@ __device__ __forceinline__ void walk_group(const GridView& g, const GroupTargets
     }
 }
 
+// Candidate runs [b, e) of kRows rows (ry, rz) of a target's stencil (empty rows
+// and rows outside it: b >= e), the cells as in probe_row_run.  The loads of all
+// rows go out together.
+template <int kRows>
+__device__ __forceinline__ void direct_rows(const GridView& g, const Probe& pr, uint32_t own,
+                                            const uint32_t* __restrict__ cs,
+                                            const uint32_t* __restrict__ ce, uint32_t n,
+                                            const int* ry, const int* rz, uint32_t* b, uint32_t* e) {
+    uint32_t first[kRows], more[kRows], start[kRows][3];
+    int end[kRows][3];
+#pragma unroll
+    for (int u = 0; u < kRows; ++u) {
+        const float gy = slab_gap(pr.fy, ry[u], g.spacing), gz = slab_gap(pr.fz, rz[u], g.spacing);
+        const float w2 = g.prune_h2 - (gy * gy + gz * gz);
+        const float w = __builtin_amdgcn_sqrtf(fmaxf(w2, 0.0f));
+        const int lo = max(pr.sx, static_cast<int>(floorf((pr.fx - w) * g.inv_spacing)));
+        const int hi = min(pr.ex, static_cast<int>(floorf((pr.fx + w) * g.inv_spacing)));
+        const bool some = w2 > 0.0f && ry[u] <= pr.ey && rz[u] <= pr.ez && lo <= hi;
+        first[u] = some ? g.cell_offset + static_cast<uint32_t>(g.dx) * (ry[u] + g.dy * rz[u]) + lo : own;
+        more[u] = some ? static_cast<uint32_t>(hi - lo) : 0u;
+        b[u] = some ? 0u : 0x80000000u;  // no start is larger: a row of none stays empty
+#pragma unroll
+        for (uint32_t k = 0; k < 3; ++k) {
+            const uint32_t c = first[u] + min(k, more[u]);
+            start[u][k] = cs[c];
+            end[u][k] = static_cast<int>(ce[c]);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < kRows; ++u) {
+        // An empty cell's start is the largest, its end (as signed) the smallest.
+        b[u] = max(b[u], min(start[u][0], min(start[u][1], start[u][2])));
+        int last = max(end[u][0], max(end[u][1], end[u][2]));
+        for (uint32_t k = 3; k <= more[u]; ++k) {  // cells of less than h
+            b[u] = min(b[u], cs[first[u] + k]);
+            last = max(last, static_cast<int>(ce[first[u] + k]));
+        }
+        e[u] = min(static_cast<uint32_t>(max(last, 0)), n);
+    }
+}
+
 // The candidates of the targets in `todo` (a mask of 32) by a direct scan: each
 // lane walks every other row of its target's own stencil and evaluates the
-// candidates in range alone, r = 0 only with kSelf.
+// candidates in range alone, r = 0 only with kSelf.  Bound by latency: three rows
+// are looked up together and four candidates read together (a step of one million
+// particles at 1 a cell, one row and candidate after the other: 386 us, now 345).
 template <uint32_t kArrays, bool kSelf, class F, class G>
 __device__ __forceinline__ void walk_direct(const GridView& g, const GroupTargets& t, uint32_t todo,
                                             const uint32_t* __restrict__ cs,
@@ -533,29 +576,45 @@ __device__ __forceinline__ void walk_direct(const GridView& g, const GroupTarget
                                             const float4* __restrict__ a1,
                                             const float4* __restrict__ a2, F&& pair, G&& every8) {
     if (((todo >> (threadIdx.x & 31u)) & 1u) == 0u) return;
+    constexpr int kRows = 3;
+    constexpr uint32_t kAhead = 4;
     const Probe pr = make_probe(g, t.x.x, t.x.y, t.x.z);
     const float h2 = g.h * g.h;
     uint32_t turn = 0u;
-    int ry = pr.sy + ((threadIdx.x & 32u) != 0u ? 1 : 0), rz = pr.sz;
-    for (;; ry += 2) {
-        for (; ry > pr.ey; ry -= pr.ey - pr.sy + 1) ++rz;
-        if (rz > pr.ez) break;
-        uint32_t b, e;
-        probe_row_run(g, pr, cs, ce, n, ry, rz, b, e);
-        for (uint32_t j = b; j < e; ++j) {
-            const v4f q = *reinterpret_cast<const v4f*>(a0 + j);
-            const float dx = t.x.x - q.x, dy = t.x.y - q.y, dz = t.x.z - q.z;
-            const float r2 = dx * dx + dy * dy + dz * dz;
-            if (!(r2 < h2) || !(kSelf || r2 > 0.0f)) continue;  // a NaN too
-            if constexpr (kArrays == 1)
-                pair(q);
-            else if constexpr (kArrays == 2)
-                pair(q, *reinterpret_cast<const v4f*>(a1 + j));
-            else
-                pair(q, *reinterpret_cast<const v4f*>(a1 + j), *reinterpret_cast<const v4f*>(a2 + j));
-            if ((++turn & 7u) == 0u) every8();
+    int y = pr.sy + ((threadIdx.x & 32u) != 0u ? 1 : 0), z = pr.sz;
+    do {
+        int ry[kRows], rz[kRows];
+        uint32_t b[kRows], e[kRows];
+#pragma unroll
+        for (int u = 0; u < kRows; ++u, y += 2) {
+            for (; y > pr.ey; y -= pr.ey - pr.sy + 1) ++z;
+            ry[u] = y;
+            rz[u] = z;
         }
-    }
+        direct_rows<kRows>(g, pr, g.cell_offset + t.key, cs, ce, n, ry, rz, b, e);
+#pragma unroll
+        for (int u = 0; u < kRows; ++u)
+            for (uint32_t j = b[u]; j < e[u]; j += kAhead) {
+                v4f q[kAhead];
+#pragma unroll
+                for (uint32_t k = 0; k < kAhead; ++k)
+                    q[k] = *reinterpret_cast<const v4f*>(a0 + min(j + k, e[u] - 1u));
+#pragma unroll
+                for (uint32_t k = 0; k < kAhead; ++k) {
+                    const float dx = t.x.x - q[k].x, dy = t.x.y - q[k].y, dz = t.x.z - q[k].z;
+                    const float r2 = dx * dx + dy * dy + dz * dz;
+                    if (j + k >= e[u] || !(r2 < h2) || !(kSelf || r2 > 0.0f)) continue;  // a NaN too
+                    if constexpr (kArrays == 1)
+                        pair(q[k]);
+                    else if constexpr (kArrays == 2)
+                        pair(q[k], *reinterpret_cast<const v4f*>(a1 + j + k));
+                    else
+                        pair(q[k], *reinterpret_cast<const v4f*>(a1 + j + k),
+                             *reinterpret_cast<const v4f*>(a2 + j + k));
+                }
+                if ((++turn & 1u) == 0u) every8();
+            }
+    } while (z <= pr.ez);
     every8();
 }
 
@@ -567,11 +626,30 @@ __device__ __forceinline__ bool filter_holds(const GroupTargets& t, float inv_h)
     return __ballot(t.active && !(far * inv_h < 0x1p20f)) == 0ull;
 }
 
+// Whether the group's targets lie in few places: at most three runs of the same
+// 2^g.bucket cells, which are about the subgroups that walk_group would take one
+// after the other, each with a look-up of rows, a wait and two lanes per member.
+// A step of spray (us; direct scans from 2 runs on / 3 / 4 / 6 / never): one
+// million at 0.2 a cell 327 / 327 / 337 / 342 / 945, at 1 a cell 342 / 345 / 393 / 473 /
+// 470, at 4 a cell 341 / 320 / 320 / 324 / 315; a film of 200,000 one cell thick
+// across the rows, 16 a cell, 165 / 154 / 163 / 165 / 160; 32,000 with a fifth of
+// them above a pool 77 / 77 / 86 / 85 / 105.  (From 4 runs on with fewer loads
+// together.)
+constexpr uint32_t kMaxRuns = 3;
+__device__ __forceinline__ bool few_subgroups(const GridView& g, const GroupTargets& t) {
+    const uint32_t b = t.key >> g.bucket;
+    const uint32_t before = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(
+        0, static_cast<int>(b), 0x138, 0xf, 0xf, false));  // wave_shr:1
+    const uint32_t heads = static_cast<uint32_t>(__ballot(t.active && b != before)) | 1u;
+    return static_cast<uint32_t>(__builtin_popcount(heads)) <= kMaxRuns;
+}
+
 // The sums of a group's targets: walk_group, which multiplies what a candidate
 // out of range carries (v, A, B, ..) by 0.  That is no 0 if it is infinite or a
 // NaN, so a target whose sums are not finite is taken again by a direct scan,
 // which leaves such candidates out: then they are those of its neighbours.
-// Groups that the filter does not hold are scanned directly at once.
+// Groups that the filter does not hold, or that are spread over many places, are
+// scanned directly at once.
 // finite(): whether this lane's sums are; reset(): makes them 0.
 template <uint32_t kArrays, bool kSelf, class F, class G, class Ok, class Reset>
 __device__ __forceinline__ void walk_targets(const GridView& g, const GroupTargets& t, float inv_h,
@@ -583,7 +661,7 @@ __device__ __forceinline__ void walk_targets(const GridView& g, const GroupTarge
                                              const float4* __restrict__ a2, uint32_t tile,
                                              F&& pair, G&& every8, Ok&& finite, Reset&& reset) {
     uint64_t bad = __ballot(t.active);
-    if (filter_holds(t, inv_h)) {
+    if (filter_holds(t, inv_h) && few_subgroups(g, t)) {
         walk_group<kArrays>(g, t, inv_h, cs, ce, bins, n, a0, a1, a2, tile, pair, every8);
         bad = __ballot(t.active && !finite());
         if (bad == 0ull) return;
