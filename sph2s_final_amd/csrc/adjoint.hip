@@ -260,7 +260,8 @@ void k_adj_force(
         [&] {
             sumA = S1 = Sd = 0.f;
             gPx = gPy = gPz = gVx = gVy = gVz = gWx = gWy = gWz = 0.f;
-        });
+        },
+        [&] { return DirectScan{g, cs, ce, n, ixa, ivb, abar}; });
     sumA = both_halves(sumA);
     S1 = both_halves(S1);
     Sd = both_halves(Sd);
@@ -339,7 +340,8 @@ void k_adj_density(
             sy += c * dy;
             sz += c * dz;
         },
-        [] {}, [&] { return __builtin_isfinite(sx + sy + sz); }, [&] { sx = sy = sz = 0.f; });
+        [] {}, [&] { return __builtin_isfinite(sx + sy + sz); }, [&] { sx = sy = sz = 0.f; },
+        [&] { return DirectScan{g, cs, ce, n, xg, nullptr, nullptr}; });
     sx = both_halves(sx);
     sy = both_halves(sy);
     sz = both_halves(sz);

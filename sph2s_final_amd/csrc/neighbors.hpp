@@ -26,7 +26,8 @@ struct GridView {
     float prune_h2;     // (h (1 + 1e-3))^2
     int reach;          // cells that h spans on one axis (pairtile.hpp)
     int span;           // cells along x that one subgroup of targets may span (pairtile.hpp)
-    uint32_t bucket;    // log2 of cells that about fill a subgroup's span, or a row
+    uint32_t run_bits;  // log2 of the cells that about fill a subgroup's span, or a row
+    float filter_max;   // coordinates from here on are too large for the range filter
     float edge;         // a target this close to its cell's y or z face looks one row further
     uint32_t mx, my;    // n / dx = (n mx) >> (31 + lx) for n < 2^31, and likewise for dy
     uint32_t lx, ly;
@@ -56,8 +57,9 @@ __host__ __device__ inline GridView make_grid_view(float ox, float oy, float oz,
                            : static_cast<int>(fminf(ceilf(cells * (1.0f - 1e-6f)),
                                                     static_cast<float>(dmax < 1 << 24 ? dmax : 1 << 24)));
     g.span = static_cast<int>(fminf(6.0f * cells, 1e6f));
-    g.bucket = 0u;
-    while ((2 << g.bucket) <= g.span + 2 && (2 << g.bucket) <= dx) ++g.bucket;
+    g.run_bits = 0u;
+    while ((2 << g.run_bits) <= g.span + 2 && (2 << g.run_bits) <= dx) ++g.run_bits;
+    g.filter_max = 0x1p20f * h;
     // Division by multiplication (l = ceil(log2 d), m = floor(2^(31 + l) / d) + 1 is
     // exact for 31-bit dividends).
     auto magic = [](uint32_t d, uint32_t& m, uint32_t& l) {

@@ -127,6 +127,7 @@ struct Subgroup {
     float x0, x1;         // first and last x offset from the grid origin (clamped into it)
     float ox, oy, oz;     // origin of the filter's coordinates: near the targets
     int y0, z0, ny, nz;   // rows reached: ny x nz from (y0, z0), inside the grid
+    bool far;             // the filter's coordinates do not hold the targets
 };
 
 // The next subgroup of the targets in `rem` (a mask of 32 targets), which
@@ -138,6 +139,11 @@ __device__ __forceinline__ Subgroup next_subgroup(const GridView& g, const Group
     const float xf = lane_f32(t.x.x, first);
     s.oy = lane_f32(t.x.y, first);
     s.oz = lane_f32(t.x.z, first);
+    // From a million h from the origin on (or at a NaN): there the rounding of
+    // o / h is h / 16 and more, then the words' fill is no longer out of range,
+    // and beyond 2^31 h a target would miss itself.
+    auto size = [](float x) { return __float_as_uint(x) & 0x7FFFFFFFu; };
+    s.far = max(size(xf), max(size(s.oy), size(s.oz))) >= __float_as_uint(g.filter_max);
     const uint32_t key = min(lane_u32(t.key, first), 0x7FFFFFFFu);
     const uint32_t line = static_cast<uint32_t>((static_cast<uint64_t>(key) * g.mx) >> (31u + g.lx));
     const uint32_t row = line * static_cast<uint32_t>(g.dx);
@@ -293,9 +299,10 @@ constexpr float kFar = 1e15f, kFar2 = 3e30f;
 // Walks the candidates of a group in the internal x-order: their arrays a0 (x, .),
 // a1 and a2 (kArrays of them).  pair(q0, ..) evaluates this lane's target with one
 // candidate; every8() is called after at most nine of them, and at the end.
-// tile: LDS address of the wave's PairTile.
+// tile: LDS address of the wave's PairTile.  Returns the targets left out, those of
+// subgroups that the filter does not hold.
 template <uint32_t kArrays, class F, class G>
-__device__ __forceinline__ void walk_group(const GridView& g, const GroupTargets& t, float inv_h,
+__device__ __forceinline__ uint32_t walk_group(const GridView& g, const GroupTargets& t, float inv_h,
                                            const uint32_t* __restrict__ cs,
                                            const uint32_t* __restrict__ ce,
                                            const uint4* __restrict__ bins, uint32_t n,
@@ -314,9 +321,14 @@ __device__ __forceinline__ void walk_group(const GridView& g, const GroupTargets
             lds_write<v4f>(at + k * T::kArray, v4f{0.0f, 0.0f, 0.0f, 0.0f});
     }
     uint32_t turn = 0u;
-    uint32_t rem = static_cast<uint32_t>(__ballot(t.active));
+    uint32_t rem = static_cast<uint32_t>(__ballot(t.active)), left = 0u;
     while (rem) {
+        const uint32_t before = rem;
         const Subgroup s = next_subgroup(g, t, rem);
+        if (s.far) {
+            left |= before & ~rem;
+            continue;
+        }
         // Fills the words: out of the members' range, yet finite in FP16 (an
         // infinity would make the products NaN, and its sign a hit).
         const v4f far = {s.ox + 100.0f * __builtin_amdgcn_rcpf(inv_h), s.oy, s.oz, 0.0f};
@@ -520,16 +532,41 @@ __device__ __forceinline__ void walk_group(const GridView& g, const GroupTargets
             wave_sync();
         }
     }
+    return left;
+}
+
+// What a direct scan reads.
+struct DirectScan {
+    GridView g;
+    const uint32_t *cs, *ce;
+    uint32_t n;
+    const float4 *a0, *a1, *a2;
+};
+
+// A kernel's first arguments again, from memory: values that only the direct scan
+// needs are then not held in registers through the group walk (force of one million
+// settled 192 us held, 187 read again).
+template <class Args>
+__device__ __forceinline__ Args first_arguments() {
+    static_assert(sizeof(Args) % 4 == 0, "copied by words");
+    typedef const __attribute__((address_space(4))) uint32_t* Words;
+    Words p = reinterpret_cast<Words>(
+        reinterpret_cast<uintptr_t>(__builtin_amdgcn_kernarg_segment_ptr()));
+    asm volatile("" : "+s"(p));
+    Args a;
+    uint32_t w[sizeof(Args) / 4];
+#pragma unroll
+    for (uint32_t k = 0; k < sizeof(Args) / 4; ++k) w[k] = p[k];
+    __builtin_memcpy(&a, w, sizeof(Args));
+    return a;
 }
 
 // Candidate runs [b, e) of kRows rows (ry, rz) of a target's stencil (empty rows
 // and rows outside it: b >= e), the cells as in probe_row_run.  The loads of all
 // rows go out together.
 template <int kRows>
-__device__ __forceinline__ void direct_rows(const GridView& g, const Probe& pr, uint32_t own,
-                                            const uint32_t* __restrict__ cs,
-                                            const uint32_t* __restrict__ ce, uint32_t n,
-                                            const int* ry, const int* rz, uint32_t* b, uint32_t* e) {
+__device__ __forceinline__ void direct_rows(const GridView& g, const Probe& pr, const uint32_t* cs,
+                                            const uint32_t* ce, uint32_t n, const int* ry, const int* rz, uint32_t* b, uint32_t* e) {
     uint32_t first[kRows], more[kRows], start[kRows][3];
     int end[kRows][3];
 #pragma unroll
@@ -540,7 +577,8 @@ __device__ __forceinline__ void direct_rows(const GridView& g, const Probe& pr, 
         const int lo = max(pr.sx, static_cast<int>(floorf((pr.fx - w) * g.inv_spacing)));
         const int hi = min(pr.ex, static_cast<int>(floorf((pr.fx + w) * g.inv_spacing)));
         const bool some = w2 > 0.0f && ry[u] <= pr.ey && rz[u] <= pr.ez && lo <= hi;
-        first[u] = some ? g.cell_offset + static_cast<uint32_t>(g.dx) * (ry[u] + g.dy * rz[u]) + lo : own;
+        first[u] = some ? g.cell_offset + static_cast<uint32_t>(g.dx) * (ry[u] + g.dy * rz[u]) + lo
+                        : g.cell_offset;  // any
         more[u] = some ? static_cast<uint32_t>(hi - lo) : 0u;
         b[u] = some ? 0u : 0x80000000u;  // no start is larger: a row of none stays empty
 #pragma unroll
@@ -563,95 +601,123 @@ __device__ __forceinline__ void direct_rows(const GridView& g, const Probe& pr, 
     }
 }
 
+// This lane's half of its target's rows, three at a time: the next row to look up
+// and the candidate runs [b, e) of the last three.
+struct DirectRows {
+    Probe pr;
+    int y, z;
+    uint32_t b[3], e[3];
+};
+__device__ __forceinline__ void next_rows(const DirectScan& d, DirectRows& r) {
+    int ry[3], rz[3];
+#pragma unroll
+    for (int u = 0; u < 3; ++u, r.y += 2) {
+        for (; r.y > r.pr.ey; r.y -= r.pr.ey - r.pr.sy + 1) ++r.z;
+        ry[u] = r.y;
+        rz[u] = r.z;
+    }
+    direct_rows<3>(d.g, r.pr, d.cs, d.ce, d.n, ry, rz, r.b, r.e);
+}
+__device__ __forceinline__ DirectRows first_rows(const DirectScan& d, const GroupTargets& t) {
+    DirectRows r;
+    r.pr = make_probe(d.g, t.x.x, t.x.y, t.x.z);
+    r.y = r.pr.sy + ((threadIdx.x & 32u) != 0u ? 1 : 0);
+    r.z = r.pr.sz;
+    next_rows(d, r);
+    return r;
+}
+
 // The candidates of the targets in `todo` (a mask of 32) by a direct scan: each
-// lane walks every other row of its target's own stencil and evaluates the
-// candidates in range alone, r = 0 only with kSelf.  Bound by latency: three rows
-// are looked up together and four candidates read together (a step of one million
-// particles at 1 a cell, one row and candidate after the other: 386 us, now 345).
+// lane walks every other row of its target's own stencil (r: the first three) and
+// evaluates the candidates in range alone, r = 0 only with kSelf.  Bound by latency:
+// three rows are looked up together and four candidates read together (a step of one
+// million particles at 1 a cell, one row and candidate after the other: 386 us, now
+// 335).
 template <uint32_t kArrays, bool kSelf, class F, class G>
-__device__ __forceinline__ void walk_direct(const GridView& g, const GroupTargets& t, uint32_t todo,
-                                            const uint32_t* __restrict__ cs,
-                                            const uint32_t* __restrict__ ce, uint32_t n,
-                                            const float4* __restrict__ a0,
-                                            const float4* __restrict__ a1,
-                                            const float4* __restrict__ a2, F&& pair, G&& every8) {
+__device__ __forceinline__ void walk_direct(const DirectScan& d, DirectRows r, const GroupTargets& t,
+                                            uint32_t todo, F&& pair, G&& every8) {
     if (((todo >> (threadIdx.x & 31u)) & 1u) == 0u) return;
-    constexpr int kRows = 3;
     constexpr uint32_t kAhead = 4;
-    const Probe pr = make_probe(g, t.x.x, t.x.y, t.x.z);
-    const float h2 = g.h * g.h;
+    const float h2 = d.g.h * d.g.h;
     uint32_t turn = 0u;
-    int y = pr.sy + ((threadIdx.x & 32u) != 0u ? 1 : 0), z = pr.sz;
-    do {
-        int ry[kRows], rz[kRows];
-        uint32_t b[kRows], e[kRows];
+    auto run = [&](uint32_t b, uint32_t e) {
+        for (uint32_t j = b; j < e; j += kAhead) {
+            v4f q0[kAhead], q1[kAhead], q2[kAhead];
 #pragma unroll
-        for (int u = 0; u < kRows; ++u, y += 2) {
-            for (; y > pr.ey; y -= pr.ey - pr.sy + 1) ++z;
-            ry[u] = y;
-            rz[u] = z;
-        }
-        direct_rows<kRows>(g, pr, g.cell_offset + t.key, cs, ce, n, ry, rz, b, e);
-#pragma unroll
-        for (int u = 0; u < kRows; ++u)
-            for (uint32_t j = b[u]; j < e[u]; j += kAhead) {
-                v4f q[kAhead];
-#pragma unroll
-                for (uint32_t k = 0; k < kAhead; ++k)
-                    q[k] = *reinterpret_cast<const v4f*>(a0 + min(j + k, e[u] - 1u));
-#pragma unroll
-                for (uint32_t k = 0; k < kAhead; ++k) {
-                    const float dx = t.x.x - q[k].x, dy = t.x.y - q[k].y, dz = t.x.z - q[k].z;
-                    const float r2 = dx * dx + dy * dy + dz * dz;
-                    if (j + k >= e[u] || !(r2 < h2) || !(kSelf || r2 > 0.0f)) continue;  // a NaN too
-                    if constexpr (kArrays == 1)
-                        pair(q[k]);
-                    else if constexpr (kArrays == 2)
-                        pair(q[k], *reinterpret_cast<const v4f*>(a1 + j + k));
-                    else
-                        pair(q[k], *reinterpret_cast<const v4f*>(a1 + j + k),
-                             *reinterpret_cast<const v4f*>(a2 + j + k));
-                }
-                if ((++turn & 1u) == 0u) every8();
+            for (uint32_t k = 0; k < kAhead; ++k) {
+                const uint32_t at = min(j + k, e - 1u);
+                q0[k] = *reinterpret_cast<const v4f*>(d.a0 + at);
+                if constexpr (kArrays > 1) q1[k] = *reinterpret_cast<const v4f*>(d.a1 + at);
+                if constexpr (kArrays > 2) q2[k] = *reinterpret_cast<const v4f*>(d.a2 + at);
             }
-    } while (z <= pr.ez);
+#pragma unroll
+            for (uint32_t k = 0; k < kAhead; ++k) {
+                const float dx = t.x.x - q0[k].x, dy = t.x.y - q0[k].y, dz = t.x.z - q0[k].z;
+                const float r2 = dx * dx + dy * dy + dz * dz;
+                if (j + k >= e || !(r2 < h2) || !(kSelf || r2 > 0.0f)) continue;  // a NaN too
+                if constexpr (kArrays == 1)
+                    pair(q0[k]);
+                else if constexpr (kArrays == 2)
+                    pair(q0[k], q1[k]);
+                else
+                    pair(q0[k], q1[k], q2[k]);
+            }
+            if ((++turn & 1u) == 0u) every8();
+        }
+    };
+    for (;;) {
+#pragma unroll
+        for (int u = 0; u < 3; ++u) run(r.b[u], r.e[u]);
+        if (r.z > r.pr.ez) break;
+        next_rows(d, r);
+    }
     every8();
 }
 
-// Whether the filter's coordinates hold the group: from a million h on (or at a
-// NaN) their origin is off by h / 16 and more, then the words' fill is no longer
-// out of range, and beyond 2^31 h a target would miss itself.
-__device__ __forceinline__ bool filter_holds(const GroupTargets& t, float inv_h) {
-    const float far = fabsf(t.x.x) + fabsf(t.x.y) + fabsf(t.x.z);
-    return __ballot(t.active && !(far * inv_h < 0x1p20f)) == 0ull;
+// Whether the group's targets lie in few places: at most three runs of the same
+// 2^g.run_bits cells, which are about the subgroups that walk_group would take one
+// after the other, each with a look-up of rows, a wait and two lanes per member.
+// A step of spray (us; direct scans from 3 runs on / 4 / 5 / 7 / never): one million
+// at 0.2 a cell 327 / 327 / 337 / 342 / 945, at 1 a cell 342 / 345 / 393 / 473 / 470, at 4 a
+// cell 341 / 320 / 320 / 324 / 315; a film of 200,000 one cell thick across the rows, 16
+// a cell, 165 / 154 / 163 / 165 / 160.  (From 5 runs on with fewer loads together.)
+constexpr uint32_t kMaxRuns = 3;
+__device__ __forceinline__ bool few_runs(const GridView& g, const GroupTargets& t) {
+    const uint32_t active = static_cast<uint32_t>(__ballot(t.active));
+    const uint32_t from = lane_u32(t.key, 0) >> g.run_bits;
+    const uint32_t to = lane_u32(t.key, 31 - __builtin_clz(active)) >> g.run_bits;
+    if (to - from < kMaxRuns) return true;  // nearly all groups of a dense state
+    const uint32_t run = t.key >> g.run_bits;
+    const uint32_t before = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(
+        0, static_cast<int>(run), 0x138, 0xf, 0xf, false));  // wave_shr:1
+    const uint32_t heads = static_cast<uint32_t>(__ballot(t.active && run != before)) | 1u;
+    return static_cast<uint32_t>(__builtin_popcount(heads)) <= kMaxRuns;
 }
 
-// Whether the group's targets lie in few places: at most three runs of the same
-// 2^g.bucket cells, which are about the subgroups that walk_group would take one
-// after the other, each with a look-up of rows, a wait and two lanes per member.
-// A step of spray (us; direct scans from 2 runs on / 3 / 4 / 6 / never): one
-// million at 0.2 a cell 327 / 327 / 337 / 342 / 945, at 1 a cell 342 / 345 / 393 / 473 /
-// 470, at 4 a cell 341 / 320 / 320 / 324 / 315; a film of 200,000 one cell thick
-// across the rows, 16 a cell, 165 / 154 / 163 / 165 / 160; 32,000 with a fifth of
-// them above a pool 77 / 77 / 86 / 85 / 105.  (From 4 runs on with fewer loads
-// together.)
-constexpr uint32_t kMaxRuns = 3;
-__device__ __forceinline__ bool few_subgroups(const GridView& g, const GroupTargets& t) {
-    const uint32_t b = t.key >> g.bucket;
-    const uint32_t before = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(
-        0, static_cast<int>(b), 0x138, 0xf, 0xf, false));  // wave_shr:1
-    const uint32_t heads = static_cast<uint32_t>(__ballot(t.active && b != before)) | 1u;
-    return static_cast<uint32_t>(__builtin_popcount(heads)) <= kMaxRuns;
+// Whether some lane has more candidates in its first three rows than a direct scan is
+// the faster for: spread groups at the surface of a dense state are walked together.
+// A step (us, limit 28 / 40 / 56 / 72 / 100): 32,000 with a fifth above a pool 102 / 102 /
+// 87 / 85 / 73, a film across the rows, 200,000, at 4 a cell 145 / 129 / 129 / 130 / 130,
+// at 16 a cell 166 / 167 / 161 / 153 / 154; 24 scenes of 4096 to 98304, 24 steps, 5421 /
+// 5417 / 5414 / 5429 / 5439.  Without a limit a step of one settled million took 9 us
+// more.
+constexpr uint32_t kMostCandidates = 72;
+__device__ __forceinline__ bool many_candidates(const DirectRows& r, const GroupTargets& t) {
+    uint32_t count = 0u;
+#pragma unroll
+    for (int u = 0; u < 3; ++u) count += r.e[u] > r.b[u] ? r.e[u] - r.b[u] : 0u;
+    return __ballot(t.active && count > kMostCandidates) != 0ull;
 }
 
 // The sums of a group's targets: walk_group, which multiplies what a candidate
 // out of range carries (v, A, B, ..) by 0.  That is no 0 if it is infinite or a
 // NaN, so a target whose sums are not finite is taken again by a direct scan,
 // which leaves such candidates out: then they are those of its neighbours.
-// Groups that the filter does not hold, or that are spread over many places, are
-// scanned directly at once.
-// finite(): whether this lane's sums are; reset(): makes them 0.
-template <uint32_t kArrays, bool kSelf, class F, class G, class Ok, class Reset>
+// Targets that the filter does not hold are scanned directly too, and so are groups
+// that are spread over many places.
+// finite(): whether this lane's sums are; reset(): makes them 0; scan(): the
+// DirectScan.
+template <uint32_t kArrays, bool kSelf, class F, class G, class Ok, class Reset, class Scan>
 __device__ __forceinline__ void walk_targets(const GridView& g, const GroupTargets& t, float inv_h,
                                              const uint32_t* __restrict__ cs,
                                              const uint32_t* __restrict__ ce,
@@ -659,16 +725,27 @@ __device__ __forceinline__ void walk_targets(const GridView& g, const GroupTarge
                                              const float4* __restrict__ a0,
                                              const float4* __restrict__ a1,
                                              const float4* __restrict__ a2, uint32_t tile,
-                                             F&& pair, G&& every8, Ok&& finite, Reset&& reset) {
-    uint64_t bad = __ballot(t.active);
-    if (filter_holds(t, inv_h) && few_subgroups(g, t)) {
-        walk_group<kArrays>(g, t, inv_h, cs, ce, bins, n, a0, a1, a2, tile, pair, every8);
-        bad = __ballot(t.active && !finite());
-        if (bad == 0ull) return;
+                                             F&& pair, G&& every8, Ok&& finite, Reset&& reset,
+                                             Scan&& scan) {
+    uint32_t todo = static_cast<uint32_t>(__ballot(t.active));
+    bool together = few_runs(g, t);
+    DirectScan d;
+    DirectRows rows;
+    if (!together) {
+        d = scan();
+        rows = first_rows(d, t);
+        together = many_candidates(rows, t);
     }
-    const uint32_t todo = static_cast<uint32_t>(bad) | static_cast<uint32_t>(bad >> 32);
+    if (together) {
+        todo = walk_group<kArrays>(g, t, inv_h, cs, ce, bins, n, a0, a1, a2, tile, pair, every8);
+        const uint64_t bad = __ballot(t.active && !finite());
+        todo |= static_cast<uint32_t>(bad) | static_cast<uint32_t>(bad >> 32);
+        if (todo == 0u) return;
+        d = scan();
+        rows = first_rows(d, t);
+    }
     if ((todo >> (threadIdx.x & 31u)) & 1u) reset();
-    walk_direct<kArrays, kSelf>(g, t, todo, cs, ce, n, a0, a1, a2, pair, every8);
+    walk_direct<kArrays, kSelf>(d, rows, t, todo, pair, every8);
 }
 
 }  // namespace sph

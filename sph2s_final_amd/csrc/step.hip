@@ -332,6 +332,20 @@ __device__ __forceinline__ float poly6_unit(const float4& xi, const v4f& xj, flo
     return __builtin_amdgcn_fmed3f(__builtin_fmaf(-r2, inv_h2, 1.0f), 0.0f, 1.0f);
 }
 
+// The first arguments of k_density and k_force, in their order (arrays: of the
+// candidates), and their direct scan's view of them.
+struct WalkArguments {
+    GridView g;
+    const uint32_t *cs, *ce, *n_dev;
+    const float4 *a0, *a1;
+    const SceneParams* scenes;
+};
+template <bool kBatched>
+__device__ __forceinline__ DirectScan scan_again(uint32_t scene) {
+    const WalkArguments w = first_arguments<WalkArguments>();
+    return DirectScan{kBatched ? w.scenes[scene].g : w.g, w.cs, w.ce, *w.n_dev, w.a0, w.a1, nullptr};
+}
+
 // computeDensitiesPressuresD + computeDensityCell (Solver.cu:198-229,536-599):
 // rho_i = m c6 sum_{r_ij < h} (h^2 - r_ij^2)^3, self included, evaluated as
 // (m c6 h^6) sum a^3 with a = 1 - r_ij^2 / h^2 (poly6_unit).  Terms are added in
@@ -351,11 +365,11 @@ __device__ __forceinline__ float poly6_unit(const float4& xi, const v4f& xj, flo
 // global cell array.
 template <bool kKahan, bool kFinalize, bool kBatched>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(5))) void k_density(
-    const float4* __restrict__ ipos, const float4* __restrict__ ivel,
-    const uint32_t* __restrict__ skeys, const uint32_t* __restrict__ cs,
-    const uint32_t* __restrict__ ce, StepParams p_in, GridView g_in,
-    const uint32_t* __restrict__ n_dev, float* __restrict__ rho, float2* __restrict__ aux,
-    float4* __restrict__ ixa, float4* __restrict__ ivb, const SceneParams* __restrict__ scenes,
+    GridView g_in, const uint32_t* __restrict__ cs, const uint32_t* __restrict__ ce,
+    const uint32_t* __restrict__ n_dev, const float4* __restrict__ ipos,
+    const float4* __restrict__ ivel, const SceneParams* __restrict__ scenes,
+    const uint32_t* __restrict__ skeys, StepParams p_in, float* __restrict__ rho,
+    float2* __restrict__ aux, float4* __restrict__ ixa, float4* __restrict__ ivb,
     const uint4* __restrict__ groups, uint32_t n_groups, XOrder xo, LaunchShape sh) {
     extern __shared__ __align__(kTileAlign) unsigned char lds[];
     const uint32_t wave = uniform_u32(threadIdx.x >> 6), waves = blockDim.x >> 6;
@@ -386,7 +400,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(5))) void k
                         sum32 = 0.0f;
                     }
                 },
-                [] { return true; }, [] {});
+                [] { return true; }, [] {}, [&] { return scan_again<kBatched>(gr.scene); });
             const float r = p.c6m_h6 * (kKahan ? static_cast<float>(both_halves(sum64))
                                                : both_halves(sum32));
             if (t.active && (threadIdx.x & 32u) == 0u) {
@@ -517,13 +531,13 @@ __device__ __forceinline__ void force_finish(const PairSums<kTension>& S, const 
 // 116 -> 90, one million 320 -> 200, one million at rest 150 -> 110.
 template <bool kTension, bool kIntegrate, bool kBatched>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_force(
+    GridView g_in, const uint32_t* __restrict__ cs, const uint32_t* __restrict__ ce,
+    const uint32_t* __restrict__ n_dev, const float4* __restrict__ ixa,
+    const float4* __restrict__ ivb, const SceneParams* __restrict__ scenes,
     const float4* __restrict__ ipos, const float4* __restrict__ ivel,
-    const float4* __restrict__ ixa, const float4* __restrict__ ivb,
-    const uint32_t* __restrict__ skeys, const uint32_t* __restrict__ cs,
-    const uint32_t* __restrict__ ce, StepParams p_in, GridView g_in,
-    const uint32_t* __restrict__ n_dev, float dt, float4* __restrict__ pos,
-    float4* __restrict__ vel, float4* __restrict__ accel, const SceneParams* __restrict__ scenes,
-    const uint4* __restrict__ groups, uint32_t n_groups, XOrder xo, LaunchShape sh) {
+    const uint32_t* __restrict__ skeys, StepParams p_in, float dt, float4* __restrict__ pos,
+    float4* __restrict__ vel, float4* __restrict__ accel, const uint4* __restrict__ groups,
+    uint32_t n_groups, XOrder xo, LaunchShape sh) {
     extern __shared__ __align__(kTileAlign) unsigned char lds[];
     const uint32_t wave = uniform_u32(threadIdx.x >> 6), waves = blockDim.x >> 6;
     const uint32_t tile = lds_address(lds) + wave * ForceTile::kBytes;
@@ -543,7 +557,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
             walk_targets<2, false>(
                 g, t, p.inv_h, cs, ce, xo.bins, n, ixa, ivb, nullptr, tile,
                 [&](const v4f& x, const v4f& v) { S.add(xi, vi, t.x.w, p.h, p.h2, x, v); }, [] {},
-                [&] { return S.finite(); }, [&] { S = PairSums<kTension>{}; });
+                [&] { return S.finite(); }, [&] { S = PairSums<kTension>{}; },
+                [&] { return scan_again<kBatched>(gr.scene); });
             S.Px = both_halves(S.Px);
             S.Py = both_halves(S.Py);
             S.Pz = both_halves(S.Pz);
@@ -826,8 +841,8 @@ void launch_density(uint32_t tune, uint32_t cap_n, hipStream_t st, const StepBuf
         launch_shape(n_groups, DensityTile::kBytes, tune & 0xFu, (tune >> 8) & 0xFu,
                      (tune >> 16) & 0x3u, kBatched ? 1u : 1u + ((tune >> 20) & 1u));
     hipLaunchKernelGGL((k_density<kKahan, kFinalize, kBatched>), sh.grid, sh.block, sh.lds, st,
-                       b.ipos, b.ivel, b.skeys, b.cell_start, b.cell_end, p, g, b.n_dev, b.rho, aux,
-                       b.ixa, b.ivb, scenes, b.groups, n_groups, xo, sh);
+                       g, b.cell_start, b.cell_end, b.n_dev, b.ipos, b.ivel, scenes, b.skeys, p, b.rho,
+                       aux, b.ixa, b.ivb, b.groups, n_groups, xo, sh);
 }
 
 template <bool kTension, bool kIntegrate, bool kBatched>
@@ -840,8 +855,8 @@ void launch_force(uint32_t tune, uint32_t cap_n, hipStream_t st, const StepBuffe
         launch_shape(n_groups, ForceTile::kBytes, (tune >> 4) & 0xFu, (tune >> 12) & 0xFu,
                      (tune >> 18) & 0x3u, kBatched ? 1u : 1u + ((tune >> 22) & 1u));
     hipLaunchKernelGGL((k_force<kTension, kIntegrate, kBatched>), sh.grid, sh.block, sh.lds, st,
-                       b.ipos, b.ivel, b.ixa, b.ivb, b.skeys, b.cell_start, b.cell_end, p, g,
-                       b.n_dev, dt, pos, vel, accel, scenes, b.groups, n_groups, xo, sh);
+                       g, b.cell_start, b.cell_end, b.n_dev, b.ixa, b.ivb, scenes, b.ipos, b.ivel,
+                       b.skeys, p, dt, pos, vel, accel, b.groups, n_groups, xo, sh);
 }
 
 __global__ void k_pack_state(const float* __restrict__ pxyz, const float* __restrict__ vxyz,

@@ -727,7 +727,8 @@ void k_blend_density(
             const float a = __builtin_amdgcn_fmed3f(pa.h2 - r2, 0.0f, pa.h2);
             own += q.w * (a * a * a);
         },
-        [] {}, [&] { return __builtin_isfinite(own); }, [&] { own = 0.0f; });
+        [] {}, [&] { return __builtin_isfinite(own); }, [&] { own = 0.0f; },
+        [&] { return DirectScan{ga, cs_a, ce_a, na, ixl_a, nullptr, nullptr}; });
     own = both_halves(own);
     if (!t.active || (threadIdx.x & 32u) != 0u) return;
     const float r = pa.c6m * own;
@@ -802,7 +803,8 @@ void k_blend_force_integrate(
         [&] {
             return __builtin_isfinite(((Px + Py) + (Pz + Vx)) + ((Vy + Vz) + ((Tx + Ty) + Tz)));
         },
-        [&] { Px = Py = Pz = Vx = Vy = Vz = Tx = Ty = Tz = 0.f; });
+        [&] { Px = Py = Pz = Vx = Vy = Vz = Tx = Ty = Tz = 0.f; },
+        [&] { return DirectScan{ga, cs_a, ce_a, na, ixa_a, ivb_a, il_a}; });
     Px = both_halves(Px);
     Py = both_halves(Py);
     Pz = both_halves(Pz);
