@@ -279,20 +279,22 @@ int sph_count_pairs(sph_solver* s, uint64_t counts[2]);
  * density and force passes have launch variants, selected by a tune word:
  *   bits 0-3   density, bits 4-7 force: waves per block, each handling 32
  *              particles at a time on an LDS tile of its own: 0 = the default
- *              (4); density 1..5 and force 1..9 choose others (1 to 6)
+ *              (4), 1..5 = 1, 2, 3, 5, 6; force 6..9 = the default
  *   bits 8-11  density grid, bits 12-15 force grid: 0 = one block per its
  *              waves' particles; 1..4 = persistent grid of 1, 2, 4, 8
  *              blocks per CU looping over those blocks
  *   bits 16-17 density block size, bits 18-19 force block size: 0 = 256,
- *              1 = 128, 2 = up to 512 threads; a non-zero block size requires
- *              that pass's waves field to be 0
+ *              1 = 128, 2 = 512 threads (force: 384); a non-zero block size
+ *              requires that pass's waves field to be 0
  *   bits 20-21 density, bits 22-23 force: groups of 32 particles that a wave
  *              takes one after the other, 0 = 1, 1 = 2; 1 requires that pass's
  *              waves and block-size fields to be 0, and a batch refuses it
  *   bits 24-31 must be zero; other words are refused with SPH_ERR_ARG
- * All variants give bit-identical results.  sph_autotune times the variants
- * on the solver's current state (reps launches each), keeps the fastest and
- * returns its tune word; ms[4] (may be NULL) receives the default and tuned
+ * All variants give bit-identical results.  Some passes have one launch shape
+ * and ignore their fields: both passes of a scene with boundary particles (not
+ * with SPH_FLAG_XSPH), and the force with tension.  sph_autotune times each
+ * launch shape on the solver's current state (reps launches each), keeps the
+ * fastest (0 where there is one) and returns its tune word; ms[4] (may be NULL) receives the default and tuned
  * milliseconds of density and force.  The state is unchanged; the solver's
  * intermediate fields (density, sorted arrays) then hold the tuning pass's
  * values. */

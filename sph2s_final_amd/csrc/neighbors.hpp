@@ -13,6 +13,7 @@
 // number of candidates tested drops.
 #pragma once
 
+#include <functional>
 #include <type_traits>
 
 #include "internal.hpp"
@@ -209,6 +210,15 @@ int launch_batch_pass(int pass, const StepParams& cap, const StepBuffers& b,
 // constants) and returns the fastest tune word; ms_out (may be NULL) gets the
 // default and tuned milliseconds of density and force.  pos/vel are restored.
 bool tune_word_valid(uint32_t tune, bool batched);
+// One pass's part of it: time(word, ms) times a word; each launch shape is timed
+// once (several words choose the same).  one_shape: the pass has but one, whose word
+// is 0.
+struct TunedPass {
+    uint32_t word = 0u;
+    float default_ms = 0.0f, best_ms = 0.0f;
+};
+int tune_pass(bool force, bool one_shape, uint32_t groups, bool batched,
+              const std::function<int(uint32_t, float&)>& time, TunedPass& out);
 int tune_neighbour_passes(StepParams p, const StepBuffers& b, const SceneParams* scenes,
                           bool kahan, bool tension, float dt, uint32_t key_bits, uint32_t reps,
                           hipStream_t stream, uint32_t* tune_out, float* ms_out);

@@ -17,6 +17,8 @@
 // (vx, vy, vz, 0), one 16-byte load per particle.  Within one row (cy, cz)
 // of the grid the cells cx are consecutive hashes, so a stencil row of up to
 // three cells is one contiguous run of sorted particles.
+#include <vector>
+
 #include "neighbors.hpp"
 #include "diagnostics.hpp"
 #include "pairtile.hpp"
@@ -249,7 +251,8 @@ __global__ __launch_bounds__(kBlock) void k_order(const uint32_t* __restrict__ s
 // Launch shapes of the neighbour passes, selected at run time by the tune word
 // (StepParams::tune; 0 = the defaults).  Every shape computes bit-identical
 // results: a target's sums depend on its group of 32 alone (pairtile.hpp), and
-// the shape only decides which wave handles which group.
+// the shape only decides which wave handles which group.  Walled scenes' passes in
+// row order have one shape.
 //   bits 0-3   density, bits 4-7 force: waves per block (kTileWaves)
 //   bits 8-11  density grid:       one block per its waves' groups, or a
 //   bits 12-15 force grid:         persistent grid of 1, 2, 4, 8 blocks per CU
@@ -262,8 +265,11 @@ __global__ __launch_bounds__(kBlock) void k_order(const uint32_t* __restrict__ s
 //
 typedef PairTile<1> DensityTile;
 typedef PairTile<2> ForceTile;
-// Waves share nothing but the launch: 2 and 4 waves are within 3% of each other
-// on every size, the rest is left to the tuner.
+// Waves share nothing but the launch, so the number is a matter of tails and is left
+// to the tuner.  Density / force of 15 steps in ms with 4 waves, 1, 2, 3 and 5: 4.1 million
+// in 64 scenes 5.26 / 7.45, 4.91 / 6.72, 5.02 / 7.06, 5.17 / 7.61, 7.22 / 11.1; one million
+// 1.54 / 2.12, 1.47 / 2.01 with 1; 32,768 0.343 / 0.387 with either.  Values 6 to 9 were
+// variants of their own once and stay valid words.
 constexpr uint32_t kTileWaves[] = {4, 1, 2, 3, 5, 6, 4, 4, 4, 4};
 constexpr uint32_t kMaxBlockLds = 64u << 10;
 // Groups in a row that one XCD takes (32, 128 and 512: within 2%).
@@ -1202,6 +1208,41 @@ bool tune_word_valid(uint32_t tune, bool batched) {
            (fppl == 0u || (fvar == 0u && fblock == 0u)) && (!batched || (dppl | fppl) == 0u);
 }
 
+int tune_pass(bool force, bool one_shape, uint32_t groups, bool batched,
+              const std::function<int(uint32_t, float&)>& time, TunedPass& out) {
+    const uint32_t tile = force ? ForceTile::kBytes : DensityTile::kBytes;
+    const int waves = force ? 4 : 0, grid = force ? 12 : 8, block = force ? 18 : 16,
+              pairs = force ? 22 : 20;
+    out = TunedPass{};
+    int rc = time(0u, out.default_ms);
+    out.best_ms = out.default_ms;
+    std::vector<LaunchShape> seen;
+    auto is_new = [&](uint32_t w) {
+        const LaunchShape s = launch_shape(groups, tile, (w >> waves) & 0xFu, (w >> grid) & 0xFu,
+                                           (w >> block) & 0x3u, 1u + ((w >> pairs) & 1u));
+        for (const LaunchShape& o : seen)
+            if (o.grid.x == s.grid.x && o.block.x == s.block.x && o.per == s.per) return false;
+        seen.push_back(s);
+        return true;
+    };
+    auto consider = [&](uint32_t w) {
+        float ms = 0.0f;
+        if (rc != SPH_OK || one_shape || !is_new(w)) return;
+        rc = time(w, ms);
+        if (rc == SPH_OK && ms < out.best_ms) {
+            out.best_ms = ms;
+            out.word = w;
+        }
+    };
+    (void)is_new(0u);
+    for (uint32_t v = 1; v <= (force ? 9u : 5u); ++v) consider(v << waves);
+    for (uint32_t v = 1; v <= 2; ++v) consider(v << block);
+    if (!batched) consider(1u << pairs);
+    const uint32_t shape = out.word;
+    for (uint32_t v = 1; v <= 4; ++v) consider(shape | (v << grid));
+    return rc;
+}
+
 int tune_neighbour_passes(StepParams p, const StepBuffers& b, const SceneParams* scenes,
                           bool kahan, bool tension, float dt, uint32_t key_bits, uint32_t reps,
                           hipStream_t stream, uint32_t* tune_out, float* ms_out) {
@@ -1249,65 +1290,28 @@ int tune_neighbour_passes(StepParams p, const StepBuffers& b, const SceneParams*
         ms /= static_cast<float>(reps);
         return SPH_OK;
     };
-    // Density: tile first (256-thread blocks), then the 128- and 512-thread
-    // blocks and two particles per lane with the default tile, then the grid
-    // shape for the best of them.
-    float d_def = 0.f, d_best = 0.f, ms = 0.f;
-    uint32_t d_shape = 0, d_grid = 0;  // d_shape: tile bits, or block bits << 16
-    for (uint32_t v = 0; v <= 5 && rc == SPH_OK; ++v) {
-        rc = time_pass(kPassDensity, v, ms);
-        if (v == 0) d_def = d_best = ms;
-        else if (ms < d_best) { d_best = ms; d_shape = v; }
-    }
-    for (uint32_t bv = 1; bv <= 2 && rc == SPH_OK; ++bv) {
-        rc = time_pass(kPassDensity, bv << 16, ms);
-        if (ms < d_best) { d_best = ms; d_shape = bv << 16; }
-    }
-    if (!scenes && rc == SPH_OK) {  // two particles per lane (single scene)
-        rc = time_pass(kPassDensity, 1u << 20, ms);
-        if (ms < d_best) { d_best = ms; d_shape = 1u << 20; }
-    }
-    for (uint32_t gsh = 1; gsh <= 4 && rc == SPH_OK; ++gsh) {
-        rc = time_pass(kPassDensity, d_shape | (gsh << 8), ms);
-        if (ms < d_best) { d_best = ms; d_grid = gsh; }
-    }
-    if (rc != SPH_OK) return fail(rc);
-    const uint32_t dword = d_shape | (d_grid << 8);
-    rc = run(kPassDensity, dword);  // aux for the force pass
-    // Force: variant first, then the 128- and 512-thread blocks and two
-    // particles per lane with the default variant, then the grid shape
-    // (tension runs the default).
-    float f_def = 0.f, f_best = 0.f;
-    uint32_t f_shape = 0, f_grid = 0;  // variant bits << 4, or block bits << 18
-    for (uint32_t v = 0; v <= (tension ? 0u : 9u) && rc == SPH_OK; ++v) {
-        rc = time_pass(kPassForce, dword | (v << 4), ms);
-        if (v == 0) f_def = f_best = ms;
-        else if (ms < f_best) { f_best = ms; f_shape = v << 4; }
-    }
-    for (uint32_t bv = 1; bv <= (tension ? 0u : 2u) && rc == SPH_OK; ++bv) {
-        rc = time_pass(kPassForce, dword | (bv << 18), ms);
-        if (ms < f_best) { f_best = ms; f_shape = bv << 18; }
-    }
-    if (!scenes && !tension && rc == SPH_OK) {  // two particles per lane (single scene)
-        rc = time_pass(kPassForce, dword | (1u << 22), ms);
-        if (ms < f_best) { f_best = ms; f_shape = 1u << 22; }
-    }
-    for (uint32_t gsh = 1; gsh <= (tension ? 0u : 4u) && rc == SPH_OK; ++gsh) {
-        rc = time_pass(kPassForce, dword | f_shape | (gsh << 12), ms);
-        if (ms < f_best) { f_best = ms; f_grid = gsh; }
-    }
+    // Walled scenes and the force with tension have one shape.
+    const bool rows = !scenes && row_order(p, b);
+    const uint32_t groups = group_count(p.n, scenes ? b.n_groups : 0u);
+    TunedPass density, force;
+    rc = tune_pass(false, rows, groups, scenes != nullptr,
+                   [&](uint32_t w, float& ms) { return time_pass(kPassDensity, w, ms); }, density);
+    if (rc == SPH_OK) rc = run(kPassDensity, density.word);  // the force pass's input
+    if (rc == SPH_OK)
+        rc = tune_pass(true, rows || tension, groups, scenes != nullptr,
+                       [&](uint32_t w, float& ms) { return time_pass(kPassForce, w, ms); }, force);
     if (rc != SPH_OK) return fail(rc);
     e = hipMemcpyAsync(b.pos, saved, bytes, hipMemcpyDeviceToDevice, stream);
     if (e == hipSuccess)
         e = hipMemcpyAsync(b.vel, static_cast<char*>(saved) + bytes, bytes,
                            hipMemcpyDeviceToDevice, stream);
     if (e != hipSuccess) return fail(hip_error(e, "autotune restore", __FILE__, __LINE__));
-    *tune_out = dword | f_shape | (f_grid << 12);
+    *tune_out = density.word | force.word;
     if (ms_out) {
-        ms_out[0] = d_def;
-        ms_out[1] = d_best;
-        ms_out[2] = f_def;
-        ms_out[3] = f_best;
+        ms_out[0] = density.default_ms;
+        ms_out[1] = density.best_ms;
+        ms_out[2] = force.default_ms;
+        ms_out[3] = force.best_ms;
     }
     return fail(SPH_OK);
 }

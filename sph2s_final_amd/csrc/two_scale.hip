@@ -1833,9 +1833,8 @@ int capture_two_scale(sph_two_scale* t, float dt, bool accel) {
 
 size_t al(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
 
-// Times the launch variants of each set's own-set density and force passes
-// (tile and queue, block size, particles per lane, then the grid shape of the
-// best) on the current state and returns the fastest word per set.  It runs
+// Times the launch variants of each set's own-set density and force passes on the
+// current state and returns the fastest word per set.  It runs
 // the neighbourhood passes first; the passes it times write only the step's
 // intermediate buffers (densities, the internal-order A/B copy, the own-set
 // acceleration), which the next step recomputes, so the state is unchanged.
@@ -1887,58 +1886,27 @@ int tune_own_passes(sph_two_scale* t, uint32_t reps, uint32_t* tune_out, float* 
             ms /= static_cast<float>(reps);
             return SPH_OK;
         };
-        uint32_t word[2] = {0u, 0u};
-        float def[2] = {0.f, 0.f}, best[2] = {0.f, 0.f};
-        const bool tension = P[r].tens != 0.0f;
+        TunedPass tuned[2];
         for (int pass = 0; pass < 2; ++pass) {
             const bool force = pass == 1;
-            if (force && tension) {  // the tension form runs the default
-                int rc = time(true, 0u, def[1]);
-                if (rc != SPH_OK) return done(rc);
-                best[1] = def[1];
-                break;
-            }
-            // tile/queue field, block-size field, particles-per-lane field, grid field
-            const uint32_t nvar = force ? 9u : 5u;
-            const int vshift = force ? 4 : 0, bshift = force ? 18 : 16, pshift = force ? 22 : 20,
-                      gshift = force ? 12 : 8;
-            float ms = 0.f;
-            uint32_t shape = 0u, grid = 0u;
-            int rc = time(force, 0u, def[pass]);
-            best[pass] = def[pass];
-            for (uint32_t v = 1; v <= nvar && rc == SPH_OK; ++v) {
-                rc = time(force, v << vshift, ms);
-                if (ms < best[pass]) { best[pass] = ms; shape = v << vshift; }
-            }
-            for (uint32_t bv = 1; bv <= 2 && rc == SPH_OK; ++bv) {
-                rc = time(force, bv << bshift, ms);
-                if (ms < best[pass]) { best[pass] = ms; shape = bv << bshift; }
-            }
-            if (rc == SPH_OK) {
-                rc = time(force, 1u << pshift, ms);
-                if (ms < best[pass]) { best[pass] = ms; shape = 1u << pshift; }
-            }
-            for (uint32_t gsh = 1; gsh <= 4 && rc == SPH_OK; ++gsh) {
-                rc = time(force, shape | (gsh << gshift), ms);
-                if (ms < best[pass]) { best[pass] = ms; grid = gsh; }
-            }
+            int rc = tune_pass(force, force && P[r].tens != 0.0f,  // tension: one shape
+                               (S.cap + kGroupTargets - 1) / kGroupTargets, false,
+                               [&](uint32_t w, float& ms) { return time(force, w, ms); }, tuned[pass]);
             if (rc != SPH_OK) return done(rc);
-            word[pass] = shape | (grid << gshift);
             if (!force) {  // densities and the A, B copy for the force timings
                 StepParams p = P[r];
-                p.tune = word[0];
+                p.tune = tuned[0].word;
                 rc = launch_density_own_x(p, S.buf, st);
                 if (rc == SPH_OK) rc = launch_gather_aux(p, S.buf, st);
                 if (rc != SPH_OK) return done(rc);
             }
         }
-        tune_out[r] = word[0] | word[1];
-        if (ms_out) {
-            ms_out[4 * r + 0] = def[0];
-            ms_out[4 * r + 1] = best[0];
-            ms_out[4 * r + 2] = def[1];
-            ms_out[4 * r + 3] = best[1];
-        }
+        tune_out[r] = tuned[0].word | tuned[1].word;
+        if (ms_out)
+            for (int pass = 0; pass < 2; ++pass) {
+                ms_out[4 * r + 2 * pass] = tuned[pass].default_ms;
+                ms_out[4 * r + 2 * pass + 1] = tuned[pass].best_ms;
+            }
     }
     return done(SPH_OK);
 }
