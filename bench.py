@@ -324,7 +324,7 @@ def bench_batched(torch, steps: int, cpu_steps: int = 0) -> dict:
             "one_per_launch_serial_pu_s": n * steps / tser,
             "speedup_vs_streams": ts / tb, "speedup_vs_serial": tser / tb,
             "device_errors": errs,
-            "tune": {"word": word, "launch": autotune.describe(word),
+            "tune": {"word": word, "launch": autotune.launch_shape(word),
                      "density_ms_default_tuned": tune_ms[:2],
                      "force_ms_default_tuned": tune_ms[2:]},
             "note": "one-per-launch: each scene its own solver and graph; 'streams' "

@@ -13,9 +13,8 @@ run of the same workload reuses it without timing.
 Tune word fields (include/sph2s.h): bits 0-3 density and 4-7 force waves per
 block, 8-11 density grid, 12-15 force grid, 16-17 density block size, 18-19
 force block size, 20-21 density and 22-23 force groups per wave (single scenes
-only).  The keys and values of describe() are part of the cache file's format
-and keep their first names: the "tile", "list" and "particles_per_lane" entries
-number the variants above.
+only).  launch_shape() says what a word launches.  describe() keeps the names that
+the fields had when they chose LDS tiles, list capacities and particles per lane.
 """
 from __future__ import annotations
 
@@ -30,8 +29,27 @@ GRID_BLOCKS_PER_CU = (None, 1, 2, 4, 8)  # None: one block per block-size partic
 BLOCK_THREADS = (256, 128, 512)
 
 
+# Waves per block of a pass's waves field (step.hip) and of its block-size field.
+WAVES = (4, 1, 2, 3, 5, 6, 4, 4, 4, 4)
+
+
+def launch_shape(tune: int) -> dict:
+    """The launch a tune word selects: per pass its waves per block, the groups of 32
+    particles that a wave takes, and the blocks per CU of a persistent grid (None: as
+    many blocks as the groups need).  (Passes with one shape ignore the word: both of a
+    walled scene, and the force with tension.)"""
+    shape = {}
+    for name, waves, grid, block, groups, most in (("density", 0, 8, 16, 20, 8),
+                                                   ("force", 4, 12, 18, 22, 6)):
+        size = tune >> block & 0x3
+        shape[name] = {"waves_per_block": {1: 2, 2: most}.get(size, WAVES[tune >> waves & 0xF]),
+                       "groups_per_wave": 1 + (tune >> groups & 0x3),
+                       "blocks_per_cu": GRID_BLOCKS_PER_CU[tune >> grid & 0xF]}
+    return shape
+
+
 def describe(tune: int) -> dict:
-    """The launch shape a tune word selects."""
+    """A tune word's fields under their first names (see launch_shape for the launch)."""
     d, f = tune & 0xF, (tune >> 4) & 0xF
     dg, fg = (tune >> 8) & 0xF, (tune >> 12) & 0xF
     db, fb = (tune >> 16) & 0x3, (tune >> 18) & 0x3
@@ -82,10 +100,10 @@ def tune(solver, kind: str, particles: int, cells: int, dt: float, scenes: int =
     if not retune and key in cache:
         word = int(cache[key]["tune"])
         solver.set_tune(word)
-        return {"tune": word, "cached": True, "launch": describe(word),
+        return {"tune": word, "cached": True, "launch": launch_shape(word),
                 "ms": cache[key].get("ms")}
     word, ms = solver.autotune(dt, reps)
     if cache_path:
-        cache[key] = {"tune": word, "ms": ms, "launch": describe(word)}
+        cache[key] = {"tune": word, "ms": ms, "launch": launch_shape(word)}
         save_cache(cache_path, cache)
-    return {"tune": word, "cached": False, "launch": describe(word), "ms": ms}
+    return {"tune": word, "cached": False, "launch": launch_shape(word), "ms": ms}
