@@ -31,6 +31,9 @@ BLOCK_THREADS = (256, 128, 512)
 
 # Waves per block of a pass's waves field (step.hip) and of its block-size field.
 WAVES = (4, 1, 2, 3, 5, 6, 4, 4, 4, 4)
+# What the fields mean: part of the cache's keys, so that words tuned when they
+# meant something else are tuned anew.
+WORD_FORMAT = 2
 
 
 def launch_shape(tune: int) -> dict:
@@ -63,7 +66,8 @@ def describe(tune: int) -> dict:
 
 
 def workload_key(kind: str, particles: int, cells: int, scenes: int = 1, device: str = "") -> str:
-    return f"{device}|{kind}|n={int(particles)}|cells={int(cells)}|scenes={int(scenes)}"
+    return (f"{device}|{kind}|n={int(particles)}|cells={int(cells)}|scenes={int(scenes)}"
+            f"|words={WORD_FORMAT}")
 
 
 def _device_name() -> str:
