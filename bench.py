@@ -454,7 +454,9 @@ def bench_main(torch, args) -> dict:
     pass_ms = {name: per_pass[i] / args.steps for i, name in enumerate(C.PASS_NAMES)}
     cand /= args.steps
     nbr /= args.steps
-    flop_step = 18.0 * cand + 50.0 * nbr
+    # Pairs in range run through the FP32 pair bodies (12 flop in density, 38 in
+    # force); the others are rejected by the matrix cores' range filter.
+    flop_step = 50.0 * nbr
     valu_tflops = flop_step / (ms_per_step / 1e3) / 1e12
 
     alg = algorithmic_bytes(n, cells)
@@ -503,8 +505,10 @@ def bench_main(torch, args) -> dict:
                        "frac": valu_tflops / FP32_VALU_PEAK_TFLOPS,
                        "frac_unpacked": valu_tflops / (FP32_VALU_PEAK_TFLOPS / 2),
                        "samples": args.steps,
-                       "note": "18 flop per candidate pair (distance test, both passes) + 50 per "
-                               "in-range pair, pairs counted at every timed step; "
+                       "note": "50 flop per in-range pair (density and force), pairs counted at "
+                               "every timed step; candidates: those of a scan of each particle's "
+                               "own rows (the passes reject theirs per group of 32 with FP16 "
+                               "matrix products, which are not counted); "
                                "frac_unpacked against half the peak (packed FP32 is not used)"},
         "state_finite": finite,
         "device_errors": dev_errors,

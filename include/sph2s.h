@@ -269,9 +269,9 @@ int sph_device_errors(sph_solver* s, uint32_t* bits);
 
 /* Pair work of the most recent step (no counterpart in the reference; a
  * diagnostic for the FLOP model of the neighbour passes): counts[0] = the
- * candidates one neighbour pass walks (every particle's stencil-row runs),
- * counts[1] = the pairs among them with 0 < r < h.  Both are 0 when no step
- * has run since the state was set.  Synchronises the solver's stream. */
+ * candidates in every particle's own stencil rows (the passes themselves list
+ * candidates per group of 32 particles), counts[1] = the pairs among them with
+ * 0 < r < h.  Both are 0 when no step has run since the state was set.  Synchronises the solver's stream. */
 int sph_count_pairs(sph_solver* s, uint64_t counts[2]);
 
 /* ---- launch variants and the autotuner -------------------------------------

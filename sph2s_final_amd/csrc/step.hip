@@ -1064,9 +1064,9 @@ int launch_force_own_x(const StepParams& p, const GridView& g, const StepBuffers
     return SPH_OK;
 }
 
-// Pair work of one neighbour pass of the most recent step, over its internal
-// x-order: the candidates its runs walk (the nine rows and any rows beyond)
-// and the pairs with 0 < r < h among them.  Wave sums, then one 64-bit atomic
+// Pair work of the most recent step, over its internal x-order: the candidates in
+// every particle's own stencil rows (the nine rows and any rows beyond; a group's
+// list holds those of 32 particles) and the pairs with 0 < r < h among them.  Wave sums, then one 64-bit atomic
 // per wave per counter.
 __global__ __launch_bounds__(kBlock) void k_count_pairs(const float4* __restrict__ ipos,
                                                         const uint32_t* __restrict__ cs,
