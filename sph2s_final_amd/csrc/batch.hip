@@ -128,9 +128,9 @@ int batch_alloc(const sph_config* cfgs, uint32_t n_scenes, const uint32_t* count
 
     const size_t N = b->n, C = b->total_cells;
     const size_t sort_temp = radix_sort_temp_bytes(b->n);
-    const size_t sizes[] = {al(16 * N), al(16 * N), al(16 * N), al(16 * N), al(4 * N),
+    const size_t sizes[] = {al(16 * N), al(16 * N), al(4 * N),
                             al(16 * N), al(4 * N),  al(4 * N),  al(4 * N),  al(4 * C),
-                            al(4 * C),  al(sort_temp), al(8 * N), al(4),
+                            al(4 * C),  al(sort_temp), al(4),
                             al(sizeof(SceneParams) * n_scenes), al(4 * (n_scenes + 1)),
                             al(16 * N), al(16 * N), al(16 * N), al(16 * N), al(4 * N),
                             al(kXBinBytes * C),
@@ -157,8 +157,6 @@ int batch_alloc(const sph_config* cfgs, uint32_t n_scenes, const uint32_t* count
     };
     b->buf.pos = static_cast<float4*>(take());
     b->buf.vel = static_cast<float4*>(take());
-    b->buf.tpos = static_cast<float4*>(take());
-    b->buf.tvel = static_cast<float4*>(take());
     b->buf.rho = static_cast<float*>(take());
     b->buf.accel = static_cast<float4*>(take());
     b->buf.keys = static_cast<uint32_t*>(take());
@@ -168,7 +166,6 @@ int batch_alloc(const sph_config* cfgs, uint32_t n_scenes, const uint32_t* count
     b->buf.cell_end = static_cast<uint32_t*>(take());
     b->buf.sort_temp = take();
     b->buf.sort_temp_bytes = sort_temp;
-    b->buf.aux = static_cast<float2*>(take());
     b->buf.n_dev = static_cast<uint32_t*>(take());
     b->scenes = static_cast<SceneParams*>(take());
     b->part_offset_dev = static_cast<uint32_t*>(take());

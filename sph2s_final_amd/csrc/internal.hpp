@@ -121,13 +121,13 @@ int radix_sort_pairs(const uint32_t* keys_in, const uint32_t* vals_in,
 int hash_hist_cells(const StepParams& p, const uint32_t* n_dev, const float4* pos, uint32_t* keys,
                     uint32_t key_bits, void* temp, size_t temp_bytes, uint32_t* cell_start,
                     uint32_t* cell_end, hipStream_t stream);
-// The digit passes: (keys, slot) -> (skeys, perm).
 // Hash, sort and reset of the cell ranges in one launch, where the largest
 // segment (a scene, or all of a single scene's slots) fits a block's sort.
 bool block_sort_fits(uint32_t largest);
 int sort_cells_block(const StepParams& p, const uint32_t* n_dev, const float4* pos, uint32_t* skeys,
                      uint32_t* perm, uint32_t key_bits, uint32_t* cell_start, uint32_t* cell_end,
                      hipStream_t stream);
+// The digit passes: (keys, slot) -> (skeys, perm).
 int sort_cells(const StepParams& p, const uint32_t* keys, uint32_t* skeys, uint32_t* perm,
                uint32_t key_bits, void* temp, hipStream_t stream);
 
@@ -144,10 +144,10 @@ struct SceneSegments {
 struct StepBuffers {
     float4* pos;        // state, sorted order of the previous step (w = id bits)
     float4* vel;
-    float4* tpos;       // sorted copy used by the neighbour passes
-    float4* tvel;
+    float4* tpos;       // sorted copy for the colour, wall, XSPH and two-scale passes (a
+    float4* tvel;       // batch has none)
     float*  rho;
-    float2* aux;        // per particle (k (rho - rho0) / rho^2, 1 / rho)
+    float2* aux;        // per particle (k (rho - rho0) / rho^2, 1 / rho): XSPH, two-scale
     float4* accel;      // optional (debug)
     uint32_t* keys;     // unsorted cell hashes
     uint32_t* skeys;    // sorted cell hashes

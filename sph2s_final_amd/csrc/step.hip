@@ -1157,11 +1157,10 @@ int launch_batch_pass(int pass, const StepParams& cap, const StepBuffers& b,
             break;
         }
         case kPassReorder: {
-            // Cell ranges only, then the x-order reads the state through perm
-            // (no pass of a batched step reads the sorted copies).
+            // No pass of a batched step reads the sorted copies.
             if (!b.ipos) return set_error(SPH_ERR_INVALID_ARGUMENT, "step buffers lack the x-order");
             hipLaunchKernelGGL((k_order<true, false>), blocks_for(cap.n), dim3(kBlock), 0, stream,
-                               b.skeys, b.perm, b.pos, b.vel, b.tpos, b.tvel, b.cell_start,
+                               b.skeys, b.perm, b.pos, b.vel, nullptr, nullptr, b.cell_start,
                                b.cell_end, b.n_dev, cap, scenes, b.ipos, b.ivel, b.i2r, b.xbins);
             break;
         }
