@@ -597,8 +597,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
 // largest velocity difference, over the RMS velocity, of the same sums in the
 // group walk's order 3e-4 to 1.6e-3, by the initial jitter), so scenes with
 // walls keep this order of additions and with it their trajectories.  The group
-// walk would take the four steps from 826 to 739 us.  (The XSPH and two-scale
-// forms, which integrate in a later kernel, take the group walk with walls too.)
+// walk would take the four steps from 826 to 739 us.  The XSPH and two-scale forms,
+// which integrate in a later kernel, take the group walk with walls too.  Neither
+// order is the nearer one to 64 bits: four XSPH steps of that tank were off by at
+// most 1.16e-3, 7.7e-4 and 8.1e-4 of the RMS velocity (three initial jitters) with
+// sums by rows and by 1.11e-3, 7.6e-4 and 8.0e-4 with the walk's, the RMS by 1.92e-5 with
+// both; the orders differ by 2e-4 to 6e-4, inputs moved by one unit in the last place
+// by 2.6e-3 to 5.3e-3 (two scales: 3e-4 to 4.5e-3 against 7e-3 to 2.4e-2 in the low set,
+// 1e-2 to 0.2 against 0.27 to 1.0 in the high one).
 constexpr int kRowDensityTile = 1280, kRowForceTile = 640, kRowList = 16, kRowScan = 8;
 
 __device__ __forceinline__ v4f as_v4f(const float4& q) { return v4f{q.x, q.y, q.z, q.w}; }
