@@ -20,14 +20,19 @@
 // A word holds fours of candidates from all over the group's list, so that each
 // word has its share of every target's neighbours and the lanes stay even, and a
 // four is 64 bytes of memory (single candidates touched 60 cache lines a word:
-// the force pass spent half its time on them).  Takes per lane, modelled at 8 / 24 particles per h^3, where a lane has
-// 16 / 49 neighbours: 24 / 60 with the ring, 30 / 71 with the list in parts of
-// 320 that all lanes finish before the next, and three words or eight instead of
-// four make it 25 / 61 and 24 / 59.
+// the force pass spent half its time on them).  Takes per lane, modelled at 8 / 24
+// particles per h^3, where a lane has 16 / 49 neighbours: 24 / 60 with the ring, 30 / 71
+// with the list in parts of 320 that all lanes finish before the next, and three words
+// or eight instead of four make it 25 / 61 and 24 / 59.
+//
+// Groups spread over many cells (spray, films), targets a million h from the origin or
+// not finite, and targets whose sums are not finite are scanned directly instead: each
+// lane walks every other row of its target's stencil (walk_targets, walk_direct).
 //
 // The index of a candidate in the group's list decides the lane that takes it
-// and its place in the order, so a target's sums depend on its group alone: not
-// on the block size or the grid.
+// and its place in the order, and the way a group is taken depends on its targets and
+// their cells, so a target's sums depend on its group alone: not on the block size or
+// the grid.
 #pragma once
 
 #include "neighbors.hpp"
