@@ -346,6 +346,7 @@ struct WalkArguments {
     const float4 *a0, *a1;
     const SceneParams* scenes;
 };
+static_assert(offsetof(WalkArguments, cs) == (sizeof(GridView) + 7) / 8 * 8, "as kernel arguments lie");
 template <bool kBatched>
 __device__ __forceinline__ DirectScan scan_again(uint32_t scene) {
     const WalkArguments w = first_arguments<WalkArguments>();
@@ -407,7 +408,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(5))) void k
                         sum32 = 0.0f;
                     }
                 },
-                [] { return true; }, [] {}, [&] { return scan_again<kBatched>(gr.scene); });
+                [] { return true; },
+                [&] {
+                    sum64 = 0.0;
+                    sum32 = 0.0f;
+                },
+                [&] { return scan_again<kBatched>(gr.scene); });
             const float r = p.c6m_h6 * (kKahan ? static_cast<float>(both_halves(sum64))
                                                : both_halves(sum32));
             if (t.active && (threadIdx.x & 32u) == 0u) {
