@@ -289,7 +289,8 @@ int sph_count_pairs(sph_solver* s, uint64_t counts[2]);
  *   bits 20-21 density, bits 22-23 force: groups of 32 particles that a wave
  *              takes one after the other, 0 = 1, 1 = 2; 1 requires that pass's
  *              waves and block-size fields to be 0, and a batch refuses it
- *   bits 24-31 must be zero; other words are refused with SPH_ERR_ARG
+ *   bits 24-31 must be zero; other words are refused with
+ *              SPH_ERR_INVALID_ARGUMENT
  * All variants give bit-identical results.  Some passes have one launch shape
  * and ignore their fields: both passes of a scene with boundary particles (not
  * with SPH_FLAG_XSPH), and the force with tension.  sph_autotune times each
