@@ -267,8 +267,8 @@ class Solver:
         return int(bits.value)
 
     def count_pairs(self) -> tuple[int, int]:
-        """(candidates, pairs with 0 < r < h) that one neighbour pass of the most
-        recent step walked; (0, 0) before the first step.  Synchronises."""
+        """(candidates in every particle's own stencil rows, pairs with 0 < r < h
+        among them) at the most recent step (sph_count_pairs)."""
         out = (ctypes.c_uint64 * 2)()
         C.check(C.lib().sph_count_pairs(self._h, out))
         return int(out[0]), int(out[1])
