@@ -268,7 +268,7 @@ class Solver:
 
     def count_pairs(self) -> tuple[int, int]:
         """(candidates in every particle's own stencil rows, pairs with 0 < r < h
-        among them) at the most recent step (sph_count_pairs)."""
+        among them) at the most recent step; (0, 0) before the first step.  Synchronises."""
         out = (ctypes.c_uint64 * 2)()
         C.check(C.lib().sph_count_pairs(self._h, out))
         return int(out[0]), int(out[1])
